@@ -730,15 +730,16 @@ static int op_w8a32_ws(Workspace* ws, const float* X, const tl_weights* W, const
    * -> 16-bit widening of the weights, the VALU bound of the three-term bf16
    * path) */
   const int K = W->cols, M4 = 4 * batch;
-  const size_t tb = (size_t)tlk_cdiv(M4, 16) * W->KB * 1024;
+  const bool grouped = tlk_gemm_planes_grouped(M4, W->rows, K);
+  const size_t tb = (size_t)(grouped ? 4 * tlk_cdiv(batch, 16) : tlk_cdiv(M4, 16)) * W->KB * 1024;
   const size_t xe_off = (tb + 255) & ~(size_t)255;
   TRY(tlh_devbuf_ensure(&ws->planes, xe_off + (size_t)batch * sizeof(int), st));
   uint8_t* tiles = (uint8_t*)ws->planes.p;
   int* xe = (int*)(tiles + xe_off);
   /* one work-group per row where the shape allows it (the same planes) */
   const bool by_rows = (K == 1024 || K == 2048 || K == 4096 || K == 6144) && (((uintptr_t)X) & 15) == 0;
-  if (by_rows) HIP_TRY(tlk_launch_split_rows_planes(X, K, batch, K, tiles, xe, st));
-  else HIP_TRY(tlk_launch_split_i8x4(X, K, batch, K, tiles, xe, st));
+  if (by_rows) HIP_TRY(tlk_launch_split_rows_planes(X, K, batch, K, tiles, xe, grouped, st));
+  else HIP_TRY(tlk_launch_split_i8x4(X, K, batch, K, tiles, xe, grouped, st));
   GemmLaunch P = tlk_gemm_launch_init();
   P.amode = A_I8;
   P.A = tiles;
@@ -754,6 +755,7 @@ static int op_w8a32_ws(Workspace* ws, const float* X, const tl_weights* W, const
   P.N = W->rows;
   P.K = K;
   P.out = OUT_F32_X4;
+  P.planes_grouped = grouped;
   return run_gemm(ws, &P, st);
 }
 
@@ -917,7 +919,7 @@ int tlh_linear_w8a8(const float* X, const tl_weights* W, const float* bias, floa
 }
 
 static int linear_w8a32_planes_ws(Workspace* ws, const uint8_t* tiles, const int* xe, const tl_weights* W, float* Y, int batch,
-                            hipStream_t st) {
+                            bool grouped, hipStream_t st) {
   GemmLaunch L = tlk_gemm_launch_init();
   L.amode = A_I8;
   L.A = tiles;
@@ -930,12 +932,13 @@ static int linear_w8a32_planes_ws(Workspace* ws, const uint8_t* tiles, const int
   L.N = W->rows;
   L.K = W->cols;
   L.out = OUT_F32_X4;
+  L.planes_grouped = grouped;
   return run_gemm(ws, &L, st);
 }
 
 int tlh_linear_w8a32_planes(const uint8_t* tiles, const int* xe, const tl_weights* W, float* Y, int batch,
-                            hipStream_t st) {
-  WS_CALL(W->dev, st, linear_w8a32_planes_ws(ws_, tiles, xe, W, Y, batch, st));
+                            bool grouped, hipStream_t st) {
+  WS_CALL(W->dev, st, linear_w8a32_planes_ws(ws_, tiles, xe, W, Y, batch, grouped, st));
 }
 
 static int linear_w8a8_tiles_ws(Workspace* ws, const uint8_t* tiles, const float* xs, const tl_weights* W,

@@ -273,15 +273,18 @@ static int enqueue_prefill(const ModelWeights* m, KVCache* c, DecoderScratch* s,
   float* As = w8 ? (float*)s->p_qs.p : NULL;
   int* Ae = w8 ? NULL : (int*)s->p_qs.p;
 #define LINEAR(X, W, OUT) (w8 ? tlh_linear_w8a8(X, W, NULL, OUT, S, st) : tlh_linear_w8a32(X, W, NULL, OUT, S, st))
-#define LINEAR_Q(W, OUT) \
-  (w8 ? tlh_linear_w8a8_tiles(Aq, As, W, OUT, S, st) : tlh_linear_w8a32_planes(Aq, Ae, W, OUT, S, st))
+/* whether the planes of a linear on W are written grouped (gemm_i8.hip) */
+#define GROUPED(W) (!w8 && tlk_gemm_planes_grouped(4 * S, (W)->rows, (W)->cols))
+#define LINEAR_Q(W, OUT, G) \
+  (w8 ? tlh_linear_w8a8_tiles(Aq, As, W, OUT, S, st) : tlh_linear_w8a32_planes(Aq, Ae, W, OUT, S, G, st))
   for (int l = 0; l < num_layers(m); l++) {
     const LayerDev* L = &m->layers[l];
     float* kc = c->k + (size_t)l * layer_floats(c);
     float* vc = c->v + (size_t)l * layer_floats(c);
     if (fused_q) {
-      HIP_TRY(tlk_launch_rmsnorm_rows_q(Hd, L->norms, Aq, As, Ae, S, H, EPS, st));
-      TRY(LINEAR_Q(L->qkv, QKV));
+      const bool g = GROUPED(L->qkv);
+      HIP_TRY(tlk_launch_rmsnorm_rows_q(Hd, L->norms, Aq, As, Ae, S, H, EPS, g, st));
+      TRY(LINEAR_Q(L->qkv, QKV, g));
     } else {
       HIP_TRY(tlk_launch_rmsnorm_rows(Hd, L->norms, Xn, S, H, EPS, st));
       TRY(LINEAR(Xn, L->qkv, QKV));
@@ -293,10 +296,11 @@ static int enqueue_prefill(const ModelWeights* m, KVCache* c, DecoderScratch* s,
     TRY(LINEAR(ATT, L->o, Y));
     HIP_TRY(tlk_launch_residual_add(Y, Hd, n, st));
     if (fused_q) {
-      HIP_TRY(tlk_launch_rmsnorm_rows_q(Hd, L->norms + H, Aq, As, Ae, S, H, EPS, st));
-      TRY(LINEAR_Q(L->gu, GU));
-      HIP_TRY(tlk_launch_swiglu_rows_q(GU, Aq, As, Ae, S, FF, st));
-      TRY(LINEAR_Q(L->down, Y));
+      const bool g = GROUPED(L->gu), gd = GROUPED(L->down);
+      HIP_TRY(tlk_launch_rmsnorm_rows_q(Hd, L->norms + H, Aq, As, Ae, S, H, EPS, g, st));
+      TRY(LINEAR_Q(L->gu, GU, g));
+      HIP_TRY(tlk_launch_swiglu_rows_q(GU, Aq, As, Ae, S, FF, gd, st));
+      TRY(LINEAR_Q(L->down, Y, gd));
     } else {
       HIP_TRY(tlk_launch_rmsnorm_rows(Hd, L->norms + H, Xn, S, H, EPS, st));
       TRY(LINEAR(Xn, L->gu, GU));
@@ -307,6 +311,7 @@ static int enqueue_prefill(const ModelWeights* m, KVCache* c, DecoderScratch* s,
   }
 #undef LINEAR
 #undef LINEAR_Q
+#undef GROUPED
   return 0;
 }
 
@@ -318,7 +323,7 @@ static int ensure_prefill_buffers(DecoderScratch* s, int S) {
   TRY(tlh_devbuf_ensure(&s->p_gu, (size_t)S * 2 * FF * 4, s->st));
   TRY(tlh_devbuf_ensure(&s->p_mlp, (size_t)S * FF * 4, s->st));
   TRY(tlh_devbuf_ensure(&s->p_y, (size_t)S * H * 4, s->st));
-  TRY(tlh_devbuf_ensure(&s->p_q, (size_t)tlk_cdiv(4 * S, 16) * 16 * FF, s->st));   /* plane tiles of the widest input (K = FF) */
+  TRY(tlh_devbuf_ensure(&s->p_q, (size_t)4 * tlk_cdiv(S, 16) * 16 * FF, s->st));   /* plane tiles of the widest input (K = FF) */
   TRY(tlh_devbuf_ensure(&s->p_qs, (size_t)tlk_cdiv(S, 16) * 16 * sizeof(float), s->st));
   TRY(tlh_devbuf_ensure(&s->p_fpart, tlk_flash_split_floats(S, NQ) * 4, s->st));
   const size_t cb = tlk_flash_split_counters(S, NQ) * sizeof(int);

@@ -386,6 +386,7 @@ static hipError_t launch_mode(const GemmArgs& a, int cfg, int blocks, hipStream_
 // which kernel launch_gemm runs for L
 enum GemmKernel { GK_SMALL, GK_I8, GK_B16, GK_GENERIC };
 static GemmKernel gemm_choice(const GemmLaunch& L) {
+  if (L.planes_grouped) return GK_I8;      // only the quadrant kernel reads that layout
   // up to 16 token rows always stream the weights once; more rows too while N
   // is small (N <= 4096: the tiled kernels would leave CUs idle), up to 64
   // int8 rows; for wide N the activation
@@ -421,6 +422,18 @@ static GemmKernel gemm_choice(const GemmLaunch& L) {
   return GK_GENERIC;
 }
 
+// planes of M4 / 4 tokens: grouped where the tiled int8 GEMM (its quadrant
+// kernel) takes them, rows 4t + p for the small-M kernel
+bool gemm_planes_grouped(int M4, int N, int K) {
+  GemmLaunch L;
+  L.amode = A_I8;
+  L.out = OUT_F32_X4;
+  L.M = M4;
+  L.N = N;
+  L.K = K;
+  return gemm_choice(L) == GK_I8;
+}
+
 // split work-space of the kernel launch_gemm picks for L: partial-sum bytes
 // and zeroed arrival counters (0 and 0 when it needs none)
 void gemm_needs(const GemmLaunch& L, size_t* part_bytes, size_t* counters) {
@@ -428,7 +441,7 @@ void gemm_needs(const GemmLaunch& L, size_t* part_bytes, size_t* counters) {
   *counters = 0;
   switch (gemm_choice(L)) {
     case GK_SMALL: return;
-    case GK_I8: gemm_i8_needs(L.M, L.N, L.K, part_bytes, counters); return;
+    case GK_I8: gemm_i8_needs(L, part_bytes, counters); return;
     case GK_B16: gemm_b16_needs(L.M, L.N, L.K, part_bytes, counters); return;
     default: break;
   }
@@ -492,6 +505,7 @@ hipError_t launch_gemm(const GemmLaunch& L, hipStream_t st) {
 // C ABI of the launchers above (tl_kernels.h)
 // ---------------------------------------------------------------------------
 extern "C" {
+bool tlk_gemm_planes_grouped(int M4, int N, int K) { return tl::gemm_planes_grouped(M4, N, K); }
 void tlk_gemm_plan(int amode, int M, int N, int K, GemmPlan* plan) { *plan = tl::gemm_plan(amode, M, N, K); }
 size_t tlk_gemm_workspace_bytes(int amode, int M, int N, int K) {
   return tl::gemm_workspace_bytes(amode, M, N, K);

@@ -1,5 +1,7 @@
-// gemm_i8.hip -- W8A8 prefill GEMM: int8 codes x int8 weights on
-// v_mfma_i32_16x16x64_i8 with K stages staged through an LDS ring.
+// gemm_i8.hip -- int8 GEMMs of prefill: per-token codes (W8A8) or the four
+// int8 planes of fp32 tokens (W8A32) x int8 weights on v_mfma_i32_16x16x64_i8
+// with K stages staged through an LDS ring.  Two kernels: the LDS-staged one
+// below for few tiles of codes, the quadrant one further down for the rest.
 //
 // Reference: kernel/w8a8_kernel.c:259-268 (w8a8_gemm dequantizes both
 // operands and calls cblas_sgemm).  Here the int32 sum is exact and the fp32
@@ -44,7 +46,7 @@ struct GemmI8Args {
   int ntm, ntn;         // work-group tiles along M and N
   int out;
   const uint8_t* zero_tile;  // 1 KiB of zeros (source of k-blocks past K)
-  int S;                // K slices per tile (LDS-staged kernel; 1 elsewhere)
+  int S;                // K slices per tile
   int32_t* part;        // S > 1: int32 partial tiles [tiles][S][16 MT x 16 NT]
   uint32_t* cnt;        // S > 1: zeroed arrival counters [tiles]
   int xa;               // 2: each XCD owns a block of half the tile rows (tile_of)
@@ -86,58 +88,74 @@ __device__ __forceinline__ void tile_of(int b, int ntm, int ntn, int& tm, int& t
   }
 }
 
-// OUT_F32_X4 epilogue of one 16x16 accumulator tile (every lane calls it):
-// rows 4t .. 4t+3 are the int8 planes of token t, held by the lane quad
-// 4t .. 4t+3 (mod 16) at the same 4 columns n .. n+3; the quad's first lane
-// combines them and stores row t (16 bytes when aligned and inside N).
-__device__ __forceinline__ void planes_epilogue(const GemmI8Args& a, const v4i c, int m, int n, float4 ws4,
-                                                float4 b4, int e, int lane, bool vec_ok) {
-  float y[4];
-#pragma unroll
-  for (int r = 0; r < 4; r++)
-    y[r] = planes_sum(c[r], __shfl_xor(c[r], 1, 64), __shfl_xor(c[r], 2, 64), __shfl_xor(c[r], 3, 64));
-  if ((lane & 3) != 0 || m >= a.M || n >= a.N) return;
-  const float w[4] = {ws4.x, ws4.y, ws4.z, ws4.w};
-  const float b[4] = {b4.x, b4.y, b4.z, b4.w};
-#pragma unroll
-  for (int r = 0; r < 4; r++) {
-    y[r] = planes_scale(y[r], w[r], e);
-    if (a.bias) y[r] = __fadd_rn(y[r], b[r]);
-  }
-  float* yp = reinterpret_cast<float*>(a.Y) + (size_t)(m >> 2) * a.ldy + n;
-  if (vec_ok && n + 4 <= a.N) {
-    st_stream(yp, make_float4(y[0], y[1], y[2], y[3]));
-  } else {
-    for (int r = 0; r < 4 && n + r < a.N; r++) yp[r] = y[r];
-  }
+// The quadrant kernel's order, for any tile counts: XCD x owns an eighth of the
+// tiles, consecutive in an order that walks bands of gm tile rows column by
+// column, so that the tiles an XCD runs at once are a patch of gm rows and its
+// L2 fills gm row panels and as many columns (against tile_of over a sweep of
+// 130 shapes: 6 % faster where the columns divide over the XCDs and tiles
+// number more than 128, 10 % where they do not, equal below).
+__device__ __forceinline__ void tile_patch(int b, int ntm, int ntn, int gm, int& tm, int& tn) {
+  const int n = ntm * ntn, x = b % 8;
+  const int u = x * (n / 8) + min(x, n % 8) + b / 8;      // a bijection of [0, n)
+  const int grp = u / (gm * ntn), r = u - grp * gm * ntn;
+  const int rows = min(gm, ntm - gm * grp);
+  tm = gm * grp + r % rows;
+  tn = r / rows;
 }
 
-// After planes_epilogue over a lane's FM x FN accumulator tiles (rows m0 + 16i,
-// columns n0 + 16j): the outputs it stored for tokens flagged kXeNonFinite
-// (NaN there) are stored again with the reference's fp32 value, nonfinite_dot
-// over the fp32 row in a.xraw.  One copy per kernel, out of the unrolled
-// epilogue, run only by a lane holding a flagged token; the same lane rewrites
-// the same addresses, so its later store is the one that stays.
+// K slices (a.S > 1): every work-group of the tile stores its int32 sums
+// (16-byte write-through stores), waits for their acknowledgement and counts
+// in; the last to arrive adds the S slices into its accumulators (exact integer
+// sums, so any order gives the same bits; slice order here) and returns true.
+// flag: a word of the stage ring, which no copy or read uses any more (an LDS
+// word of its own would push the 80 KiB rings past two work-groups per CU).
 template <int FM, int FN>
-__device__ __forceinline__ void planes_fixup(const GemmI8Args& a, int m0, int n0, int lane) {
-  if ((lane & 3) != 0) return;
-#pragma unroll 1
-  for (int i = 0; i < FM; i++) {
-    const int m = m0 + 16 * i;
-    if (m >= a.M || a.xe[m >> 2] != kXeNonFinite) continue;
-    float* yp = reinterpret_cast<float*>(a.Y) + (size_t)(m >> 2) * a.ldy;
-#pragma unroll 1
-    for (int j = 0; j < FN; j++) {
-#pragma unroll 1
-      for (int r = 0; r < 4; r++) {
-        const int n = n0 + 16 * j + r;
-        if (n >= a.N) break;
-        float y = nonfinite_dot(a.xraw, 0, (size_t)(m >> 2) * a.ldxr, 0, a.K, a.Bt, a.NG, n);
-        if (a.bias) y = __fadd_rn(y, a.bias[n]);
-        yp[n] = y;
-      }
+__device__ __forceinline__ bool merge_slices(const GemmI8Args& a, v4i (&acc)[FM][FN], int wv, int lane, int bt, int ks,
+                                             int* flag) {
+  constexpr int TF = 4 * FM * FN * 256;
+  int32_t* mine = a.part + ((size_t)bt * a.S + ks) * TF;
+#pragma unroll
+  for (int i = 0; i < FM; i++)
+#pragma unroll
+    for (int j = 0; j < FN; j++)
+      st_agent4(reinterpret_cast<float*>(mine) + (((wv * FM + i) * FN + j) * 64 + lane) * 4,
+                __builtin_bit_cast(v4f, acc[i][j]));
+  asm volatile("" ::: "memory");
+  wait_vm<0>();                               // this thread's partial stores are acknowledged
+  asm volatile("" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    *flag = __hip_atomic_fetch_add(a.cnt + bt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(a.S - 1);
+  __syncthreads();
+  if (!*flag) return false;
+  // the merger's acquire: the slices are read after the counter showed them
+  // all arrived (agent scope, once per tile; plain 16-byte loads after it)
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  constexpr int QB = FM * FN <= 8 ? 4 : (FM * FN <= 16 ? 2 : 1);   // slices in flight together
+  const int32_t* slices = a.part + (size_t)bt * a.S * TF;
+  for (int q0 = 0; q0 < a.S; q0 += QB) {
+    v4i pv[QB][FM][FN];
+#pragma unroll
+    for (int u = 0; u < QB; u++)
+#pragma unroll
+      for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+          pv[u][i][j] = *reinterpret_cast<const v4i*>(slices + (size_t)min(q0 + u, a.S - 1) * TF +
+                                                      (((wv * FM + i) * FN + j) * 64 + lane) * 4);
+#pragma unroll
+    for (int u = 0; u < QB; u++) {
+      if (q0 + u >= a.S) break;
+#pragma unroll
+      for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[i][j][r] = q0 + u == 0 ? pv[u][i][j][r] : acc[i][j][r] + pv[u][i][j][r];
     }
   }
+  if (threadIdx.x == 0) __hip_atomic_store(a.cnt + bt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
 }
 
 // Stage ring of NST buffers.  Every K stage is NW*PW whole 1 KiB tiles, each
@@ -247,12 +265,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_lds_kernel(GemmI8Args a)
     e_ws[j] = make_float4(w4[0], w4[1], w4[2], w4[3]);
     e_b[j] = make_float4(b4[0], b4[1], b4[2], b4[3]);
   }
-  int e_xe[FM];
 #pragma unroll
   for (int i = 0; i < FM; i++) {
     const int m = min((mg0 + wm * FM + i) * 16 + mrow, a.M - 1);
-    e_xs[i] = (a.out == OUT_I32 || a.out == OUT_F32_X4) ? 0.0f : a.xs[m];
-    e_xe[i] = (a.out == OUT_F32_X4) ? a.xe[m >> 2] : 0;
+    e_xs[i] = a.out == OUT_I32 ? 0.0f : a.xs[m];
   }
 
   v4i acc[FM][FN];
@@ -324,56 +340,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_lds_kernel(GemmI8Args a)
 
   wait_vm<0>();   // no copy may still be landing in LDS when the work-group exits
 
-  if (a.S > 1) {
-    // K slices: every work-group of the tile stores its int32 sums (16-byte
-    // write-through stores), waits for their acknowledgement and counts in;
-    // the last to arrive adds the S slices (exact integer sums, so any order
-    // gives the same bits; slice order here) and runs the epilogue below
-    constexpr int TF = MT * 16 * NT * 16;
-    int32_t* mine = a.part + ((size_t)bt * a.S + ks) * TF;
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-      for (int j = 0; j < FN; j++)
-        st_agent4(reinterpret_cast<float*>(mine) + (((wv * FM + i) * FN + j) * 64 + lane) * 4,
-                  __builtin_bit_cast(v4f, acc[i][j]));
-    __shared__ int s_last;
-    asm volatile("" ::: "memory");
-    wait_vm<0>();                               // this thread's partial stores are acknowledged
-    asm volatile("" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0)
-      s_last = __hip_atomic_fetch_add(a.cnt + bt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(a.S - 1);
-    __syncthreads();
-    if (!s_last) return;
-    // the merger's acquire: the slices are read after the counter showed them
-    // all arrived (agent scope, once per tile; plain 16-byte loads after it)
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    constexpr int QB = FM * FN <= 8 ? 4 : (FM * FN <= 16 ? 2 : 1);   // slices in flight together
-    const int32_t* slices = a.part + (size_t)bt * a.S * TF;
-    for (int q0 = 0; q0 < a.S; q0 += QB) {
-      v4i pv[QB][FM][FN];
-#pragma unroll
-      for (int u = 0; u < QB; u++)
-#pragma unroll
-        for (int i = 0; i < FM; i++)
-#pragma unroll
-          for (int j = 0; j < FN; j++)
-            pv[u][i][j] = *reinterpret_cast<const v4i*>(slices + (size_t)min(q0 + u, a.S - 1) * TF +
-                                                        (((wv * FM + i) * FN + j) * 64 + lane) * 4);
-#pragma unroll
-      for (int u = 0; u < QB; u++) {
-        if (q0 + u >= a.S) break;
-#pragma unroll
-        for (int i = 0; i < FM; i++)
-#pragma unroll
-          for (int j = 0; j < FN; j++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) acc[i][j][r] = q0 + u == 0 ? pv[u][i][j][r] : acc[i][j][r] + pv[u][i][j][r];
-      }
-    }
-    if (threadIdx.x == 0) __hip_atomic_store(a.cnt + bt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  if (a.S > 1 && !merge_slices<FM, FN>(a, acc, wv, lane, bt, ks, reinterpret_cast<int*>(s0))) return;
 
   // epilogue: y = fl(fl(fl(acc) * ws[n]) * xs[m]) (+ bias[n]); 16-byte
   // streaming stores when the 4 columns are inside N and the row is 16-byte
@@ -381,19 +348,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_lds_kernel(GemmI8Args a)
   // N = 6144, whose write-back from L2 otherwise trails the last MFMA;
   // 23.5 -> 22.5 us per launch)
   const bool vec_ok = ((a.ldy & 3) == 0) && ((((uintptr_t)a.Y) & 15) == 0);
-  if (a.out == OUT_F32_X4) {
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-      for (int j = 0; j < FN; j++)
-        planes_epilogue(a, acc[i][j], (mg0 + wm * FM + i) * 16 + mrow, (ng0 + wn * FN + j) * 16 + ncol, e_ws[j],
-                        e_b[j], e_xe[i], lane, vec_ok);
-    bool bad = false;
-#pragma unroll
-    for (int i = 0; i < FM; i++) bad |= e_xe[i] == kXeNonFinite;
-    if (bad && a.xraw) planes_fixup<FM, FN>(a, (mg0 + wm * FM) * 16 + mrow, (ng0 + wn * FN) * 16 + ncol, lane);
-    return;
-  }
 #pragma unroll
   for (int i = 0; i < FM; i++) {
     const int m = (mg0 + wm * FM + i) * 16 + mrow;
@@ -431,199 +385,244 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_lds_kernel(GemmI8Args a)
 }
 
 // ---------------------------------------------------------------------------
-// Column-split variant: the 4 waves of a work-group split the tile's N columns
-// (wave w owns weight row groups ng0 + FN w .. ng0 + FN w + FN - 1) and all
-// share its MT activation row groups.  Weight tiles are private to one wave,
-// so they go from global memory straight into that wave's registers (one
-// 16-byte load per lane per tile, already in MFMA operand order); only the
-// shared activation tiles pass through an LDS ring.  Per 64-wide K stage and
-// work-group: MT KiB copied into LDS, 4 MT KiB of LDS fragment reads, 4 FN KiB
-// of register loads and 4 MT FN MFMAs (against 3 (MT + NT) KiB of LDS traffic
-// in gemm_i8_lds_kernel with its 2 x 2 wave grid).
+// Quadrant kernel: tiles of 32 FM x 32 FN outputs, 4 waves, each holding one
+// (16 FM) x (16 FN) quadrant in its accumulator registers (FM = FN = 8: 64
+// accumulators, 256 registers, one work-group per CU; up to 24 accumulators two
+// work-groups share a CU).  What bounds small tiles is the movement of
+// operands: per 64-wide K stage a wave reads FM + FN fragments (1 KiB each) for
+// FM FN MFMAs of 16 cycles, and the four waves share 128 B/clk of LDS, so 4 x 4
+// fragments per wave spend 384 LDS cycles (reads and the stage's copies) under
+// 256 MFMA cycles, 8 x 8 spend 768 under 1024, and 8 x 8 pulls 32 B/clk per CU
+// from L2 where 64 x 128 tiles need 96.  Measured against the kernels before it
+// (64 x 128 tiles with weights straight to registers): 2048 tokens of planes
+// over N = 12288, K = 2048 (split included) 316 -> 179 us (2.3 POP/s), 1200
+// tokens 190 -> 110 us; 1200 x 12288 x 2048 codes (128 x 128 LDS-staged tiles)
+// 58 -> 41 us.  One 256 x 256 work-group alone takes 0.47 us per stage (91 % of
+// the MFMA rate), 256 of them 0.67 us (the clock gives way).
 //
-// Pipeline: stage s's copies and loads are issued D steps ahead (its weight
-// registers are set s % (D + 1), its LDS buffer s % D).  Step s waits for
-// stage s + 1, then one barrier makes its activation tiles visible and frees
-// buffer s % D, whose copy for stage s + D follows; the MFMAs of stage s run
-// interleaved with the fragment reads of stage s + 1 and the issue of stage
-// s + D.  The loop is unrolled D + 1 times so every register set index is a
-// compile-time constant.  Copies and loads are branch-free (the compiler's
-// own vmcnt waits stay exact only over straight-line code): stages past the
-// last one re-read the last k-block, and nothing reads what they bring in.
-template <int MT, int FN, int D>
-__global__ __launch_bounds__(256) void gemm_i8_wcol_kernel(GemmI8Args a) {
-  constexpr int NW = 4, NT = NW * FN, PA = MT / NW;
-  constexpr int NB = D + 1;          // weight register sets
-  constexpr int PS = PA + FN;        // vector memory operations per wave per stage
-  static_assert(MT % NW == 0, "activation copies must divide over the waves");
-  static_assert(NB % 2 == 0, "fragment double buffer needs an even unroll");
-  static_assert(PS * (D - 1) < 64, "vmcnt range");
-  __shared__ uint4 sA[D * MT * 64];
+// Stage s lives in ring slot s % NST.  Step s waits until stage s + 1 has
+// landed, one barrier makes it visible and frees slot s % NST; the MFMAs of
+// stage s run with the fragment reads of stage s + 1 and the copies of stage
+// s + NST spread between them, one every MPO MFMAs (the rate at which the LDS
+// serves the four waves).  Sources are uniform 64-bit bases plus one per-lane
+// offset; stages past K re-read the last k-block (branch-free, so the wait
+// counts are exact), and nothing reads what they bring in.
+//
+// QUAD_PLANES: grouped planes (GemmLaunch::planes_grouped): row group 4T + p holds
+// plane p of tokens 16T .. 16T + 15, so the four sums of one output are the same
+// lane's accumulators 4T .. 4T + 3 and fold without any exchange of lanes
+// (planes_epilogue's 12 cross-lane moves per accumulator were a third of the
+// 64 x 128 kernel's time at K = 2048).
+// The accumulators are pinned to the accumulation registers: left to itself the
+// register allocator moves them (and fragments) between the two register files
+// in the loop, up to 190 moves per 64 MFMAs.
+__device__ __forceinline__ void mfma_i8_acc(v4i& c, uint4 x, uint4 y) {
+  asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(c) : "v"(__builtin_bit_cast(v4i, x)), "v"(__builtin_bit_cast(v4i, y)));
+}
+// The wait states between the last MFMA's write and the first read of an
+// accumulator, which the compiler inserts only behind MFMAs that it issued
+// (at most 18 for the 4-pass i8 MFMA and a vector ALU read).
+__device__ __forceinline__ void mfma_i8_settle() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+
+enum { QUAD_F32, QUAD_PLANES, QUAD_I32 };   // outputs: scaled codes, folded planes, the sums
+template <int FM, int FN, int NST, int MODE>
+__global__ __launch_bounds__(256, FM * FN <= 24 ? 2 : 1) void gemm_i8_quad_kernel(GemmI8Args a) {
+  constexpr int MT = 2 * FM, NT = 2 * FN, TS = MT + NT;   // row groups, column groups, tiles per stage
+  constexpr int PA = MT / 4, PW = TS / 4;                 // copies per wave per stage (PA of them activations)
+  constexpr int NMEM = FM + FN + PW;                      // memory operations per wave per stage
+  constexpr int MPO = FM * FN >= 2 * NMEM ? 2 : 1;        // MFMAs per memory operation
+  static_assert(MT % 4 == 0 && NT % 4 == 0, "copies must divide over the waves");
+  static_assert(MODE != QUAD_PLANES || FM % 4 == 0, "a wave holds whole plane groups");
+  static_assert(NST >= 3 && NST * TS <= 160 && PW * (NST - 1) < 64, "LDS size, vmcnt range");
+  constexpr uint32_t SB = TS * 1024;                      // bytes per stage
+  __shared__ uint4 sS[NST * TS * 64];
 
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-
+  const int wm = wv >> 1, wn = wv & 1;
+  // with K slices, work-group b takes slice b / tiles of tile b % tiles
+  constexpr bool SLICES = MODE == QUAD_PLANES && FM * FN <= 16;
+  const int ks = SLICES ? blockIdx.x / (a.ntm * a.ntn) : 0;
+  const int bt = blockIdx.x - ks * a.ntm * a.ntn;
   int tm, tn;
-  tile_of(blockIdx.x, a.ntm, a.ntn, tm, tn, a.xa);
-  const int mg0 = tm * MT, ng0 = tn * NT + wv * FN;
+  tile_patch(bt, a.ntm, a.ntn, FM == 8 ? 4 : 8, tm, tn);
+  const int mg0 = tm * MT, ng0 = tn * NT;
+  const int kb0 = SLICES ? (ks * a.KB) / a.S : 0;         // this work-group's k-blocks [kb0, kb0 + KB)
+  const int KB = SLICES ? ((ks + 1) * a.KB) / a.S - kb0 : a.KB;
+  const size_t astep = (size_t)a.MG * 1024, bstep = (size_t)a.NG * 1024;
 
-  const uint4* A4 = reinterpret_cast<const uint4*>(a.At) + lane;
-  const uint4* B4 = reinterpret_cast<const uint4*>(a.Bt) + lane;
-  const int KB = a.KB;
-  const size_t astride = (size_t)a.MG * 64, bstride = (size_t)a.NG * 64;
-  // rows / columns past the matrix edge re-read a valid tile (their
-  // accumulators are never stored)
-  const uint4* asrc[PA];
+  // copy p of a stage: tile wv + 4 p of its A then B tiles; rows / columns
+  // past the matrix edge re-read a valid tile (never stored)
+  const uint8_t* src[PW];
 #pragma unroll
-  for (int p = 0; p < PA; p++) asrc[p] = A4 + (size_t)min(mg0 + wv + NW * p, a.MG - 1) * 64;
-  const uint4* bsrc[FN];
-#pragma unroll
-  for (int j = 0; j < FN; j++) bsrc[j] = B4 + (size_t)min(ng0 + j, a.NG - 1) * 64;
-  const uint32_t sbase = lds_addr(sA);
-  constexpr uint32_t SBYTES = MT * 1024;
-
-  uint4 wb[NB][FN];
-  auto copy_a = [&](int st, int p) {
-    const uint4* g = asrc[p] + (size_t)min(st, KB - 1) * astride;
-    dma_tile(g, sbase + (uint32_t)(st % D) * SBYTES + (uint32_t)(wv + NW * p) * 1024u);
+  for (int p = 0; p < PW; p++)
+    src[p] = p < PA ? a.At + kb0 * astep + (size_t)min(mg0 + wv + 4 * p, a.MG - 1) * 1024
+                    : a.Bt + kb0 * bstep + (size_t)min(ng0 + wv + 4 * (p - PA), a.NG - 1) * 1024;
+  const uint32_t lane16 = lane * 16;
+  const uint32_t sbase = lds_addr(sS);
+  auto copy = [&](size_t oa, size_t ob, uint32_t slot, int p) {
+    dma_tile_s(lane16, src[p] + (p < PA ? oa : ob), sbase + slot + (uint32_t)(wv + 4 * p) * 1024u);
   };
-  auto load_b = [&](int st, int c, int j) { wb[c][j] = bsrc[j][(size_t)min(st, KB - 1) * bstride]; };
 
-  // epilogue operands first (older than every copy, so the first wait covers them)
-  const int mrow = lane & 15;
-  const int ncol = (lane >> 4) * 4;
-  float4 e_ws[FN], e_b[FN];
-  float e_xs[MT];
+  v4i acc[FM][FN];
 #pragma unroll
-  for (int j = 0; j < FN; j++) {
-    const int n = (ng0 + j) * 16 + ncol;
-    float w4[4], b4[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int nn = min(n + r, a.N - 1);
-      w4[r] = a.ws[nn];
-      b4[r] = a.bias ? a.bias[nn] : 0.0f;
-    }
-    e_ws[j] = make_float4(w4[0], w4[1], w4[2], w4[3]);
-    e_b[j] = make_float4(b4[0], b4[1], b4[2], b4[3]);
-  }
-  int e_xe[MT];
-#pragma unroll
-  for (int i = 0; i < MT; i++) {
-    const int m = min((mg0 + i) * 16 + mrow, a.M - 1);
-    e_xs[i] = (a.out == OUT_I32 || a.out == OUT_F32_X4) ? 0.0f : a.xs[m];
-    e_xe[i] = (a.out == OUT_F32_X4) ? a.xe[m >> 2] : 0;
-  }
-
-  v4i acc[MT][FN];
-#pragma unroll
-  for (int i = 0; i < MT; i++)
+  for (int i = 0; i < FM; i++)
 #pragma unroll
     for (int j = 0; j < FN; j++) acc[i][j] = v4i{0, 0, 0, 0};
 
-  uint4 fa[2][MT];
-  auto read_frags = [&](int st, int c) {
-    const uint4* buf = sA + (size_t)(st % D) * (MT * 64);
-#pragma unroll
-    for (int i = 0; i < MT; i++) fa[c][i] = buf[i * 64 + lane];
-  };
+  uint4 fa[2][FM], fb[2][FN];
+  const uint4* ra = sS + wm * FM * 64 + lane;             // this lane's A and B fragments in slot 0
+  const uint4* rb = sS + (MT + wn * FN) * 64 + lane;
 
-  // prologue: stages 0 .. D-1 in flight, stage 0 visible and its fragments read
+  // prologue: stages 0 .. NST-1 in flight, stage 0's fragments read
 #pragma unroll
-  for (int b = 0; b < D; b++) {
+  for (int b = 0; b < NST; b++) {
+    const size_t sc = min(b, KB - 1);
 #pragma unroll
-    for (int p = 0; p < PA; p++) copy_a(b, p);
-#pragma unroll
-    for (int j = 0; j < FN; j++) load_b(b, b, j);
+    for (int p = 0; p < PW; p++) copy(sc * astep, sc * bstep, b * SB, p);
   }
-  wait_vm<PS * (D - 1)>();
+  wait_vm<PW * (NST - 1)>();
   stage_barrier();
-  read_frags(0, 0);
+#pragma unroll
+  for (int i = 0; i < FM; i++) fa[0][i] = ra[i * 64];
+#pragma unroll
+  for (int j = 0; j < FN; j++) fb[0][j] = rb[j * 64];
 
-  // step s (set b = s % NB, fragment set f = s & 1)
-  auto step = [&](int st, int b, int f) {
-    wait_vm<PS * (D - 2)>();   // stage s + 1 landed (this wave's part)
-    wait_lgkm0();              // this wave's reads of stage s are done
-    stage_barrier();           // stage s + 1 visible; buffer s % D free
-    constexpr int NMEM = MT + PS;
-    const int nb = (b + D) % NB;
+  uint32_t slot = 0;                                      // slot of stage s (bytes)
+  auto step = [&](int st, int c) {
+    wait_vm<PW * (NST - 2)>();                            // stage s + 1 landed (this wave's part)
+    wait_lgkm0();                                         // this wave's reads of stage s are done
+    stage_barrier();                                      // stage s + 1 visible; slot of stage s free
+    const uint32_t nxt = slot + SB == NST * SB ? 0u : slot + SB;
+    const uint4* na = ra + nxt / 16;
+    const uint4* nb = rb + nxt / 16;
+    const size_t sc = min(st + NST, KB - 1);
+    const size_t oa = sc * astep, ob = sc * bstep;
     auto mem_op = [&](int q) {
-      if (q < PA) copy_a(st + D, q);
-      else if (q < PS) load_b(st + D, nb, q - PA);
-      else {
-        const uint4* buf = sA + (size_t)((st + 1) % D) * (MT * 64);
-        fa[f ^ 1][q - PS] = buf[(q - PS) * 64 + lane];
-      }
+      if (q < FN) fb[c ^ 1][q] = nb[q * 64];
+      else if (q < FN + FM) fa[c ^ 1][q - FN] = na[(q - FN) * 64];
+      else copy(oa, ob, slot, q - FN - FM);
     };
 #pragma unroll
-    for (int m = 0; m < MT * FN; m++) {
+    for (int m = 0; m < FM * FN; m++) {
       const int i = m / FN, j = m % FN;
-      acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, wb[b][j]),
-                                                        __builtin_bit_cast(v4i, fa[f][i]), acc[i][j], 0, 0, 0);
+      mfma_i8_acc(acc[i][j], fb[c][j], fa[c][i]);
       __builtin_amdgcn_sched_barrier(0);
-      if (m < NMEM) mem_op(m);
+      if (m % MPO == 0 && m / MPO < NMEM) mem_op(m / MPO);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int q = MT * FN; q < NMEM; q++) mem_op(q);
+    for (int q = (FM * FN + MPO - 1) / MPO; q < NMEM; q++) mem_op(q);
     __builtin_amdgcn_sched_barrier(0);
+    slot = nxt;
   };
-  const int kfull = KB - KB % NB;
-  for (int st = 0; st < kfull; st += NB) {
-#pragma unroll
-    for (int b = 0; b < NB; b++) step(st + b, b, b & 1);
+  // two steps a round, so that the fragment set is a compile-time constant
+  int st = 0;
+  for (; st + 2 <= KB; st += 2) {
+    step(st, 0);
+    step(st + 1, 1);
   }
-#pragma unroll
-  for (int b = 0; b < NB - 1; b++)
-    if (kfull + b < KB) step(kfull + b, b, b & 1);
-
+  if (st < KB) step(st, 0);
   wait_vm<0>();   // no copy may still be landing in LDS when the work-group exits
+  mfma_i8_settle();
+  if constexpr (SLICES) {
+    if (a.S > 1 && !merge_slices<FM, FN>(a, acc, wv, lane, bt, ks, reinterpret_cast<int*>(sS))) return;
+  }
 
-  const bool vec_ok = ((a.ldy & 3) == 0) && ((((uintptr_t)a.Y) & 15) == 0);
-  if (a.out == OUT_F32_X4) {
+  // Epilogue.  Every operand is loaded before the first store: memory
+  // operations retire in order, so a load behind stores waits for their
+  // acknowledgements (bias and scales loaded where they are used cost 25 us at
+  // 64 accumulators).  No bias is -0, which added changes nothing.
+  const int mrow = lane & 15, ncol = (lane >> 4) * 4;
+  const int c0 = ng0 + wn * FN;                           // the wave's first column group
+  float4 e_ws[FN], e_b[FN];
 #pragma unroll
-    for (int i = 0; i < MT; i++)
+  for (int j = 0; j < FN; j++) {
+    const int n = (c0 + j) * 16 + ncol;
+    e_ws[j] = *reinterpret_cast<const float4*>(a.ws + min(c0 + j, a.NG - 1) * 16 + ncol);   // padded to 16 NG
+    e_b[j] = make_float4(-0.0f, -0.0f, -0.0f, -0.0f);
+    if (a.bias)
+      e_b[j] = make_float4(a.bias[min(n, a.N - 1)], a.bias[min(n + 1, a.N - 1)], a.bias[min(n + 2, a.N - 1)],
+                           a.bias[min(n + 3, a.N - 1)]);
+  }
+  // the lane's row of accumulator row group i: a token per 4 groups of planes,
+  // or a token; its exponent or scale
+  constexpr int RI = MODE == QUAD_PLANES ? 4 : 1;
+  const int rows = MODE == QUAD_PLANES ? a.M >> 2 : a.M;
+  const int r0 = (mg0 + wm * FM) * (16 / RI) + mrow;
+  int e_xe[FM / RI];
+  float e_xs[FM / RI];
+#pragma unroll
+  for (int i = 0; i < FM / RI; i++) {
+    const int row = min(r0 + 16 * i, rows - 1);
+    e_xe[i] = MODE == QUAD_PLANES ? a.xe[row] : 0;
+    e_xs[i] = MODE == QUAD_F32 ? a.xs[row] : 0.0f;
+  }
+  auto value = [&](int i, int j) {                        // the 4 outputs of row i, column group j
+    const float w[4] = {e_ws[j].x, e_ws[j].y, e_ws[j].z, e_ws[j].w};
+    const float b[4] = {e_b[j].x, e_b[j].y, e_b[j].z, e_b[j].w};
+    v4f y;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      if constexpr (MODE == QUAD_I32) {
+        y[r] = __int_as_float(acc[i][j][r]);
+      } else {
+        if constexpr (MODE == QUAD_PLANES)
+          y[r] = planes_scale(planes_sum(acc[RI * i][j][r], acc[RI * i + 1][j][r], acc[RI * i + 2][j][r],
+                                         acc[RI * i + 3][j][r]), w[r], e_xe[i]);
+        else
+          y[r] = __fmul_rn(__fmul_rn((float)acc[i][j][r], w[r]), e_xs[i]);
+        y[r] = __fadd_rn(y[r], b[r]);
+      }
+    }
+    return y;
+  };
+  float* Y = reinterpret_cast<float*>(a.Y);               // int32 bits with QUAD_I32
+  if ((c0 + FN) * 16 <= a.N && (a.ldy & 3) == 0 && (((uintptr_t)a.Y) & 15) == 0) {
+    // whole columns, 16-byte aligned rows: streaming stores
+#pragma unroll
+    for (int i = 0; i < FM / RI; i++) {
+      const int row = r0 + 16 * i;
+      if (row >= rows) continue;
 #pragma unroll
       for (int j = 0; j < FN; j++)
-        planes_epilogue(a, acc[i][j], (mg0 + i) * 16 + mrow, (ng0 + j) * 16 + ncol, e_ws[j], e_b[j], e_xe[i], lane,
-                        vec_ok);
+        __builtin_nontemporal_store(value(i, j), reinterpret_cast<v4f*>(Y + (size_t)row * a.ldy + (c0 + j) * 16 + ncol));
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < FM / RI; i++) {
+      const int row = r0 + 16 * i;
+      if (row >= rows) continue;
+#pragma unroll
+      for (int j = 0; j < FN; j++) {
+        const v4f y = value(i, j);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int n = (c0 + j) * 16 + ncol + r;
+          if (n < a.N) Y[(size_t)row * a.ldy + n] = y[r];
+        }
+      }
+    }
+  }
+  if constexpr (MODE == QUAD_PLANES) {
+    // tokens flagged kXeNonFinite: the same lane stores their outputs again
+    // with the reference's fp32 value (as planes_fixup)
     bool bad = false;
 #pragma unroll
-    for (int i = 0; i < MT; i++) bad |= e_xe[i] == kXeNonFinite;
-    if (bad && a.xraw) planes_fixup<MT, FN>(a, mg0 * 16 + mrow, ng0 * 16 + ncol, lane);
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < MT; i++) {
-    const int m = (mg0 + i) * 16 + mrow;
-    if (m >= a.M) continue;
-#pragma unroll
-    for (int j = 0; j < FN; j++) {
-      const int n = (ng0 + j) * 16 + ncol;
-      if (n >= a.N) continue;
-      const v4i c = acc[i][j];
-      if (a.out == OUT_I32) {
-        int32_t* yp = reinterpret_cast<int32_t*>(a.Y) + (size_t)m * a.ldy + n;
-        if (vec_ok && n + 4 <= a.N) {
-          st_stream(yp, make_int4(c[0], c[1], c[2], c[3]));
-        } else {
-          for (int r = 0; r < 4 && n + r < a.N; r++) yp[r] = c[r];
+    for (int i = 0; i < FM / RI; i++) bad |= e_xe[i] == kXeNonFinite;
+    if (bad && a.xraw) {
+#pragma unroll 1
+      for (int i = 0; i < FM / RI; i++) {
+        const int t = r0 + 16 * i;
+        if (t >= rows || a.xe[t] != kXeNonFinite) continue;
+#pragma unroll 1
+        for (int q = 0; q < 4 * FN; q++) {
+          const int n = (c0 + (q >> 2)) * 16 + ncol + (q & 3);
+          if (n >= a.N) continue;
+          float y = nonfinite_dot(a.xraw, 0, (size_t)t * a.ldxr, 0, a.K, a.Bt, a.NG, n);
+          if (a.bias) y = __fadd_rn(y, a.bias[n]);
+          Y[(size_t)t * a.ldy + n] = y;
         }
-        continue;
-      }
-      const float ws4[4] = {e_ws[j].x, e_ws[j].y, e_ws[j].z, e_ws[j].w};
-      const float b4[4] = {e_b[j].x, e_b[j].y, e_b[j].z, e_b[j].w};
-      float y[4];
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        y[r] = __fmul_rn(__fmul_rn((float)c[r], ws4[r]), e_xs[i]);
-        if (a.bias) y[r] = __fadd_rn(y[r], b4[r]);
-      }
-      float* yp = reinterpret_cast<float*>(a.Y) + (size_t)m * a.ldy + n;
-      if (vec_ok && n + 4 <= a.N) {
-        st_stream(yp, make_float4(y[0], y[1], y[2], y[3]));
-      } else {
-        for (int r = 0; r < 4 && n + r < a.N; r++) yp[r] = y[r];
       }
     }
   }
@@ -632,22 +631,14 @@ __global__ __launch_bounds__(256) void gemm_i8_wcol_kernel(GemmI8Args a) {
 // ---------------------------------------------------------------------------
 // planning and launch
 // ---------------------------------------------------------------------------
-// Measured on MI355X at M = 1024 (ring depth and stage width swept):
-// cfg 0: 128 x 192 tiles (8 x 12 fragments), K stage 64, 4 buffers (80 KiB)
-//        (N = 6144, K = 2048: 22.0 us; cfg 4 below takes its place)
-// cfg 1:  64 x 128 tiles (4 x 8),  K stage 64, 8 buffers (96 KiB)
-//        best for N = 2048, K = 6144 (256 work-groups)
-// cfg 2: 128 x 128 tiles (8 x 8),  K stage 64, 8 buffers (128 KiB)
-// cfg 3..7: column-split kernel (weights straight to registers)
-//   3: 128 x 192, prefetch 3   4: 128 x 192, prefetch 5   5: 128 x 192, prefetch 7
-//   6:  64 x 128, prefetch 7   7: 128 x 128, prefetch 7
+// cfg 0..2: LDS-staged kernel, 128 x 192, 64 x 128, 128 x 128 tiles (4, 8, 8
+//   stage buffers); cfg 1 is the planner's for small tile counts, 0 and 2 run
+//   only when forced
+// cfg 3..6: quadrant kernel, 256 x 256, 256 x 192, 128 x 192, 128 x 128 tiles
 static void i8_cfg(int cfg, int& mt, int& nt) {
-  if (cfg == 0) { mt = 8; nt = 12; }
-  else if (cfg == 1) { mt = 4; nt = 8; }
-  else if (cfg == 2) { mt = 8; nt = 8; }
-  else if (cfg <= 5) { mt = 8; nt = 12; }
-  else if (cfg == 6) { mt = 4; nt = 8; }
-  else { mt = 8; nt = 8; }
+  static const int dims[7][2] = {{8, 12}, {4, 8}, {8, 8}, {16, 16}, {16, 12}, {8, 12}, {8, 8}};
+  mt = dims[cfg][0];
+  nt = dims[cfg][1];
 }
 
 // tuning overrides; atomic, since a setter may run while other threads plan launches
@@ -656,72 +647,106 @@ static std::atomic<int> g_i8_force_split{0};
 void gemm_i8_set_cfg(int cfg) { g_i8_force_cfg.store(cfg, std::memory_order_relaxed); }
 void gemm_i8_set_split(int s) { g_i8_force_split.store(s > 0 ? s : 0, std::memory_order_relaxed); }
 
-int gemm_i8_pick_cfg(int M, int N, int K) {
-  const int force = g_i8_force_cfg.load(std::memory_order_relaxed);
-  if (force >= 0) return force;
-  (void)K;
-  // 2048 rows and more (the 4 x 1200 plane rows of a 1200-token fp32 batch):
-  // many tiles per CU, where the deepest weight prefetch on 64 x 128 tiles
-  // measured best on every decoder shape (per layer 594 -> 442 us at 4800
-  // rows); below, tiles that fill the CUs (at 1024-1200 rows cfg 6 was
-  // faster on some shapes and slower on others)
-  if (M >= 2048) return 6;
-  const int MG = cdiv(M, 16), NG = cdiv(N, 16);
-  // the configuration whose tile count best fills 256 CUs (at least one
-  // full wave of work-groups, then the fewest idle CUs in the last wave).
-  // 128 x 192 tiles run on the register-loaded weight kernel (cfg 4: 20.7 us
-  // against 22.0 us for cfg 0 at M = 1024, N = 6144, K = 2048); at 64 x 128
-  // the two kernels measured the same (23.7 / 24.0 us, N = 2048, K = 6144).
-  int best = 2;
-  double best_eff = -1.0;
-  for (int cfg : {4, 1, 2}) {
+// K slices of `tiles` tiles whose work-groups would leave most CUs idle.  A merge
+// costs three dependent memory round trips (partials stored, arrival counted,
+// partials read back), about 3 us, and at K = 2048 every slice count measured
+// slower than none.
+// Codes, 64 x 128 tiles: below 128 tiles at K >= 4096 up to 4 slices of at
+// least 16 k-blocks (200 x 2048 x 6144: 18.2 -> 14.9 us).
+static int codes_slices(int tiles, int KB) {
+  if (tiles >= 128 || KB < 64) return 1;
+  return std::min(std::min(4, 256 / tiles), KB / 16);
+}
+// Planes, 128 x 128 tiles: 4 slices up to 32 tiles, 3 up to 64, 2 up to 95 (the
+// last from K = 6144), measured with 1..8 (20 / 100 / 160 tokens, 2048 x 6144:
+// 24.9 -> 18.1, 27.6 -> 23.3, 28.2 -> 26.4 us).
+static int planes_slices(int tiles, int KB) {
+  if (KB < 64) return 1;
+  return tiles <= 32 ? 4 : (tiles <= 64 ? 3 : (tiles < 96 && KB >= 96 ? 2 : 1));
+}
+
+// the configuration that runs where `cfg` is forced: planes have no 128 x 192
+// tiles and only quadrant ones, codes no 256-row ones (7 is 128 x 128 too)
+static int i8_resolve(int cfg, bool planes) {
+  if (planes) return cfg == 3 || cfg == 4 ? cfg : 6;
+  return cfg == 3 || cfg == 4 ? 5 : std::min(cfg, 6);
+}
+
+// Plan: the configuration of least estimated time, rounds of work-groups times
+// the time of one over KB k-blocks, the constants fitted to measured launches
+// (130 shapes: 17..2048 tokens, N = 1024..12288, K = 1024..6144; the choice is
+// on average 0.1 % and at most 5 % slower than the best configuration of its
+// shape).  Codes over 256 x 192 or 256 x 256 tiles were the best at none: their
+// fp32 outputs (64 KiB per 128 x 128) drain under the next work-group's loop
+// only where two share a CU.
+static void gemm_i8_plan(const GemmLaunch& L, int& cfg, int& split) {
+  const bool planes = L.out == OUT_F32_X4;
+  const int MG = planes ? planes_groups(L.M / 4, true) : cdiv(L.M, 16), NG = cdiv(L.N, 16), KB = cdiv(L.K, 64);
+  auto tiles = [&](int c) {
     int mt, nt;
-    i8_cfg(cfg, mt, nt);
-    const int tiles = cdiv(MG, mt) * cdiv(NG, nt);
-    const int waves = cdiv(tiles, 256);
-    const double eff = (double)tiles / (waves * 256);
-    if (eff > best_eff + 1e-9) {
-      best_eff = eff;
-      best = cfg;
+    i8_cfg(c, mt, nt);
+    return cdiv(MG, mt) * cdiv(NG, nt);
+  };
+  float best = 3.0e38f;
+  auto offer = [&](int c, float us, int s) {
+    if (us < best) {
+      best = us;
+      cfg = c;
+      split = s;
     }
+  };
+  // two work-groups share a CU: a last round of up to 256 runs one per CU
+  auto paired = [&](int t, float fixed, float alone, float pair) {
+    const int n = t / 512, rem = t % 512;
+    return n * (fixed + KB * pair) + (rem == 0 ? 0.0f : fixed + KB * (rem <= 256 ? alone : pair));
+  };
+  if (planes) {
+    offer(3, cdiv(tiles(3), 256) * (11.0f + 0.59f * KB), 1);
+    offer(4, cdiv(tiles(4), 256) * (8.0f + 0.50f * KB), 1);
+    offer(6, paired(tiles(6), 3.9f, 0.265f, 0.435f), planes_slices(tiles(6), KB));
+  } else {
+    offer(1, cdiv(tiles(1), 256) * (5.7f + 0.073f * KB), codes_slices(tiles(1), KB));
+    offer(5, paired(tiles(5), 6.1f, 0.195f, 0.526f), 1);
+    offer(6, paired(tiles(6), 4.1f, 0.183f, 0.36f), 1);
   }
-  return best;
-}
-
-// Plan: configuration and K slices.  With fewer than 128 tiles (a few
-// hundred rows over a narrow N: the int8 planes of 17..64 fp32 tokens, small
-// W8A8 batches) and K >= 4096, the K range of every tile is split over up to
-// 4 work-groups on the LDS-staged kernel (its configuration of the same
-// tile); slices keep at least 16 k-blocks.  The merge costs three dependent
-// memory round trips (partials stored, arrival counted, partials read back),
-// about 3 us: at K = 2048 every split measured slower than none, at K = 4096
-// and 6144 a split of 4 (3 from 64 tiles up, 2 from 96) was the fastest or
-// within 3 % of it (2048 x 6144 at 128 plane rows: 28.5 -> 19.7 us).  The
-// int32 partial sums are exact, so the result is the same bits for every split.
-static void gemm_i8_plan(int M, int N, int K, int& cfg, int& split) {
-  cfg = gemm_i8_pick_cfg(M, N, K);
-  int mt, nt;
-  i8_cfg(cfg, mt, nt);
-  const int tiles = cdiv(cdiv(M, 16), mt) * cdiv(cdiv(N, 16), nt);
-  const int KB = cdiv(K, 64);
-  split = 1;
-  if (tiles < 128 && KB >= 64) split = std::min(std::min(4, 256 / tiles), KB / 16);
+  const int fc = g_i8_force_cfg.load(std::memory_order_relaxed);
+  if (fc >= 0) {
+    cfg = i8_resolve(fc, planes);
+    split = 1;
+  }
   const int fs = g_i8_force_split.load(std::memory_order_relaxed);
-  if (fs > 0) split = std::min(fs, KB);
-  if (split > 1) {              // the LDS-staged kernel of the same tile
-    if (cfg == 3 || cfg == 4 || cfg == 5) cfg = 0;
-    else if (cfg == 6) cfg = 1;
-    else if (cfg == 7) cfg = 2;
+  if (fs > 0) {
+    split = std::min(fs, KB);
+    if (split > 1 && cfg >= 3) cfg = planes ? 6 : 1;   // the kernels that take slices
   }
 }
 
-void gemm_i8_needs(int M, int N, int K, size_t* part_bytes, size_t* counters) {
+void gemm_i8_needs(const GemmLaunch& L, size_t* part_bytes, size_t* counters) {
   int cfg, sp, mt, nt;
-  gemm_i8_plan(M, N, K, cfg, sp);
+  gemm_i8_plan(L, cfg, sp);
   i8_cfg(cfg, mt, nt);
-  const size_t tiles = (size_t)cdiv(cdiv(M, 16), mt) * cdiv(cdiv(N, 16), nt);
+  const int MG = L.out == OUT_F32_X4 ? planes_groups(L.M / 4, true) : cdiv(L.M, 16);
+  const size_t tiles = (size_t)cdiv(MG, mt) * cdiv(cdiv(L.N, 16), nt);
   *part_bytes = sp > 1 ? tiles * sp * (size_t)(256 * mt * nt) * sizeof(int32_t) : 0;
   *counters = sp > 1 ? tiles : 0;
+}
+
+// planes on 256 x 256, 256 x 192 and 128 x 128 tiles, codes on 128 x 192 and
+// 128 x 128 (i8_resolve)
+template <int FM, int FN, int NST>
+static void launch_quad(const GemmI8Args& a, int blocks, hipStream_t st) {
+  if constexpr (FM * FN != 24) {
+    if (a.out == OUT_F32_X4) {
+      hipLaunchKernelGGL((gemm_i8_quad_kernel<FM, FN, NST, QUAD_PLANES>), dim3(blocks), dim3(256), 0, st, a);
+      return;
+    }
+  }
+  if constexpr (FM * FN <= 24) {
+    if (a.out == OUT_I32)
+      hipLaunchKernelGGL((gemm_i8_quad_kernel<FM, FN, NST, QUAD_I32>), dim3(blocks), dim3(256), 0, st, a);
+    else
+      hipLaunchKernelGGL((gemm_i8_quad_kernel<FM, FN, NST, QUAD_F32>), dim3(blocks), dim3(256), 0, st, a);
+  }
 }
 
 hipError_t launch_gemm_i8(const GemmLaunch& L, hipStream_t st) {
@@ -740,15 +765,17 @@ hipError_t launch_gemm_i8(const GemmLaunch& L, hipStream_t st) {
   a.N = L.N;
   a.K = L.K;
   a.KB = cdiv(L.K, 64);
-  a.MG = cdiv(L.M, 16);
+  a.MG = L.planes_grouped ? planes_groups(L.M / 4, true) : cdiv(L.M, 16);
   a.NG = cdiv(L.N, 16);
   a.out = L.out;
   a.zero_tile = L.zero_tile;
   if (L.out == OUT_F32_X4 && (!L.xe || L.M % 4 != 0)) return hipErrorInvalidValue;
   if (L.out != OUT_I32 && L.out != OUT_F32_X4 && !L.xs) return hipErrorInvalidValue;
   if (!L.zero_tile) return hipErrorInvalidValue;
+  // planes come grouped (gemm_planes_grouped)
+  if (L.out == OUT_F32_X4 && !L.planes_grouped) return hipErrorInvalidValue;
   int cfg, sp;
-  gemm_i8_plan(L.M, L.N, L.K, cfg, sp);
+  gemm_i8_plan(L, cfg, sp);
   int mt, nt;
   i8_cfg(cfg, mt, nt);
   a.ntm = cdiv(a.MG, mt);
@@ -762,7 +789,7 @@ hipError_t launch_gemm_i8(const GemmLaunch& L, hipStream_t st) {
     a.xa = 2;
   a.part = static_cast<int32_t*>(L.part);
   a.cnt = L.cnt;
-  if (sp > 1 && (!a.part || !a.cnt || cfg > 2)) return hipErrorInvalidValue;
+  if (sp > 1 && (!a.part || !a.cnt)) return hipErrorInvalidValue;
   const long long blocks_ll = (long long)a.ntm * a.ntn * sp;
   if (blocks_ll > 0x7fffffffLL) return hipErrorInvalidValue;
   const int blocks = (int)blocks_ll;
@@ -770,11 +797,10 @@ hipError_t launch_gemm_i8(const GemmLaunch& L, hipStream_t st) {
     case 0: hipLaunchKernelGGL((gemm_i8_lds_kernel<8, 12, 1, 4, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;
     case 1: hipLaunchKernelGGL((gemm_i8_lds_kernel<4, 8, 1, 8, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;
     case 2: hipLaunchKernelGGL((gemm_i8_lds_kernel<8, 8, 1, 8, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;
-    case 3: hipLaunchKernelGGL((gemm_i8_wcol_kernel<8, 3, 3>), dim3(blocks), dim3(256), 0, st, a); break;
-    case 4: hipLaunchKernelGGL((gemm_i8_wcol_kernel<8, 3, 5>), dim3(blocks), dim3(256), 0, st, a); break;
-    case 5: hipLaunchKernelGGL((gemm_i8_wcol_kernel<8, 3, 7>), dim3(blocks), dim3(256), 0, st, a); break;
-    case 6: hipLaunchKernelGGL((gemm_i8_wcol_kernel<4, 2, 7>), dim3(blocks), dim3(256), 0, st, a); break;
-    default: hipLaunchKernelGGL((gemm_i8_wcol_kernel<8, 2, 7>), dim3(blocks), dim3(256), 0, st, a); break;
+    case 3: launch_quad<8, 8, 4>(a, blocks, st); break;
+    case 4: launch_quad<8, 6, 5>(a, blocks, st); break;
+    case 5: launch_quad<4, 6, 4>(a, blocks, st); break;
+    default: launch_quad<4, 4, 5>(a, blocks, st); break;
   }
   return hipGetLastError();
 }

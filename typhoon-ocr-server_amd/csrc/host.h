@@ -111,4 +111,4 @@ int tlh_linear_w8a8_tiles(const uint8_t* tiles, const float* xs, const tl_weight
 /* the fp32-semantics GEMM (w8a32_linear at batch > 32) on activations already
  * split into four int8 planes per token (code rows 4t + p) with their exponents */
 int tlh_linear_w8a32_planes(const uint8_t* tiles, const int* xe, const tl_weights* W, float* Y, int batch,
-                            hipStream_t st);
+                            bool grouped, hipStream_t st);

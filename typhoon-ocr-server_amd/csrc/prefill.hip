@@ -64,13 +64,13 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restri
 // the arithmetic of quantize_rows_tiled_vec_kernel (quant.hip) on the same
 // values, so the codes equal those of quantizing the stored row afterwards.
 //
-// PLANES: instead, the four int8 planes of the row as code rows 4 row + p
-// (MG = ceil(4 rows / 16)) and its exponent in `xe` (split_i8x4_kernel's
+// PLANES: instead, the four int8 planes of the row as code rows
+// planes_row(row, p, grouped) and its exponent in `xe` (split_i8x4_kernel's
 // arithmetic, quant.hip), the activations of the fp32-semantics GEMM.
 template <int NV, bool PLANES>
 __device__ __forceinline__ void quantize_row_to_tiles(const float4 (&v)[NV], int n4, int row, int MG,
                                                       uint8_t* __restrict__ tiles, float* __restrict__ scales,
-                                                      int* __restrict__ xe, uint32_t* s_mx) {
+                                                      int* __restrict__ xe, uint32_t* s_mx, bool grouped) {
   const int tid = threadIdx.x;
   uint32_t mx = 0;
 #pragma unroll
@@ -96,7 +96,7 @@ __device__ __forceinline__ void quantize_row_to_tiles(const float4 (&v)[NV], int
       planes4_i8(w4, e, code);
 #pragma unroll
       for (int p = 0; p < 4; p++) {
-        const int rr = 4 * row + p;
+        const int rr = planes_row(row, p, grouped);
         t32[(((size_t)(f >> 4) * MG + (rr >> 4)) * 64 + (rr & 15) + 16 * ((f >> 2) & 3)) * 4 + (f & 3)] = code[p];
       }
     }
@@ -126,7 +126,7 @@ template <bool PLANES>
 __global__ __launch_bounds__(256) void rmsnorm_rows_q_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                              int rows, int K, float eps, int MG,
                                                              uint8_t* __restrict__ tiles, float* __restrict__ scales,
-                                                             int* __restrict__ xe) {
+                                                             int* __restrict__ xe, bool grouped) {
   __shared__ float s_part[4];
   __shared__ uint32_t s_mx[4];
   const int rr = xcd_grouped_row(blockIdx.x);
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_q_kernel(const float* __rest
   for (int i = 0; i < 2; i++)
     y[i] = make_float4(__fmul_rn(__fmul_rn(v[i].x, r), wv[i].x), __fmul_rn(__fmul_rn(v[i].y, r), wv[i].y),
                        __fmul_rn(__fmul_rn(v[i].z, r), wv[i].z), __fmul_rn(__fmul_rn(v[i].w, r), wv[i].w));
-  quantize_row_to_tiles<2, PLANES>(y, n4, (int)row, MG, tiles, scales, xe, s_mx);
+  quantize_row_to_tiles<2, PLANES>(y, n4, (int)row, MG, tiles, scales, xe, s_mx, grouped);
 }
 
 // fp32 token rows -> their four int8 planes and exponents (split_i8x4_kernel's
@@ -170,7 +170,8 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_q_kernel(const float* __rest
 template <int NV, bool PLANES>
 __global__ __launch_bounds__(256) void split_rows_planes_kernel(const float* __restrict__ x, int ldx, int rows,
                                                                 int MG, uint8_t* __restrict__ tiles,
-                                                                float* __restrict__ scales, int* __restrict__ xe) {
+                                                                float* __restrict__ scales, int* __restrict__ xe,
+                                                                bool grouped) {
   __shared__ uint32_t s_mx[4];
   const int rr = xcd_grouped_row(blockIdx.x);
   if (rr >= rows) return;                   // the whole work-group
@@ -178,7 +179,7 @@ __global__ __launch_bounds__(256) void split_rows_planes_kernel(const float* __r
   float4 v[NV];
 #pragma unroll
   for (int j = 0; j < NV; j++) v[j] = xr[threadIdx.x + 256 * j];
-  quantize_row_to_tiles<NV, PLANES>(v, 256 * NV, rr, MG, tiles, scales, xe, s_mx);
+  quantize_row_to_tiles<NV, PLANES>(v, 256 * NV, rr, MG, tiles, scales, xe, s_mx, grouped);
 }
 
 // SwiGLU of one token's interleaved gate/up row (the values of
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(256) void split_rows_planes_kernel(const float* __r
 template <int NV, bool PLANES>
 __global__ __launch_bounds__(256) void swiglu_rows_q_kernel(const float* __restrict__ gu, int S, int ffn, int MG,
                                                             uint8_t* __restrict__ tiles, float* __restrict__ scales,
-                                                            int* __restrict__ xe) {
+                                                            int* __restrict__ xe, bool grouped) {
   __shared__ uint32_t s_mx[4];
   __shared__ float4 s_y[NV][256];
   const int tt = xcd_grouped_row(blockIdx.x);
@@ -223,7 +224,7 @@ __global__ __launch_bounds__(256) void swiglu_rows_q_kernel(const float* __restr
   float4 y[NV];
 #pragma unroll
   for (int j = 0; j < NV; j++) y[j] = s_y[j][threadIdx.x];
-  quantize_row_to_tiles<NV, PLANES>(y, ffn >> 2, (int)t, MG, tiles, scales, xe, s_mx);
+  quantize_row_to_tiles<NV, PLANES>(y, ffn >> 2, (int)t, MG, tiles, scales, xe, s_mx, grouped);
 }
 
 // One wave per 128-wide head vector of a token: the token's nq = 2 nkv q
@@ -592,57 +593,57 @@ hipError_t launch_rmsnorm_rows(const float* x, const float* w, float* out, int r
 }
 
 hipError_t launch_rmsnorm_rows_q(const float* x, const float* w, uint8_t* tiles, float* scales, int* xe, int rows,
-                                 int K, float eps, hipStream_t st) {
+                                 int K, float eps, bool grouped, hipStream_t st) {
   if (K % 64 != 0 || K > 2048 || rows < 1 || (!scales == !xe)) return hipErrorInvalidValue;
   const dim3 grid(cdiv(rows, 64) * 64);     // xcd_grouped_row: whole groups of 64 rows
   if (xe)
-    hipLaunchKernelGGL(rmsnorm_rows_q_kernel<true>, grid, dim3(256), 0, st, x, w, rows, K, eps, cdiv(4 * rows, 16),
-                       tiles, scales, xe);
+    hipLaunchKernelGGL(rmsnorm_rows_q_kernel<true>, grid, dim3(256), 0, st, x, w, rows, K, eps,
+                       planes_groups(rows, grouped), tiles, scales, xe, grouped);
   else
     hipLaunchKernelGGL(rmsnorm_rows_q_kernel<false>, grid, dim3(256), 0, st, x, w, rows, K, eps, cdiv(rows, 16),
-                       tiles, scales, xe);
+                       tiles, scales, xe, false);
   return hipGetLastError();
 }
 
 template <bool PLANES>
 static hipError_t launch_rows_q(const float* x, int ldx, int rows, int K, uint8_t* tiles, float* scales, int* xe,
-                                hipStream_t st) {
+                                bool grouped, hipStream_t st) {
   if (rows < 1 || ldx < K || ldx % 4 != 0 || (((uintptr_t)x) & 15) != 0) return hipErrorInvalidValue;
   const dim3 grid(cdiv(rows, 64) * 64);     // xcd_grouped_row: whole groups of 64 rows
-  const int MG = cdiv(PLANES ? 4 * rows : rows, 16);
+  const int MG = PLANES ? planes_groups(rows, grouped) : cdiv(rows, 16);
   switch (K) {
-    case 1024: hipLaunchKernelGGL((split_rows_planes_kernel<1, PLANES>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe); break;
-    case 2048: hipLaunchKernelGGL((split_rows_planes_kernel<2, PLANES>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe); break;
-    case 4096: hipLaunchKernelGGL((split_rows_planes_kernel<4, PLANES>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe); break;
-    case 6144: hipLaunchKernelGGL((split_rows_planes_kernel<6, PLANES>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe); break;
+    case 1024: hipLaunchKernelGGL((split_rows_planes_kernel<1, PLANES>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe, grouped); break;
+    case 2048: hipLaunchKernelGGL((split_rows_planes_kernel<2, PLANES>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe, grouped); break;
+    case 4096: hipLaunchKernelGGL((split_rows_planes_kernel<4, PLANES>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe, grouped); break;
+    case 6144: hipLaunchKernelGGL((split_rows_planes_kernel<6, PLANES>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe, grouped); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
 hipError_t launch_split_rows_planes(const float* x, int ldx, int rows, int K, uint8_t* tiles, int* xe,
-                                    hipStream_t st) {
-  return launch_rows_q<true>(x, ldx, rows, K, tiles, nullptr, xe, st);
+                                    bool grouped, hipStream_t st) {
+  return launch_rows_q<true>(x, ldx, rows, K, tiles, nullptr, xe, grouped, st);
 }
 
 hipError_t launch_quantize_rows_by_row(const float* x, int rows, int K, uint8_t* tiles, float* scales,
                                        hipStream_t st) {
-  return launch_rows_q<false>(x, K, rows, K, tiles, scales, nullptr, st);
+  return launch_rows_q<false>(x, K, rows, K, tiles, scales, nullptr, false, st);
 }
 
 hipError_t launch_swiglu_rows_q(const float* gu, uint8_t* tiles, float* scales, int* xe, int S, int ffn,
-                                hipStream_t st) {
+                                bool grouped, hipStream_t st) {
   if (S < 1 || (!scales == !xe)) return hipErrorInvalidValue;
-  const int MG = xe ? cdiv(4 * S, 16) : cdiv(S, 16);
+  const int MG = xe ? planes_groups(S, grouped) : cdiv(S, 16);
   const dim3 grid(cdiv(S, 64) * 64);        // xcd_grouped_row: whole groups of 64 rows
   if (ffn == 6144 && xe)
-    hipLaunchKernelGGL((swiglu_rows_q_kernel<6, true>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe);
+    hipLaunchKernelGGL((swiglu_rows_q_kernel<6, true>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe, grouped);
   else if (ffn == 6144)
-    hipLaunchKernelGGL((swiglu_rows_q_kernel<6, false>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe);
+    hipLaunchKernelGGL((swiglu_rows_q_kernel<6, false>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe, grouped);
   else if (ffn == 2048 && xe)
-    hipLaunchKernelGGL((swiglu_rows_q_kernel<2, true>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe);
+    hipLaunchKernelGGL((swiglu_rows_q_kernel<2, true>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe, grouped);
   else if (ffn == 2048)
-    hipLaunchKernelGGL((swiglu_rows_q_kernel<2, false>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe);
+    hipLaunchKernelGGL((swiglu_rows_q_kernel<2, false>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe, grouped);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();
@@ -746,20 +747,20 @@ hipError_t tlk_launch_swiglu_rows(const float* gu, float* mlp, int S, int ffn, h
   return tl::launch_swiglu_rows(gu, mlp, S, ffn, st);
 }
 hipError_t tlk_launch_split_rows_planes(const float* x, int ldx, int rows, int K, uint8_t* tiles, int* xe,
-                                        hipStream_t st) {
-  return tl::launch_split_rows_planes(x, ldx, rows, K, tiles, xe, st);
+                                        bool grouped, hipStream_t st) {
+  return tl::launch_split_rows_planes(x, ldx, rows, K, tiles, xe, grouped, st);
 }
 hipError_t tlk_launch_quantize_rows_by_row(const float* x, int rows, int K, uint8_t* tiles, float* scales,
                                            hipStream_t st) {
   return tl::launch_quantize_rows_by_row(x, rows, K, tiles, scales, st);
 }
 hipError_t tlk_launch_rmsnorm_rows_q(const float* x, const float* w, uint8_t* tiles, float* scales, int* xe,
-                                     int rows, int K, float eps, hipStream_t st) {
-  return tl::launch_rmsnorm_rows_q(x, w, tiles, scales, xe, rows, K, eps, st);
+                                     int rows, int K, float eps, bool grouped, hipStream_t st) {
+  return tl::launch_rmsnorm_rows_q(x, w, tiles, scales, xe, rows, K, eps, grouped, st);
 }
 hipError_t tlk_launch_swiglu_rows_q(const float* gu, uint8_t* tiles, float* scales, int* xe, int S, int ffn,
-                                    hipStream_t st) {
-  return tl::launch_swiglu_rows_q(gu, tiles, scales, xe, S, ffn, st);
+                                    bool grouped, hipStream_t st) {
+  return tl::launch_swiglu_rows_q(gu, tiles, scales, xe, S, ffn, grouped, st);
 }
 hipError_t tlk_launch_residual_add(const float* y, float* h, long long n, hipStream_t st) {
   return tl::launch_residual_add(y, h, n, st);

@@ -225,8 +225,8 @@ __global__ __launch_bounds__(256) void quantize_rows_tiled_vec_kernel(const floa
 // K inside the last k-block gets zero codes).  A row holding Inf or NaN gets
 // xe = kXeNonFinite and zero codes.
 __global__ __launch_bounds__(256) void split_i8x4_kernel(const float* __restrict__ X, int ldx, int M, int K,
-                                                         int KB, int MG, uint8_t* __restrict__ tiles,
-                                                         int* __restrict__ xe) {
+                                                         int KB, int MG, bool grouped,
+                                                         uint8_t* __restrict__ tiles, int* __restrict__ xe) {
   const int lane = threadIdx.x & 63;
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= M) return;
@@ -252,9 +252,8 @@ __global__ __launch_bounds__(256) void split_i8x4_kernel(const float* __restrict
   const int ee = planes_exponent(mx);
   const int e = finite ? ee : 0;
   if (lane == 0) xe[t] = ee;
-  // tile dword of plane p for float4 group f: row 4t + p of group (4t + p) >> 4
+  // tile dword of plane p for float4 group f: code row planes_row(t, p)
   uint32_t* t32 = reinterpret_cast<uint32_t*>(tiles);
-  const int r0 = 4 * t;
   for (int f = lane; f < nf; f += 64) {
     const int k = 4 * f;
     float v[4] = {0.f, 0.f, 0.f, 0.f};
@@ -271,17 +270,18 @@ __global__ __launch_bounds__(256) void split_i8x4_kernel(const float* __restrict
     planes4_i8(v, e, code);
 #pragma unroll
     for (int p = 0; p < 4; p++) {
-      const int rr = r0 + p;
+      const int rr = planes_row(t, p, grouped);
       // k-block f >> 4, tile lane (rr & 15) + 16 ((f >> 2) & 3), dword f & 3
       t32[(((size_t)(f >> 4) * MG + (rr >> 4)) * 64 + (rr & 15) + 16 * ((f >> 2) & 3)) * 4 + (f & 3)] = code[p];
     }
   }
 }
 
-hipError_t launch_split_i8x4(const float* X, int ldx, int M, int K, uint8_t* tiles, int* xe, hipStream_t st) {
+hipError_t launch_split_i8x4(const float* X, int ldx, int M, int K, uint8_t* tiles, int* xe, bool grouped,
+                             hipStream_t st) {
   if (M <= 0 || K <= 0 || ldx < K || !X || !tiles || !xe) return hipErrorInvalidValue;
-  const int KB = cdiv(K, 64), MG = cdiv(4 * M, 16);
-  hipLaunchKernelGGL(split_i8x4_kernel, dim3(cdiv(M, 4)), dim3(256), 0, st, X, ldx, M, K, KB, MG, tiles, xe);
+  const int KB = cdiv(K, 64), MG = planes_groups(M, grouped);
+  hipLaunchKernelGGL(split_i8x4_kernel, dim3(cdiv(M, 4)), dim3(256), 0, st, X, ldx, M, K, KB, MG, grouped, tiles, xe);
   return hipGetLastError();
 }
 
@@ -474,8 +474,9 @@ hipError_t tlk_launch_pack_tiles_rows(const int8_t* w, int rows, int cols, int N
 hipError_t tlk_launch_unpack_tiles(const uint8_t* tiles, int rows, int cols, int8_t* w, hipStream_t st) {
   return tl::launch_unpack_tiles(tiles, rows, cols, w, st);
 }
-hipError_t tlk_launch_split_i8x4(const float* X, int ldx, int M, int K, uint8_t* tiles, int* xe, hipStream_t st) {
-  return tl::launch_split_i8x4(X, ldx, M, K, tiles, xe, st);
+hipError_t tlk_launch_split_i8x4(const float* X, int ldx, int M, int K, uint8_t* tiles, int* xe, bool grouped,
+                                 hipStream_t st) {
+  return tl::launch_split_i8x4(X, ldx, M, K, tiles, xe, grouped, st);
 }
 hipError_t tlk_launch_copy_words(const void* src, void* dst, size_t bytes, hipStream_t st) {
   return tl::launch_copy_words(src, dst, bytes, st);

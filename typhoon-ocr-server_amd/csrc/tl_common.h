@@ -318,6 +318,15 @@ __device__ __forceinline__ void planes4_i8(const float (&v)[4], int e, uint32_t 
     code[3] |= bp[2] << (8 * q);
   }
 }
+// Code row of plane p of token t: 4t + p, or grouped, where row group 4T + p
+// holds plane p of tokens 16T .. 16T + 15 (the layout of the quadrant GEMM);
+// and the code row groups of `rows` tokens.
+__host__ __device__ __forceinline__ int planes_row(int t, int p, bool grouped) {
+  return grouped ? 64 * (t >> 4) + 16 * p + (t & 15) : 4 * t + p;
+}
+__host__ __device__ __forceinline__ int planes_groups(int rows, bool grouped) {
+  return grouped ? 4 * cdiv(rows, 16) : cdiv(4 * rows, 16);
+}
 // the row exponent of the planes: frexp exponent of the absmax - 6 (0 for a
 // zero row), or kXeNonFinite when the row holds Inf or NaN
 __device__ __forceinline__ int planes_exponent(uint32_t absmax_bits) {

@@ -67,9 +67,11 @@ hipError_t tlk_launch_unpack_tiles(const uint8_t* tiles, int rows, int cols, int
 // MG = ceil(4M / 16), k-blocks ceil(K / 64); row 4t + p is plane p of token
 // t) and per-token exponents xe[M]: x = 2^e (q0 + q1/254 + q2/254^2 +
 // q3/254^3) up to 2^-32 of the row's absmax; a row holding Inf or NaN gets
-// xe = kXeNonFinite (tl_common.h; the GEMM epilogues given the fp32 rows in
+// (grouped: MG = 4 ceil(M / 16), row t % 16 of row group 4 (t / 16) + p instead);
+// a row holding Inf or NaN gets xe = kXeNonFinite (tl_common.h; the GEMM epilogues given the fp32 rows in
 // GemmLaunch.xraw take that row's outputs from them, nonfinite_dot, else NaN)
-hipError_t tlk_launch_split_i8x4(const float* X, int ldx, int M, int K, uint8_t* tiles, int* xe, hipStream_t st);
+hipError_t tlk_launch_split_i8x4(const float* X, int ldx, int M, int K, uint8_t* tiles, int* xe, bool grouped,
+                                 hipStream_t st);
 // 4-byte-word copy by a kernel (bytes % 4 == 0), e.g. from mapped pinned host memory
 hipError_t tlk_launch_copy_words(const void* src, void* dst, size_t bytes, hipStream_t st);
 // dst[0, npad) = src[0, n) followed by zeros, by a kernel (src null when n == 0):
@@ -153,18 +155,18 @@ hipError_t tlk_launch_swiglu_rows(const float* gu, float* mlp, int S, int ffn, h
 //   xe:     the four int8 planes per row (code rows 4t + p, ceil(4 rows / 16)
 //           row groups) and exponents of launch_split_i8x4, bit for bit
 hipError_t tlk_launch_rmsnorm_rows_q(const float* x, const float* w, uint8_t* tiles, float* scales, int* xe,
-                                     int rows, int K, float eps, hipStream_t st);
+                                     int rows, int K, float eps, bool grouped, hipStream_t st);
 // the result of tlk_launch_split_i8x4 with one work-group per row, for
 // K = 1024, 2048, 4096 or 6144 and 16-byte aligned rows (else
 // hipErrorInvalidValue)
 hipError_t tlk_launch_split_rows_planes(const float* x, int ldx, int rows, int K, uint8_t* tiles, int* xe,
-                                        hipStream_t st);
+                                        bool grouped, hipStream_t st);
 // the result of tlk_launch_quantize_rows_tiled (clamp127) with one
 // work-group per row, for the same K and alignment
 hipError_t tlk_launch_quantize_rows_by_row(const float* x, int rows, int K, uint8_t* tiles, float* scales,
                                            hipStream_t st);
 hipError_t tlk_launch_swiglu_rows_q(const float* gu, uint8_t* tiles, float* scales, int* xe, int S, int ffn,
-                                    hipStream_t st);
+                                    bool grouped, hipStream_t st);
 hipError_t tlk_launch_residual_add(const float* y, float* h, long long n, hipStream_t st);
 
 // ---- M=1 GEMV (gemv.hip) --------------------------------------------------
@@ -232,6 +234,7 @@ typedef struct GemmLaunch {
   const int* xe TLK_DEF(nullptr);        // OUT_F32_X4: per-token power-of-two exponents (split_i8x4)
   const float* xraw TLK_DEF(nullptr);    // OUT_F32_X4: the fp32 token rows [M / 4][ldxr] the planes came
   int ldxr TLK_DEF(0);                   //   from (outputs of a non-finite row from them); null: NaN
+  bool planes_grouped TLK_DEF(false);    // OUT_F32_X4: row group 4T + p holds plane p of tokens 16T .. 16T + 15
 } GemmLaunch;
 static inline GemmLaunch tlk_gemm_launch_init(void) {
   GemmLaunch L;
@@ -250,6 +253,9 @@ hipError_t tlk_launch_gemm(const GemmLaunch* L, hipStream_t st);
 // split work-space of the kernel tlk_launch_gemm picks for *L: partial-sum
 // bytes (L->part) and zeroed arrival counters (L->cnt); 0 when none
 void tlk_gemm_needs(const GemmLaunch* L, size_t* part_bytes, size_t* counters);
+// whether the GEMM of M4 = 4 x tokens plane rows takes them grouped
+// (GemmLaunch.planes_grouped; the split launches' `grouped`)
+bool tlk_gemm_planes_grouped(int M4, int N, int K);
 void tlk_gemm_i8_set_cfg(int cfg);   // tuning override of the int8 GEMM (-1 = planner)
 void tlk_gemm_i8_set_split(int s);   // tuning override of its K slices (0 = planner)
 // tuning override of the 16-bit GEMM: tile configuration 0..2 (-1 = planner)
@@ -294,7 +300,8 @@ hipError_t launch_pack_tiles_rows(const int8_t* w, int rows, int cols, int NGt, 
 hipError_t launch_unpack_tiles(const uint8_t* tiles, int rows, int cols, int8_t* w, hipStream_t st);
 hipError_t launch_rmsnorm_np(const float* h, const float* w, float* out, int K, float eps, hipStream_t st);
 hipError_t launch_argmax_keys(const uint64_t* keys, int n, int32_t* token, float* value, hipStream_t st);
-hipError_t launch_split_i8x4(const float* X, int ldx, int M, int K, uint8_t* tiles, int* xe, hipStream_t st);
+hipError_t launch_split_i8x4(const float* X, int ldx, int M, int K, uint8_t* tiles, int* xe, bool grouped,
+                             hipStream_t st);
 hipError_t launch_stream_read(const void* p, size_t bytes, int grid, int u, uint32_t* sink, hipStream_t st);
 hipError_t launch_copy_words(const void* src, void* dst, size_t bytes, hipStream_t st);
 hipError_t launch_copy_pad_bytes(const void* src, size_t n, void* dst, size_t npad, hipStream_t st);
@@ -318,13 +325,13 @@ hipError_t launch_flash_prefill(const float* qkv, const float* kc, const float* 
                                 hipStream_t st);
 hipError_t launch_swiglu_rows(const float* gu, float* mlp, int S, int ffn, hipStream_t st);
 hipError_t launch_split_rows_planes(const float* x, int ldx, int rows, int K, uint8_t* tiles, int* xe,
-                                    hipStream_t st);
+                                    bool grouped, hipStream_t st);
 hipError_t launch_quantize_rows_by_row(const float* x, int rows, int K, uint8_t* tiles, float* scales,
                                        hipStream_t st);
 hipError_t launch_rmsnorm_rows_q(const float* x, const float* w, uint8_t* tiles, float* scales, int* xe, int rows,
-                                 int K, float eps, hipStream_t st);
+                                 int K, float eps, bool grouped, hipStream_t st);
 hipError_t launch_swiglu_rows_q(const float* gu, uint8_t* tiles, float* scales, int* xe, int S, int ffn,
-                                hipStream_t st);
+                                bool grouped, hipStream_t st);
 hipError_t launch_residual_add(const float* y, float* h, long long n, hipStream_t st);
 
 GemvPlan gemv_plan(int N, int K);
@@ -340,10 +347,10 @@ hipError_t launch_gemm(const GemmLaunch& L, hipStream_t st);
 
 // W8A8 LDS-staged int8 MFMA GEMM (gemm_i8.hip), used for M > 16
 hipError_t launch_gemm_i8(const GemmLaunch& L, hipStream_t st);
-int gemm_i8_pick_cfg(int M, int N, int K);
 void gemm_i8_set_cfg(int cfg);
 void gemm_i8_set_split(int s);
-void gemm_i8_needs(int M, int N, int K, size_t* part_bytes, size_t* counters);
+void gemm_i8_needs(const GemmLaunch& L, size_t* part_bytes, size_t* counters);
+bool gemm_planes_grouped(int M4, int N, int K);
 
 // LDS-staged 16-bit MFMA GEMM (gemm_b16.hip): A_BF16 / A_F16, used for M > 16
 // when X rows are 16-byte aligned pieces
