@@ -395,20 +395,19 @@ static GemmKernel gemm_choice(const GemmLaunch& L) {
   // work-group share each fragment): the int8 planes of 5-8 fp32 tokens,
   // 81 -> 70 us for the lm_head at 8 tokens
   const bool b16 = L.amode == A_BF16 || L.amode == A_F16;
-  if (b16) {   // tuning override: 3 the small-M kernel, 0..2 a tile of the tiled one
+  if (b16) {   // tuning override: 3 the small-M kernel, others a configuration of the tiled one
     const int fc = gemm_b16_forced_cfg();
     if (fc == 3 && gemm_small_supported(L)) return GK_SMALL;
     if (((fc >= 0 && fc <= 2) || fc >= 4) && L.M > 16 && gemm_b16_supported(L)) return GK_B16;
   }
-  // 16-bit rows (the grid's y extent over the token groups): up to 256 rows at
-  // N <= 4096 and 64 rows on wider N, measured at K = 2048 against every tile
-  // of the tiled kernel (M = 96 / 128 / 192 / 256, N = 2048: 6.8 / 6.9 / 9.2 /
-  // 9.3 us against 11.5 / 11.5 / 11.6 / 11.8; N = 4096: 9.4 / 9.5 / 14.9 /
-  // 15.0 against 11.8 / 11.9 / 16.1 / 16.2; N = 12288 at 32 / 64 rows 10.3 /
-  // 15.7 against 12.0 / 16.6; from 96 rows there the tiled kernel wins: 20.7
-  // against 25.2 us)
+  // 16-bit rows (the grid's y extent over the token groups), measured against
+  // the tiled kernel's best: 128 rows at N = 2048 / 4096, K = 2048 7.4 / 9.9 us
+  // against 12.2 / 13.9, 256 rows at N = 2048, K = 4096 14.6 against 16.7 (K = 6144
+  // 19.5 against 19.2; N = 4096, K = 4096 24.2 against 21.4), 64 rows at N = 8192,
+  // K = 3072 13.1 against 15.8, at N = 12288 15.6 against 13.8
   const int ng = cdiv(L.N, 16);
-  const bool b16_small = b16 && L.M <= 256 && (ng <= 256 || L.M <= 64);
+  const bool b16_small = b16 && (L.M <= 32 || (L.M <= 64 && ng <= 512) || (L.M <= 128 && ng <= 256) ||
+                                 (L.M <= 256 && ng <= 128 && L.K <= 4096));
   const bool wide_i8 = L.amode == A_I8 && L.M <= 32 && ng >= 2048;
   // int8 codes and fp32 rows: up to 64 rows at N <= 6144 and 32 rows at
   // N <= 12288 (W8A8 at K = 2048, N = 6144, 24..64 rows: 8.1-11.0 us against

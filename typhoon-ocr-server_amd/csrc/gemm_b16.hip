@@ -1,25 +1,23 @@
 // gemm_b16.hip -- prefill GEMMs with 16-bit MFMAs over int8 weight tiles:
 //   A_BF16  W8A16 (kernel/w8a16_kernel.c:203-216): bf16 X x int8 W (exact in
-//           bf16) on v_mfma_f32_16x16x32_bf16, fp32 accumulation, fp32 scale
+//           bf16) on v_mfma_f32_*_bf16, fp32 accumulation, fp32 scale
 //           after the sum, fp32 / bf16 (RNE) / fp16 output.
-//   A_F16   the same with fp16 X on v_mfma_f32_16x16x32_f16.
+//   A_F16   the same with fp16 X on v_mfma_f32_*_f16.
 //
-// Same skeleton as gemm_i8.hip: a ring of NST LDS stage buffers filled by
+// Two kernels: the wave-grid one for every X under 4 GiB, the LDS-staged one
+// (64-bit addresses) past that.  Both are a ring of LDS stage buffers filled by
 // direct global -> LDS copies (one 16-byte piece per lane per copy), one
 // barrier per 64-wide K stage, transposed accumulators (weights as the MFMA's
-// first operand) so each lane stores 4 consecutive output columns.
+// first operand) so each lane holds 4 consecutive output columns.
 //
-// Within a 64-wide K block the int8 weight tile gives lane l row (l & 15) and
-// k = 16 (l >> 4) + 0..15; the bf16 MFMA consumes 8 k per lane, so the block
-// is two MFMAs, half h taking k = 16 (l >> 4) + 8 h + 0..7.  X (row-major in
-// memory) is copied a whole 128-byte row segment per 8 lanes into a swizzled
-// row-major LDS tile (xtile_* below: 2 copies per row group and K block), and
-// a wave reads each MFMA operand with one conflict-free ds_read_b128.  (Copies
-// in MFMA operand order, lane l reading 16 bytes of row l & 15, spread every
-// copy over 16 half-used lines: about 10 B/clk per CU against the int8
-// GEMM's 22-38.)  Weight tiles stay int8 and are widened to bf16/fp16 in
-// registers after the read.  Lanes whose row is past M or whose k is past K
-// copy 16 bytes of zeros.
+// X (row-major in memory) is copied a whole 128-byte row segment per 8 lanes
+// into a swizzled row-major LDS tile (xtile_* below: 2 copies per 16-row group
+// and K block), and a wave reads each MFMA operand with one conflict-free
+// ds_read_b128.  (Copies in MFMA operand order, lane l reading 16 bytes of row
+// l & 15, spread every copy over 16 half-used lines: about 10 B/clk per CU
+// against the int8 GEMM's 22-38.)  Weight tiles stay int8 and are widened to
+// bf16/fp16 in registers after the read.  Lanes whose k is past K copy 16 bytes
+// of zeros.
 #include <algorithm>
 #include <atomic>
 
@@ -40,7 +38,7 @@ struct GemmB16Args {
   int ldy;
   int M, N, K, KB, MG, NG;
   int ntm, ntn;
-  int ep, out;
+  int out;
   const uint8_t* zero_tile;
   int S;                 // K slices per tile (work-groups per tile)
   float* part;           // S > 1: fp32 partial tiles [tiles][S][MT*16 x NT*16]
@@ -98,73 +96,78 @@ __device__ __forceinline__ int xtile_frag(int lane, int h) {
   return j * 64 + r8 * 8 + (kc ^ r8 ^ j);
 }
 
-// The end of a tile's work-group: with K slices (a.S > 1) the K-slice merge,
-// then the epilogue (scale, bias, conversion, stores).  acc[i][j] holds row
-// group rg0 + i (lane: row lane & 15) and column group cg0 + j (lane: columns
-// 4 (lane >> 4) .. + 3); slot0 + i is this wave's slot of row i in the
-// partial tile (the slots of the waves of a work-group do not overlap).
+// K slices (a.S > 1): merges a tile's partial sums; true in the work-group that
+// holds the whole sums afterwards.  acc[i][j] is this wave's fragment in slot
+// slot0 + i of the partial tile (the slots of the waves of a work-group do not
+// overlap).  flag: a word of the stage ring, which no copy or read uses any more
+// (an LDS word of its own would push an 80 KiB ring past two work-groups per CU).
 template <int FM, int FN>
-__device__ __forceinline__ void b16_finish(const GemmB16Args& a, v4f (&acc)[FM][FN], int rg0, int cg0, int slot0,
-                                           int bt, int ks, const float (&e_ws)[FN][4], const float (&e_b)[FN][4]) {
+__device__ __forceinline__ bool b16_merge(const GemmB16Args& a, v4f (&acc)[FM][FN], int slot0, int bt, int ks, int* flag) {
+  const int lane = threadIdx.x & 63;
+  // K slices: every work-group of the tile stores its fp32 sums, waits for
+  // the stores' acknowledgement and counts in; the last to arrive adds the
+  // S slices in slice order (its own from registers, the same sums and
+  // order whichever work-group merges), then runs the epilogue below
+  constexpr int TF = 4 * FM * FN * 256;         // floats per partial tile: 4 waves x FM x FN fragments
+  float* mine = a.part + ((size_t)bt * a.S + ks) * TF;
+#pragma unroll
+  for (int i = 0; i < FM; i++)
+#pragma unroll
+    for (int j = 0; j < FN; j++) st_agent4(mine + (((slot0 + i) * FN + j) * 64 + lane) * 4, acc[i][j]);
+  asm volatile("" ::: "memory");
+  wait_vm<0>();                               // this thread's partial stores are acknowledged
+  asm volatile("" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    *flag = __hip_atomic_fetch_add(a.cnt + bt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(a.S - 1);
+  __syncthreads();
+  if (!*flag) return false;
+  // the merger's acquire: the slices are read after the counter showed
+  // them all arrived (agent scope, once per tile: it invalidates this
+  // CU's caches, so the plain 16-byte loads below fetch what the stores
+  // wrote through).  All S slices come from memory, this work-group's own
+  // too (the values it stored), one slice's loads in flight at a time and
+  // added in slice order.
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  // QB slices' loads are in flight together (indices past S re-read the
+  // last slice and are not added)
+  constexpr int QB = FM * FN <= 2 ? 8 : (FM * FN <= 8 ? 4 : 1);
+  const float* slices = a.part + (size_t)bt * a.S * TF;
+  for (int q0 = 0; q0 < a.S; q0 += QB) {
+    v4f p[QB][FM][FN];
+#pragma unroll
+    for (int u = 0; u < QB; u++)
+#pragma unroll
+      for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+          p[u][i][j] = *reinterpret_cast<const v4f*>(slices + (size_t)min(q0 + u, a.S - 1) * TF +
+                                                    (((slot0 + i) * FN + j) * 64 + lane) * 4);
+#pragma unroll
+    for (int u = 0; u < QB; u++) {
+      if (q0 + u >= a.S) break;
+#pragma unroll
+      for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            acc[i][j][r] = q0 + u == 0 ? p[u][i][j][r] : __fadd_rn(acc[i][j][r], p[u][i][j][r]);
+    }
+  }
+  if (threadIdx.x == 0) __hip_atomic_store(a.cnt + bt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
+// Epilogue of the LDS-staged kernel: scale, bias, conversion, stores.  acc[i][j]
+// holds row group rg0 + i (lane: row lane & 15) and column group cg0 + j (lane:
+// columns 4 (lane >> 4) .. + 3).
+template <int FM, int FN>
+__device__ __forceinline__ void b16_finish(const GemmB16Args& a, v4f (&acc)[FM][FN], int rg0, int cg0,
+                                           const float (&e_ws)[FN][4], const float (&e_b)[FN][4]) {
   const int lane = threadIdx.x & 63;
   const int mrow = lane & 15;
   const int ncol = (lane >> 4) * 4;
-  if (a.S > 1) {
-    // K slices: every work-group of the tile stores its fp32 sums, waits for
-    // the stores' acknowledgement and counts in; the last to arrive adds the
-    // S slices in slice order (its own from registers, the same sums and
-    // order whichever work-group merges), then runs the epilogue below
-    constexpr int TF = 4 * FM * FN * 256;         // floats per partial tile: 4 waves x FM x FN fragments
-    float* mine = a.part + ((size_t)bt * a.S + ks) * TF;
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-      for (int j = 0; j < FN; j++) st_agent4(mine + (((slot0 + i) * FN + j) * 64 + lane) * 4, acc[i][j]);
-    __shared__ int s_last;
-    asm volatile("" ::: "memory");
-    wait_vm<0>();                               // this thread's partial stores are acknowledged
-    asm volatile("" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0)
-      s_last = __hip_atomic_fetch_add(a.cnt + bt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(a.S - 1);
-    __syncthreads();
-    if (!s_last) return;
-    // the merger's acquire: the slices are read after the counter showed
-    // them all arrived (agent scope, once per tile: it invalidates this
-    // CU's caches, so the plain 16-byte loads below fetch what the stores
-    // wrote through).  All S slices come from memory, this work-group's own
-    // too (the values it stored), one slice's loads in flight at a time and
-    // added in slice order.
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    // QB slices' loads are in flight together (indices past S re-read the
-    // last slice and are not added)
-    constexpr int QB = FM * FN <= 2 ? 8 : (FM * FN <= 8 ? 4 : 1);
-    const float* slices = a.part + (size_t)bt * a.S * TF;
-    for (int q0 = 0; q0 < a.S; q0 += QB) {
-      v4f p[QB][FM][FN];
-#pragma unroll
-      for (int u = 0; u < QB; u++)
-#pragma unroll
-        for (int i = 0; i < FM; i++)
-#pragma unroll
-          for (int j = 0; j < FN; j++)
-            p[u][i][j] = *reinterpret_cast<const v4f*>(slices + (size_t)min(q0 + u, a.S - 1) * TF +
-                                                      (((slot0 + i) * FN + j) * 64 + lane) * 4);
-#pragma unroll
-      for (int u = 0; u < QB; u++) {
-        if (q0 + u >= a.S) break;
-#pragma unroll
-        for (int i = 0; i < FM; i++)
-#pragma unroll
-          for (int j = 0; j < FN; j++)
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-              acc[i][j][r] = q0 + u == 0 ? p[u][i][j][r] : __fadd_rn(acc[i][j][r], p[u][i][j][r]);
-      }
-    }
-    if (threadIdx.x == 0) __hip_atomic_store(a.cnt + bt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-
   const bool vec_ok = ((a.ldy & 3) == 0) &&
                       ((((uintptr_t)a.Y) & (a.out == OUT_F32 ? 15 : 7)) == 0);
 #pragma unroll
@@ -179,12 +182,8 @@ __device__ __forceinline__ void b16_finish(const GemmB16Args& a, v4f (&acc)[FM][
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const float c = acc[i][j][r];
-        if (a.ep == EP_SCALE_FMA) {
-          y[r] = __fmaf_rn(c, e_ws[j][r], e_b[j][r]);
-        } else {
-          y[r] = __fmul_rn(c, e_ws[j][r]);
-          if (a.bias) y[r] = __fadd_rn(y[r], e_b[j][r]);
-        }
+        y[r] = __fmul_rn(c, e_ws[j][r]);
+        if (a.bias) y[r] = __fadd_rn(y[r], e_b[j][r]);
       }
       const size_t o = (size_t)m * a.ldy + n;
       const bool full = vec_ok && n + 4 <= a.N;
@@ -211,9 +210,7 @@ __device__ __forceinline__ void b16_finish(const GemmB16Args& a, v4f (&acc)[FM][
   }
 }
 
-// KF: K is a multiple of 64 (every copy a per-lane offset from a uniform
-// per-stage base; the general path masks pieces past K and rows past M)
-template <int AMODE, int MT, int NT, int NST, int WM, int WN, bool KF>
+template <int AMODE, int MT, int NT, int NST, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_b16_lds_kernel(GemmB16Args a) {
   constexpr int NW = WM * WN;
   constexpr int AP = 2;                                // A copies per (row group, K block)
@@ -289,35 +286,19 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_b16_lds_kernel(GemmB16Args 
   // copies would let the last NST-2 steps' waits return before their own
   // stage had landed; waiting for every copy there instead measured 7% slower
   // at M = 64..256.)
-  // K a multiple of 64 (no piece past K) and X under 4 GiB (the launcher's
-  // condition for KF): each copy is a 32-bit per-lane byte offset from a
-  // uniform per-stage base (rows past M read row M - 1; their outputs are
-  // never stored)
-  constexpr bool kfull = KF;
-  uint32_t qvo[PW];
-#pragma unroll
-  for (int p = 0; p < PW; p++)
-    qvo[p] = (uint32_t)(qsrc[p] - (qkoff[p] >= 0 ? Xb : reinterpret_cast<const char*>(a.Bt)));
   auto issue = [&](int st, uint4* buf) {
     const int sc = kb0 + min(st, nst - 1);
     const uint32_t base = lds_addr(buf);
-    if constexpr (kfull) {
-      const char* sa = Xb + (size_t)sc * 64 * ESZ;
-      const char* sb = reinterpret_cast<const char*>(a.Bt) + (size_t)sc * bstride;
 #pragma unroll
-      for (int p = 0; p < PW; p++) dma_tile_s(qvo[p], (wv + NW * p < TA) ? sa : sb, base + qlds[p]);
-    } else {
-#pragma unroll
-      for (int p = 0; p < PW; p++) {
-        const uint4* g;
-        if (qkoff[p] >= 0) {
-          const int k = sc * 64 + qkoff[p];
-          g = (qrow_ok[p] && k < a.K) ? reinterpret_cast<const uint4*>(qsrc[p] + (size_t)sc * 64 * ESZ) : Z4;
-        } else {
-          g = reinterpret_cast<const uint4*>(qsrc[p] + (size_t)sc * bstride);
-        }
-        dma_tile(g, base + qlds[p]);
+    for (int p = 0; p < PW; p++) {
+      const uint4* g;
+      if (qkoff[p] >= 0) {
+        const int k = sc * 64 + qkoff[p];
+        g = (qrow_ok[p] && k < a.K) ? reinterpret_cast<const uint4*>(qsrc[p] + (size_t)sc * 64 * ESZ) : Z4;
+      } else {
+        g = reinterpret_cast<const uint4*>(qsrc[p] + (size_t)sc * bstride);
       }
+      dma_tile(g, base + qlds[p]);
     }
   };
 
@@ -417,7 +398,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_b16_lds_kernel(GemmB16Args 
   }
   wait_vm<0>();   // no copy may still be landing in LDS when the work-group exits
 
-  b16_finish<FM, FN>(a, acc, mg0 + wm * FM, ng0 + wn * FN, wv * FM, bt, ks, e_ws, e_b);
+  if (a.S > 1 && !b16_merge<FM, FN>(a, acc, wv * FM, bt, ks, reinterpret_cast<int*>(s0))) return;
+  b16_finish<FM, FN>(a, acc, mg0 + wm * FM, ng0 + wn * FN, e_ws, e_b);
 }
 
 // One output dword of the widening: int8 elements 2p, 2p + 1 of a lane's 16
@@ -428,8 +410,7 @@ __device__ __forceinline__ uint32_t widen_pair(uint4 w, int p) {
   const int sh = (p & 1) * 16;
   const float f0 = (float)(int8_t)((d >> sh) & 0xff), f1 = (float)(int8_t)((d >> (sh + 8)) & 0xff);
   if constexpr (AMODE == A_F16) {
-    const _Float16 h0 = (_Float16)f0, h1 = (_Float16)f1;
-    return (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(f0, f1));
   } else {
     return __builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
   }
@@ -441,203 +422,295 @@ __device__ __forceinline__ void set_dword(uint4& u, int c, uint32_t v) {
   else u.w = v;
 }
 
-// Column-split variant: the 4 waves split the tile's N columns (wave w owns
-// weight row groups ng0 + FN w .. + FN - 1) and share its MT row groups of X.
-// Each weight tile is private to one wave, so it goes from global memory
-// straight into that wave's registers (one 16-byte load per lane per tile, in
-// MFMA operand order) and is widened once per work-group; only the shared X
-// tiles pass through the LDS ring (2 MT KiB per stage, so the ring holds D
-// stages in 2 MT D KiB).  Per 64-wide K stage and work-group: 2 MT KiB
-// copied into LDS, 8 MT KiB of fragment reads, 4 FN KiB of register loads,
-// 8 MT FN MFMAs.
+// ---------------------------------------------------------------------------
+// Wave-grid kernel: WM x WN waves, each holding a (32 RM) x (32 CN) block of the tile
+// in its accumulation registers (RM x CN accumulators of 32 x 32).  X (swizzled
+// row-major tiles, xtile_*) and the int8 weight tiles of a 64-wide K stage pass
+// through one LDS ring; a wave widens the weights it reads.
 //
-// Pipeline (as the int8 column-split kernel): stage s's copies and loads are
-// issued D steps ahead (weight register set s % (D + 1), LDS buffer s % D).
-// Step s waits for stage s + 1, one barrier makes its X tiles visible and
-// frees buffer s % D, whose copy for stage s + D follows; the MFMAs of stage
-// s run interleaved with the fragment reads of stage s + 1, the issue of
-// stage s + D and the widening of the next weight column, two elements at a
-// time between MFMAs.  Stages past the work-group's K range re-read its last
-// K block (branch-free, so every wait counts exactly); nothing reads what
-// they bring in.  K is a multiple of 64.
-template <int AMODE, int MT, int FN, int D>
-__global__ __launch_bounds__(256) void gemm_b16_wcol_kernel(GemmB16Args a) {
-  constexpr int NW = 4, NT = NW * FN, AP = 2, ESZ = 2;
-  constexpr int TA = MT * AP;          // X copies (1 KiB each) per stage
-  constexpr int PA = TA / NW;          // ... per wave
-  constexpr int NB = D + 1;            // weight register sets
-  constexpr int PS = PA + FN;          // vector memory operations per wave per stage
+// What bounds it is instruction issue: one wave issues an instruction every 8
+// cycles, two waves on a SIMD one every 4.  A widened dword (two weights) costs
+// 3 vector instructions, so a 16 x 16 tile of weights costs 24 and feeds four
+// 32 x 32 x 16 MFMAs (32 cycles each) per 64 rows of X.  Hence 32 x 32 MFMAs
+// (half the instructions of 16 x 16 ones), and two waves per SIMD everywhere:
+// 8 waves on the large tiles, two work-groups per CU on the small ones.  A small
+// tile's waves split its columns only (WM = 1), so that each weight is widened
+// once.  The outputs leave through LDS for the same reason: unrolled over the
+// accumulators, scaling and storing took 17 us per 256 x 192 work-group, now 5.
+// Measured against the column-split kernel before it (bf16 out): 1024 x 12288 x
+// 2048 65 -> 52 us, 333 x 2048 x 6144 40 -> 23 us, 400 x 2048 x 2048 17 -> 14 us.
+// Accumulators are left to the register allocator (at most 256 registers, it
+// keeps them in place; with asm MFMAs pinned to the accumulation registers it
+// copied operands right in front of their use, without the wait states).
+//
+// Stage s lives in ring slot s % NST.  Step s waits until stage s + 1 has
+// landed, one barrier makes it visible and frees slot s % NST; the 8 CN MFMAs
+// of stage s run with the widening of the next operand, the fragment reads of
+// stage s + 1 and the copies of stage s + NST spread between them.  Stages past
+// the work-group's K range re-read its last K block (branch-free, so the wait
+// counts are exact), and nothing reads what they bring in.
+//
+// KF: K is a multiple of 64.  Otherwise the lanes whose 8 columns of X lie past K
+// copy 16 bytes of zeros (the next row's values there could be Inf or NaN, which
+// the weight tile's zero padding would not cancel).
+typedef float v16f __attribute__((ext_vector_type(16)));
+template <int AMODE>
+__device__ __forceinline__ void mfma32_acc(v16f& c, uint4 w, uint4 x) {
+  if constexpr (AMODE == A_F16) c = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_h(w), as_h(x), c, 0, 0, 0);
+  else c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf(w), as_bf(x), c, 0, 0, 0);
+}
+template <int AMODE, int WM, int WN, int RM, int CN, int NST, bool KF>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_b16_wave_kernel(GemmB16Args a) {
+  constexpr int NW = WM * WN;
+  constexpr int MT = 2 * RM * WM, NT = 2 * CN * WN;            // row groups, column groups
+  constexpr int TA = 2 * MT, TS = TA + NT;                // X copies, copies per stage (1 KiB each)
+  constexpr int PA = TA / NW, PW = (TS + NW - 1) / NW;    // copies per wave per stage (PA of them X)
+  constexpr int NMEM = 4 * RM + 2 * CN + PW;                 // memory operations per wave per stage
+  constexpr int NM = 4 * RM * CN;                         // MFMAs per wave per stage
+  constexpr int MO = (NMEM + NM - 1) / NM;                // memory operations behind an MFMA
   static_assert(TA % NW == 0, "X copies must divide over the waves");
-  static_assert(NB % 2 == 0, "fragment double buffer needs an even unroll");
-  static_assert(PS * (D - 1) < 64, "vmcnt range");
-  __shared__ uint4 sA[D * TA * 64];
+  static_assert(NST >= 3 && NST * TS <= 160 && PW * (NST - 1) < 64, "LDS size, vmcnt range");
+  constexpr uint32_t SB = TS * 1024;                      // bytes per stage
+  __shared__ uint4 sS[NST * TS * 64];
 
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wv / WN, wn = wv % WN;
+  // with K slices, work-group b takes slice b / tiles of tile b % tiles
+  constexpr bool SLICES = NW == 4;
+  const int ks = SLICES ? blockIdx.x / (a.ntm * a.ntn) : 0;
+  const int bt = blockIdx.x - ks * a.ntm * a.ntn;
+  int tm, tn;
+  tile_patch(bt, a.ntm, a.ntn, MT >= 16 ? 4 : 8, tm, tn);
+  const int mg0 = tm * MT, ng0 = tn * NT;
+  // this work-group's k-blocks [kb0, kb0 + KB) (divisions run on the vector unit)
+  const int kb0 = SLICES ? __builtin_amdgcn_readfirstlane((ks * a.KB) / a.S) : 0;
+  const int KB = SLICES ? __builtin_amdgcn_readfirstlane(((ks + 1) * a.KB) / a.S) - kb0 : a.KB;
+  const size_t bstep = (size_t)a.NG * 1024;
 
-  // work-group b: K slice b / ntiles of tile b % ntiles (XCD-grouped tile
-  // order as the LDS-staged kernel's)
-  const int ntiles = a.ntm * a.ntn;
-  const int ks = blockIdx.x / ntiles;
-  const int bt = blockIdx.x - ks * ntiles;
-  int t = bt;
-  if (ntiles % 8 == 0) t = (bt % 8) * (ntiles / 8) + bt / 8;
-  const int tn = t / a.ntm, tm = t - (t / a.ntm) * a.ntm;
-  const int mg0 = tm * MT, ng0 = tn * NT + wv * FN;
-  const int KB = a.KB;
-  const int kb0 = (ks * KB) / a.S;
-  const int nst = ((ks + 1) * KB) / a.S - kb0;
-
-  // X copies: copy q = wv + NW p holds rows 8 (q % AP) .. + 7 of row group
-  // q / AP in the swizzled layout of xtile_row / xtile_chunk (rows past M
-  // read row M - 1; their outputs are never stored)
-  const char* Xb = static_cast<const char*>(a.X);
-  uint32_t avo[PA];
+  // Copy p of a stage is q = wv + NW p: X copies first (q < TA; rows 8 (q % 2) ..
+  // + 7 of row group q / 2; q % 2 = wv % 2, so a lane's 16-byte chunk of the row
+  // is the same in all of them), then weight tiles; where NW does not divide TS
+  // the last waves have one copy less.  Rows / columns past the matrix edge
+  // re-read a valid one (never stored).
+  const char* Xb = static_cast<const char*>(a.X) + (size_t)kb0 * 128;
+  const int chunk = xtile_chunk(lane, wv & 1);
+  uint32_t xo[PA];
 #pragma unroll
   for (int p = 0; p < PA; p++) {
-    const int q = wv + NW * p;
-    const int row = min((mg0 + q / AP) * 16 + xtile_row(lane, q % AP), a.M - 1);
-    avo[p] = (uint32_t)(((size_t)row * a.lda + 8 * xtile_chunk(lane, q % AP)) * ESZ);
+    const int row = min((mg0 + (wv >> 1) + NW / 2 * p) * 16 + xtile_row(lane, wv & 1), a.M - 1);
+    xo[p] = (uint32_t)row * (uint32_t)(a.lda * 2) + 16u * chunk;
   }
-  const uint4* B4 = reinterpret_cast<const uint4*>(a.Bt) + lane;
-  const uint4* bsrc[FN];
+  const int kroom = a.K - kb0 * 64 - 8 * chunk;           // stage st's chunk lies inside K while 64 st < kroom
+  const uint8_t* bs[PW - PA];
 #pragma unroll
-  for (int j = 0; j < FN; j++) bsrc[j] = B4 + (size_t)min(ng0 + j, a.NG - 1) * 64;
-  const size_t bstride = (size_t)a.NG * 64;
-  const uint32_t sbase = lds_addr(sA);
-  constexpr uint32_t SBYTES = TA * 1024;
-
-  uint4 wb[NB][FN];
-  auto copy_a = [&](int st, int p) {
-    const int sc = kb0 + min(st, nst - 1);
-    dma_tile_s(avo[p], Xb + (size_t)sc * 64 * ESZ, sbase + (uint32_t)(st % D) * SBYTES + (uint32_t)(wv + NW * p) * 1024u);
-  };
-  auto load_b = [&](int st, int c, int j) { wb[c][j] = bsrc[j][(size_t)(kb0 + min(st, nst - 1)) * bstride]; };
-
-  // epilogue operands first (older than every copy, so the first wait covers them)
-  const int ncol = (lane >> 4) * 4;
-  float e_ws[FN][4], e_b[FN][4];
-#pragma unroll
-  for (int j = 0; j < FN; j++)
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int n = min((ng0 + j) * 16 + ncol + r, a.N - 1);
-      e_ws[j][r] = a.ws[n];
-      e_b[j][r] = a.bias ? a.bias[n] : 0.0f;
+  for (int p = 0; p < PW - PA; p++)
+    bs[p] = a.Bt + kb0 * bstep + (size_t)min(ng0 + wv + NW * p, a.NG - 1) * 1024;
+  constexpr bool EVEN = TS % NW == 0;
+  const bool last = EVEN || wv < TS % NW;                 // this wave has copy PW - 1
+  const uint32_t lane16 = lane * 16;
+  const uint32_t sbase = lds_addr(sS);
+  auto copy = [&](int sc, uint32_t slot, int p) {
+    const uint32_t dst = sbase + slot + (uint32_t)(wv + NW * p) * 1024u;
+    if (p >= PA) {
+      if (EVEN || p < PW - 1 || last) dma_tile_s(lane16, bs[p - PA] + (size_t)sc * bstep, dst);
+    } else if (KF) {
+      dma_tile_s(xo[p], Xb + (size_t)sc * 128, dst);
+    } else {
+      uint32_t o = xo[p];
+      asm volatile("" : "+v"(o));                         // no 64-bit address is kept per copy
+      const char* g = Xb + (size_t)sc * 128 + o;
+      if (sc * 64 >= kroom) g = reinterpret_cast<const char*>(a.zero_tile);
+      dma_tile(reinterpret_cast<const uint4*>(g), dst);
     }
-
-  v4f acc[MT][FN];
-#pragma unroll
-  for (int i = 0; i < MT; i++)
-#pragma unroll
-    for (int j = 0; j < FN; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  uint4 fa[2][TA];
-  const int xf[AP] = {xtile_frag(lane, 0), xtile_frag(lane, 1)};
-  auto read_frags = [&](int st, int c) {
-    const uint4* buf = sA + (size_t)(st % D) * (TA * 64);
-#pragma unroll
-    for (int i = 0; i < TA; i++) fa[c][i] = buf[(i / AP) * AP * 64 + xf[i % AP]];
+  };
+  auto wait_stages = [&](auto n) {                        // all but the latest n stages' copies landed
+    if (EVEN || last) wait_vm<PW * n()>();
+    else wait_vm<(PW - 1) * n()>();
   };
 
-  // prologue: stages 0 .. D-1 in flight, stage 0 visible and its fragments read
+  v16f acc[RM][CN];
 #pragma unroll
-  for (int b = 0; b < D; b++) {
+  for (int i = 0; i < RM; i++)
 #pragma unroll
-    for (int p = 0; p < PA; p++) copy_a(b, p);
+    for (int j = 0; j < CN; j++)
 #pragma unroll
-    for (int j = 0; j < FN; j++) load_b(b, b, j);
+      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+
+  // Operands of a 32 x 32 x 16 MFMA: lane l holds row l & 31 of its matrix and 8
+  // values of K.  MFMA (u, h) of a stage takes k = 32 u + 16 (l >> 5) + 8 h + 0..7,
+  // so a lane's 16 weight bytes (k = 32 u + 16 (l >> 5) + 0..15) are its operands
+  // for h = 0 and 1.
+  uint4 fa[2][RM][4], fb[2][CN][2], wc[2];                 // X operands, int8 weights, widened operands
+  const int half = (lane >> 4) & 1;                       // which of a block's two 16-row groups
+  const uint4* ra[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    const int rr = lane & 15, j = rr >> 3, r8 = rr & 7, kc = 4 * (t >> 1) + 2 * (lane >> 5) + (t & 1);
+    ra[t] = sS + (wm * 2 * RM + half) * 128 + j * 64 + r8 * 8 + (kc ^ r8 ^ j);   // xtile layout
   }
-  wait_vm<PS * (D - 1)>();
+  const uint4* rb = sS + (TA + wn * 2 * CN + half) * 64 + (lane & 15) + 16 * (lane >> 5);
+
+  // prologue: stages 0 .. NST-1 in flight, stage 0's fragments read
+#pragma unroll
+  for (int b = 0; b < NST; b++)
+#pragma unroll
+    for (int p = 0; p < PW; p++) copy(min(b, KB - 1), b * SB, p);
+  wait_stages([]() constexpr { return NST - 1; });
   stage_barrier();
-  read_frags(0, 0);
+#pragma unroll
+  for (int q = 0; q < 2 * CN; q++) fb[0][q >> 1][q & 1] = rb[(q >> 1) * 128 + (q & 1) * 32];
+#pragma unroll
+  for (int q = 0; q < 4 * RM; q++) fa[0][q >> 2][q & 3] = ra[q & 3][(q >> 2) * 256];
 
-  // step s (weight set b = s % NB, fragment set f = s & 1)
-  auto step = [&](int st, int b, int f) {
-    wait_vm<PS * (D - 2)>();   // stage s + 1 landed (this wave's part)
-    wait_lgkm0();              // this wave's reads of stage s are done
-    stage_barrier();           // stage s + 1 visible; buffer s % D free
-    constexpr int NMEM = TA + PS;
-    const int nb = (b + D) % NB;
+  uint32_t slot = 0;                                      // slot of stage s (bytes)
+  auto step = [&](int st, int c) {
+    wait_stages([]() constexpr { return NST - 2; });      // stage s + 1 landed (this wave's part)
+    wait_lgkm0();                                         // this wave's reads of stage s are done
+#pragma unroll
+    for (int q = 0; q < 4; q++) set_dword(wc[0], q, widen_pair<AMODE>(fb[c][0][0], q));
+    __builtin_amdgcn_sched_barrier(0);
+    stage_barrier();                                      // stage s + 1 visible; slot of stage s free
+    const uint32_t nxt = slot + SB == NST * SB ? 0u : slot + SB;
+    const int sc = min(st + NST, KB - 1);
     auto mem_op = [&](int q) {
-      if (q < PA) copy_a(st + D, q);
-      else if (q < PS) load_b(st + D, nb, q - PA);
-      else fa[f ^ 1][q - PS] = sA[(size_t)((st + 1) % D) * (TA * 64) + ((q - PS) / AP) * AP * 64 + xf[(q - PS) % AP]];
-    };
-    uint4 wcol[2][2];          // widened weight column j (set j & 1): the two K halves
-#pragma unroll
-    for (int p = 0; p < 8; p++) set_dword(wcol[0][p >> 2], p & 3, widen_pair<AMODE>(wb[b][0], p));
-    __builtin_amdgcn_sched_barrier(0);
-    constexpr int NM = 2 * MT;           // MFMAs per weight column
-#pragma unroll
-    for (int j = 0; j < FN; j++) {
-#pragma unroll
-      for (int u = 0; u < NM; u++) {
-        const int h = u / MT, i = u % MT;
-        acc[i][j] = mfma16<AMODE>(wcol[j & 1][h], fa[f][i * AP + h], acc[i][j]);
-        __builtin_amdgcn_sched_barrier(0);
-        const int m = j * NM + u;
-        if (m < NMEM) mem_op(m);
-        // the next column's widening, one output dword per MFMA slot
-        if (j + 1 < FN && u < 8) set_dword(wcol[(j + 1) & 1][u >> 2], u & 3, widen_pair<AMODE>(wb[b][j + 1], u));
-        __builtin_amdgcn_sched_barrier(0);
+      if (q < 2 * CN) fb[c ^ 1][q >> 1][q & 1] = rb[nxt / 16 + (q >> 1) * 128 + (q & 1) * 32];
+      else if (q < 2 * CN + 4 * RM) {
+        const int f = q - 2 * CN;
+        fa[c ^ 1][f >> 2][f & 3] = ra[f & 3][nxt / 16 + (f >> 2) * 256];
+      } else {
+        copy(sc, slot, q - 2 * CN - 4 * RM);
       }
+    };
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+      const int ph = m / RM, i = m % RM, j = ph >> 2, t = ph & 3;   // phase ph: K part t = 2 u + h of column j
+      // the next phase's operand, spread before this phase's MFMAs
+      if (ph + 1 < 4 * CN) {
+        const int nj = (ph + 1) >> 2, nt = (ph + 1) & 3;
+#pragma unroll
+        for (int q = 4 / RM * i; q < 4 / RM * (i + 1); q++)
+          set_dword(wc[(ph + 1) & 1], q, widen_pair<AMODE>(fb[c][nj][nt >> 1], 4 * (nt & 1) + q));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      mfma32_acc<AMODE>(acc[i][j], wc[ph & 1], fa[c][i][t]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = m * MO; q < (m + 1) * MO; q++)
+        if (q < NMEM) mem_op(q);
+      __builtin_amdgcn_sched_barrier(0);
     }
-#pragma unroll
-    for (int q = FN * NM; q < NMEM; q++) mem_op(q);
-    __builtin_amdgcn_sched_barrier(0);
+    slot = nxt;
   };
-  const int kfull = nst - nst % NB;
-  for (int st = 0; st < kfull; st += NB) {
-#pragma unroll
-    for (int b = 0; b < NB; b++) step(st + b, b, b & 1);
+  // two steps a round, so that the fragment set is a compile-time constant
+  int st = 0;
+  for (; st + 2 <= KB; st += 2) {
+    step(st, 0);
+    step(st + 1, 1);
   }
-#pragma unroll
-  for (int b = 0; b < NB - 1; b++)
-    if (kfull + b < nst) step(kfull + b, b, b & 1);
-
+  if (st < KB) step(st, 0);
   wait_vm<0>();   // no copy may still be landing in LDS when the work-group exits
 
-  b16_finish<MT, FN>(a, acc, mg0, ng0, wv * MT, bt, ks, e_ws, e_b);
+  // the sums as 4-column pieces: piece g of block (i, j) is row 32 i + (lane & 31),
+  // columns 32 j + 8 g + 4 (lane >> 5) .. + 3 of the wave's block
+  v4f sum[RM][4 * CN];
+#pragma unroll
+  for (int i = 0; i < RM; i++)
+#pragma unroll
+    for (int q = 0; q < 4 * CN; q++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) sum[i][q][r] = acc[i][q >> 2][4 * (q & 3) + r];
+  if constexpr (SLICES) {
+    if (a.S > 1 && !b16_merge<RM, 4 * CN>(a, sum, wv * RM, bt, ks, reinterpret_cast<int*>(sS))) return;
+  }
+
+  // Epilogue.  A wave's outputs go through its own part of LDS, 32 rows at a time,
+  // already scaled and in the output type, and leave as 16 bytes per lane of
+  // consecutive columns (stored straight from the accumulators a store covers 16
+  // or 32 bytes of each of 32 rows).
+  constexpr int COLS = 32 * CN;
+  constexpr int LDB = 4 * COLS + 16;                      // bytes per LDS row (fp32; 16-bit rows use half)
+  static_assert(NW * 32 * LDB <= NST * TS * 1024, "rows of a pass fit the ring");
+  uint8_t* const lw = reinterpret_cast<uint8_t*>(sS) + wv * (32 * LDB);
+  const int n0 = (ng0 + wn * 2 * CN) * 16;
+  const int lrow = lane & 31, lcol = 4 * (lane >> 5);
+  const bool wide = a.out == OUT_F32;
+  const int esz = wide ? 4 : 2;
+  const bool vec = (a.ldy * esz) % 16 == 0 && (((uintptr_t)a.Y) & 15) == 0;
+  const int room = min(COLS, a.N - n0);                   // the wave's columns inside N
+  v4f ws[4 * CN], b[4 * CN];
+#pragma unroll
+  for (int q = 0; q < 4 * CN; q++) {
+    // scales are padded with zeros to 16 NG
+    ws[q] = *reinterpret_cast<const v4f*>(a.ws + min(n0 + 8 * q + lcol, a.NG * 16 - 4));
+#pragma unroll
+    for (int r = 0; r < 4; r++) b[q][r] = a.bias ? a.bias[min(n0 + 8 * q + lcol + r, a.N - 1)] : 0.0f;
+  }
+  __syncthreads();                                        // every wave's fragment reads are done
+#pragma unroll
+  for (int i = 0; i < RM; i++) {
+    const int m0 = (mg0 + wm * 2 * RM + 2 * i) * 16;
+#pragma unroll
+    for (int q = 0; q < 4 * CN; q++) {
+      v4f y;
+#pragma unroll
+      for (int r = 0; r < 4; r++) y[r] = __fmul_rn(sum[i][q][r], ws[q][r]);
+      if (a.bias) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) y[r] = __fadd_rn(y[r], b[q][r]);
+      }
+      if (wide) {
+        *reinterpret_cast<v4f*>(lw + lrow * LDB + (8 * q + lcol) * 4) = y;
+      } else {
+        uint2 h;
+        if (a.out == OUT_BF16) {
+          h = make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+        } else {
+          h = make_uint2(pack_f16x2(y[0], y[1]), pack_f16x2(y[2], y[3]));
+        }
+        *reinterpret_cast<uint2*>(lw + lrow * (LDB / 2) + (8 * q + lcol) * 2) = h;
+      }
+    }
+    auto rows_out = [&](auto width) {
+      constexpr int E = width(), PC = 16 / E, CPR = COLS / PC;   // bytes per output, outputs per piece, pieces per row
+#pragma unroll 4
+      for (int t = 0; t < 32 * CPR / 64; t++) {
+        const int c = t * 64 + lane, r = c / CPR, col = (c - r * CPR) * PC;
+        const v4i v = *reinterpret_cast<const v4i*>(lw + r * (LDB * E / 4) + col * E);
+        uint8_t* yp = static_cast<uint8_t*>(a.Y) + ((size_t)(m0 + r) * a.ldy + n0 + col) * E;
+        if (m0 + r >= a.M) continue;
+        if (vec && col + PC <= room) {
+          if (E == 4) __builtin_nontemporal_store(v, reinterpret_cast<v4i*>(yp));   // streaming, as the int8 GEMM's
+          else *reinterpret_cast<v4i*>(yp) = v;
+        } else {
+#pragma unroll
+          for (int k = 0; k < PC; k++) {
+            if (col + k >= room) continue;
+            if (E == 4) reinterpret_cast<int*>(yp)[k] = v[k];
+            else reinterpret_cast<uint16_t*>(yp)[k] = (uint16_t)((uint32_t)v[k >> 1] >> (16 * (k & 1)));
+          }
+        }
+      }
+    };
+    if (wide) rows_out([]() constexpr { return 4; });
+    else rows_out([]() constexpr { return 2; });
+  }
 }
 
 // ---------------------------------------------------------------------------
 // planning and launch
 // ---------------------------------------------------------------------------
-// cfg 0  128 x 192 tiles, 4-deep ring (112 KiB)
-// cfg 1   64 x 128 tiles, 8-deep ring (128 KiB)
-// cfg 2   32 x  64 tiles, 8-deep ring (64 KiB)
-// The smaller tiles exist for mid-size M (64 < M <= 512) with small N, where
-// the larger ones leave most CUs idle.
-// cfg 4  128 x 192 tiles, column-split (weights to registers), 5-deep X ring (80 KiB)
-// cfg 5  128 x 192 tiles, column-split, 7-deep X ring (112 KiB)
-// cfg 6  128 x 128 tiles, column-split, 7-deep X ring (112 KiB)
-// cfg 7   64 x 192 tiles, column-split, 7-deep X ring (56 KiB)
-// cfg 8   64 x 128 tiles, column-split, 9-deep X ring (72 KiB; two work-groups
-//         share a CU.  11- and 13-deep rings measured no faster with one
-//         work-group per CU and 20-35% slower where a CU runs several)
-// (the column-split kernel needs K % 64 == 0; other K run cfg 0's tiles)
+// cfg 0: LDS-staged kernel, 128 x 192 tiles
+// cfg 4..8: wave-grid kernel, 256 x 192 and 256 x 128 (8 waves), 128 x 128 (two
+//   work-groups per CU), 64 x 128 tiles with a 5-deep (two per CU) or 3-deep
+//   ring (three per CU)
 static void b16_cfg(int cfg, int& mt, int& nt) {
-  if (cfg >= 4) {
-    mt = cfg >= 7 ? 4 : 8;
-    nt = (cfg == 6 || cfg == 8) ? 8 : 12;
-    return;
-  }
-  mt = (cfg == 0) ? 8 : (cfg == 1 ? 4 : 2);
-  nt = (cfg == 0) ? 12 : (cfg == 1 ? 8 : 4);
+  static const int dims[9][2] = {{8, 12}, {0, 0}, {0, 0}, {0, 0}, {16, 12}, {16, 8}, {8, 8}, {4, 8}, {4, 8}};
+  mt = dims[cfg][0];
+  nt = dims[cfg][1];
 }
 
-// Plan: tile configuration and K slices, from the measured W8A16 sweep
-// (M = 64 .. 1024, N = 2048 .. 12288, K = 2048, every configuration and
-// 1..8 slices).  K a multiple of 64: the column-split kernel (b16_plan).
-// Other K, the LDS-staged kernel: the 32 x 64 tiles while they number at
-// most 512 (two work-groups of 64 KiB share a CU), else the 64 x 128 tiles
-// while they fit one wave of 256 CUs, else the 128 x 192 tiles while they
-// do, else the configuration whose tile count best fills 256 CUs.  The loop is bound by
-// the latency of its stage copies rather than by bytes, so K slices pay only
-// where the tiles are few: at most 64 tiles are split until 256 work-groups
-// run (M = 64, N = 2048: 11.4 -> 10.5 us); with more tiles the slices' store,
-// arrival and reload cost more than they save.
+// tuning overrides; atomic, since a setter may run while other threads plan launches
 static std::atomic<int> g_b16_force_cfg{-1};
 static std::atomic<int> g_b16_force_split{0};
 void gemm_b16_set_plan(int cfg, int split) {
@@ -658,63 +731,63 @@ static int b16_tiles(int cfg, int MG, int NG) {
   return cdiv(MG, mt) * cdiv(NG, nt);
 }
 
-static void b16_plan(int MG, int NG, int KB, bool kf, int& cfg_out, int& split_out) {
-  int best;
-  if (kf) {
-    // column-split kernel: the configuration of least estimated time, rounds
-    // of 256 work-groups times the measured time of one work-group at
-    // K = 2048 (one per CU, bound by its per-CU load rate: 64 x 128 tiles
-    // 16.0 us, 64 x 192 20.5, 128 x 128 23.3, 128 x 192 30.3; MI355X sweep of
-    // M = 64..1024, N = 2048..12288, every configuration)
-    static const int kc[4] = {8, 7, 6, 4};
-    static const float kt[4] = {16.0f, 20.5f, 23.3f, 30.3f};
-    best = 8;
-    float tbest = 3.0e38f;
-    for (int c = 0; c < 4; c++) {
-      const float t = (float)cdiv(b16_tiles(kc[c], MG, NG), 256) * kt[c];
-      if (t < tbest) {
-        tbest = t;
-        best = kc[c];
+// Plan: the configuration and K slices of least estimated time, rounds of
+// work-groups times the time of one over KB k-blocks, the constants fitted to
+// measured launches (148 shapes: 40..2048 rows, N = 1024..12288, K = 1024..6144;
+// the choice is on average 0.8 % and at most 10 % slower than the best of its
+// shape).  K slices (the 4-wave configurations take them) cost a merge of three
+// dependent memory round trips, so they pay only where the tiles leave most CUs
+// idle: up to 96 tiles (333 x 2048 x 6144: 30.6 us unsplit, 23.3 with 4 slices of
+// 128 x 128; 1024 x 2048 x 6144, 128 tiles: 38.2 with 2, 34.1 unsplit).
+static void b16_plan(int MG, int NG, int KB, bool off32, int& cfg_out, int& split_out) {
+  int cfg = 0, split = 1;
+  if (off32) {
+    float best = 3.0e38f;
+    auto offer = [&](int c, int s, float us) {
+      if (us < best) {
+        best = us;
+        cfg = c;
+        split = s;
       }
-    }
-  } else if (b16_tiles(2, MG, NG) <= 512) best = 2;
-  else if (b16_tiles(1, MG, NG) <= 256) best = 1;
-  else if (b16_tiles(0, MG, NG) <= 256) best = 0;
-  else {
-    best = 0;
-    double best_eff = -1.0;
-    for (int cfg : {0, 1, 2}) {
-      const int tiles = b16_tiles(cfg, MG, NG);
-      const double eff = (double)tiles / (cdiv(tiles, 256) * 256);
-      if (eff > best_eff + 1e-9) {
-        best_eff = eff;
-        best = cfg;
+    };
+    // 8 waves, one work-group per CU
+    offer(4, 1, cdiv(b16_tiles(4, MG, NG), 256) * (11.0f + 1.0f * KB));
+    offer(5, 1, cdiv(b16_tiles(5, MG, NG), 256) * (6.6f + 0.64f * KB));
+    // 4 waves, work-groups share CUs: the time of a k-block grows with each half
+    // round of 256
+    static const float fixed[3] = {6.2f, 5.2f, 4.7f}, alone[3] = {0.40f, 0.253f, 0.265f},
+                       shared[3] = {0.438f, 0.25f, 0.234f}, merge[2] = {4.6f, 4.3f};
+    for (int c = 6; c <= 8; c++) {
+      const int tiles = b16_tiles(c, MG, NG);
+      for (int s = 1; s <= (c < 8 && tiles <= 96 ? 4 : 1) && s <= KB; s++) {
+        const float half = 0.5f * (float)cdiv(tiles * s, 128), kb = (float)KB / s;
+        offer(c, s, fixed[c - 6] + (tiles * s <= 256 ? kb * alone[c - 6] : kb * shared[c - 6] * half + 1.2f * (half - 1.0f)) +
+                        (s > 1 ? merge[c - 6] + 0.0018f * tiles * s : 0.0f));
       }
     }
   }
-  const int tiles = b16_tiles(best, MG, NG);
-  int sp = 1;
-  if (tiles <= 64) sp = std::min(std::max(1, 256 / tiles), std::max(1, KB / 8));
-  sp = std::min(sp, 4);
   const int fc = g_b16_force_cfg.load(std::memory_order_relaxed);
   const int fs = g_b16_force_split.load(std::memory_order_relaxed);
-  if ((fc >= 0 && fc <= 2) || fc >= 4) best = fc;
-  if (best >= 4 && !kf) best = 0;   // the column-split kernel needs K % 64 == 0
-  if (fs > 0) sp = std::min(fs, std::max(1, KB));
-  cfg_out = best;
-  split_out = sp;
+  if (fc >= 0 && fc != 3) {
+    cfg = fc >= 4 && off32 ? fc : 0;
+    split = 1;
+  }
+  if (fs > 0) split = std::min(fs, std::max(1, KB));
+  if (split > 1 && (cfg == 4 || cfg == 5)) cfg = 6;   // the 4-wave configurations take slices
+  cfg_out = cfg;
+  split_out = split;
 }
 
 // partial-sum bytes and arrival counters the launch of this shape needs (the
-// larger of the two plans: whether the launch takes the K-multiple-of-64 path
-// also depends on the row stride, which is not known here)
+// larger of the two plans: which one the launch takes depends on the row stride,
+// which is not known here)
 void gemm_b16_needs(int M, int N, int K, size_t* part_bytes, size_t* counters) {
   const int MG = cdiv(M, 16), NG = cdiv(N, 16);
   *part_bytes = 0;
   *counters = 0;
-  for (int kf = 0; kf < 2; kf++) {
+  for (int off32 = 0; off32 < 2; off32++) {
     int cfg, sp, mt, nt;
-    b16_plan(MG, NG, cdiv(K, 64), kf != 0 && K % 64 == 0, cfg, sp);
+    b16_plan(MG, NG, cdiv(K, 64), off32 != 0, cfg, sp);
     b16_cfg(cfg, mt, nt);
     const size_t tiles = (size_t)cdiv(MG, mt) * cdiv(NG, nt);
     if (sp > 1) {
@@ -724,33 +797,22 @@ void gemm_b16_needs(int M, int N, int K, size_t* part_bytes, size_t* counters) {
   }
 }
 
-template <int AMODE, bool KF>
-static void launch_b16(const GemmB16Args& a, int cfg, dim3 grid, dim3 block, hipStream_t st) {
-  if constexpr (KF) {
-    if (cfg == 4) {
-      hipLaunchKernelGGL((gemm_b16_wcol_kernel<AMODE, 8, 3, 5>), grid, block, 0, st, a);
-      return;
-    }
-    if (cfg == 5) {
-      hipLaunchKernelGGL((gemm_b16_wcol_kernel<AMODE, 8, 3, 7>), grid, block, 0, st, a);
-      return;
-    }
-    if (cfg == 6) {
-      hipLaunchKernelGGL((gemm_b16_wcol_kernel<AMODE, 8, 2, 7>), grid, block, 0, st, a);
-      return;
-    }
-    if (cfg == 7) {
-      hipLaunchKernelGGL((gemm_b16_wcol_kernel<AMODE, 4, 3, 7>), grid, block, 0, st, a);
-      return;
-    }
-    if (cfg == 8) {
-      hipLaunchKernelGGL((gemm_b16_wcol_kernel<AMODE, 4, 2, 9>), grid, block, 0, st, a);
-      return;
-    }
+template <int AMODE, int WM, int WN, int RM, int CN, int NST>
+static void launch_b16_wave(const GemmB16Args& a, int blocks, hipStream_t st) {
+  const dim3 grid(blocks), block(64 * WM * WN);
+  if (a.K % 64 == 0) hipLaunchKernelGGL((gemm_b16_wave_kernel<AMODE, WM, WN, RM, CN, NST, true>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((gemm_b16_wave_kernel<AMODE, WM, WN, RM, CN, NST, false>), grid, block, 0, st, a);
+}
+template <int AMODE>
+static void launch_b16(const GemmB16Args& a, int cfg, int blocks, hipStream_t st) {
+  switch (cfg) {
+    case 0: hipLaunchKernelGGL((gemm_b16_lds_kernel<AMODE, 8, 12, 4, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;
+    case 4: launch_b16_wave<AMODE, 4, 2, 2, 3, 3>(a, blocks, st); break;
+    case 5: launch_b16_wave<AMODE, 2, 4, 4, 1, 4>(a, blocks, st); break;
+    case 6: launch_b16_wave<AMODE, 1, 4, 4, 1, 3>(a, blocks, st); break;
+    case 7: launch_b16_wave<AMODE, 1, 4, 2, 1, 5>(a, blocks, st); break;
+    default: launch_b16_wave<AMODE, 1, 4, 2, 1, 3>(a, blocks, st); break;
   }
-  if (cfg == 0) hipLaunchKernelGGL((gemm_b16_lds_kernel<AMODE, 8, 12, 4, 2, 2, KF>), grid, block, 0, st, a);
-  else if (cfg == 1) hipLaunchKernelGGL((gemm_b16_lds_kernel<AMODE, 4, 8, 8, 2, 2, KF>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((gemm_b16_lds_kernel<AMODE, 2, 4, 8, 2, 2, KF>), grid, block, 0, st, a);
 }
 
 bool gemm_b16_supported(const GemmLaunch& L) {
@@ -761,7 +823,7 @@ bool gemm_b16_supported(const GemmLaunch& L) {
 }
 
 hipError_t launch_gemm_b16(const GemmLaunch& L, hipStream_t st) {
-  if (!gemm_b16_supported(L)) return hipErrorInvalidValue;
+  if (!gemm_b16_supported(L) || L.ep != EP_SCALE) return hipErrorInvalidValue;
   GemmB16Args a;
   a.X = L.A;
   a.lda = L.lda;
@@ -776,14 +838,13 @@ hipError_t launch_gemm_b16(const GemmLaunch& L, hipStream_t st) {
   a.KB = cdiv(L.K, 64);
   a.MG = cdiv(L.M, 16);
   a.NG = cdiv(L.N, 16);
-  a.ep = L.ep;
   a.out = L.out;
   a.zero_tile = L.zero_tile;
   int best, sp;
-  // K a multiple of 64, and every X byte offset fits the copies' 32-bit
-  // per-lane offsets (else the general path, with 64-bit addresses)
-  const bool kf = (L.K % 64) == 0 && (size_t)L.M * (size_t)L.lda * 2 < ((size_t)1 << 32);
-  b16_plan(a.MG, a.NG, a.KB, kf, best, sp);
+  // the wave-grid kernel where every X byte offset fits 32 bits, else the
+  // LDS-staged one with its 64-bit addresses
+  const bool off32 = (size_t)L.M * (size_t)L.lda * 2 < ((size_t)1 << 32);
+  b16_plan(a.MG, a.NG, a.KB, off32, best, sp);
   int mt, nt;
   b16_cfg(best, mt, nt);
   a.ntm = cdiv(a.MG, mt);
@@ -795,14 +856,8 @@ hipError_t launch_gemm_b16(const GemmLaunch& L, hipStream_t st) {
   const long long blocks_ll = (long long)a.ntm * a.ntn * sp;
   if (blocks_ll > 0x7fffffffLL) return hipErrorInvalidValue;
   const int blocks = (int)blocks_ll;
-  const dim3 grid(blocks), block(256);
-  if (L.amode == A_BF16) {
-    if (kf) launch_b16<A_BF16, true>(a, best, grid, block, st);
-    else launch_b16<A_BF16, false>(a, best, grid, block, st);
-  } else {
-    if (kf) launch_b16<A_F16, true>(a, best, grid, block, st);
-    else launch_b16<A_F16, false>(a, best, grid, block, st);
-  }
+  if (L.amode == A_BF16) launch_b16<A_BF16>(a, best, blocks, st);
+  else launch_b16<A_F16>(a, best, blocks, st);
   return hipGetLastError();
 }
 

@@ -88,21 +88,6 @@ __device__ __forceinline__ void tile_of(int b, int ntm, int ntn, int& tm, int& t
   }
 }
 
-// The quadrant kernel's order, for any tile counts: XCD x owns an eighth of the
-// tiles, consecutive in an order that walks bands of gm tile rows column by
-// column, so that the tiles an XCD runs at once are a patch of gm rows and its
-// L2 fills gm row panels and as many columns (against tile_of over a sweep of
-// 130 shapes: 6 % faster where the columns divide over the XCDs and tiles
-// number more than 128, 10 % where they do not, equal below).
-__device__ __forceinline__ void tile_patch(int b, int ntm, int ntn, int gm, int& tm, int& tn) {
-  const int n = ntm * ntn, x = b % 8;
-  const int u = x * (n / 8) + min(x, n % 8) + b / 8;      // a bijection of [0, n)
-  const int grp = u / (gm * ntn), r = u - grp * gm * ntn;
-  const int rows = min(gm, ntm - gm * grp);
-  tm = gm * grp + r % rows;
-  tn = r / rows;
-}
-
 // K slices (a.S > 1): every work-group of the tile stores its int32 sums
 // (16-byte write-through stores), waits for their acknowledgement and counts
 // in; the last to arrive adds the S slices into its accumulators (exact integer
