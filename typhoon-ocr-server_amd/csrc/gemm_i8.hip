@@ -370,26 +370,26 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_lds_kernel(GemmI8Args a)
 }
 
 // ---------------------------------------------------------------------------
-// Quadrant kernel: tiles of 32 FM x 32 FN outputs, 4 waves, each holding one
-// (16 FM) x (16 FN) quadrant in its accumulator registers (FM = FN = 8: 64
-// accumulators, 256 registers, one work-group per CU; up to 24 accumulators two
-// work-groups share a CU).  What bounds small tiles is the movement of
-// operands: per 64-wide K stage a wave reads FM + FN fragments (1 KiB each) for
-// FM FN MFMAs of 16 cycles, and the four waves share 128 B/clk of LDS, so 4 x 4
-// fragments per wave spend 384 LDS cycles (reads and the stage's copies) under
-// 256 MFMA cycles, 8 x 8 spend 768 under 1024, and 8 x 8 pulls 32 B/clk per CU
-// from L2 where 64 x 128 tiles need 96.  Measured against the kernels before it
-// (64 x 128 tiles with weights straight to registers): 2048 tokens of planes
-// over N = 12288, K = 2048 (split included) 316 -> 179 us (2.3 POP/s), 1200
-// tokens 190 -> 110 us; 1200 x 12288 x 2048 codes (128 x 128 LDS-staged tiles)
-// 58 -> 41 us.  One 256 x 256 work-group alone takes 0.47 us per stage (91 % of
-// the MFMA rate), 256 of them 0.67 us (the clock gives way).
+// Quadrant kernel: tiles of 16 WM FM x 32 FN outputs, WM x 2 waves, each holding
+// a (16 FM) x (16 FN) block in its accumulators.  What bounds small tiles is the
+// movement of operands: per 64-wide K stage a wave reads FM + FN fragments (1 KiB
+// each) for FM FN MFMAs of 16 cycles, and a 256 x 256 tile pulls 32 B/clk per CU
+// from L2 where 64 x 128 tiles need 96.  Two waves per SIMD keep the matrix pipe
+// fed through each other's reads, copies and barriers (one wave issues an
+// instruction every 8-9 cycles, two every 5): 8 waves on 256 x 256 tiles (4 waves
+// of twice the block, in 512 registers: 116 -> 109 us at 1200 tokens of planes
+// over N = 12288, K = 2048), two work-groups per CU on 128-row ones.  256 x 192
+// tiles keep 4 waves (8 waves: 54 -> 57 us at N = 2048, K = 6144).  Against the
+// kernels before it (64 x 128 tiles with weights straight to registers): 2048
+// tokens of planes over N = 12288, K = 2048 (split included) 313 -> 173 us (2.4
+// POP/s), 1200 x 12288 x 2048 codes (128 x 128 LDS-staged tiles) 59 -> 45 us.  A
+// stage of 256 x 256 takes 0.43 us at the MFMA rate, 0.58 on 152 CUs, 0.67 on all
+// (the clock gives way).
 //
 // Stage s lives in ring slot s % NST.  Step s waits until stage s + 1 has
 // landed, one barrier makes it visible and frees slot s % NST; the MFMAs of
 // stage s run with the fragment reads of stage s + 1 and the copies of stage
-// s + NST spread between them, one every MPO MFMAs (the rate at which the LDS
-// serves the four waves).  Sources are uniform 64-bit bases plus one per-lane
+// s + NST spread between them, one every MPO MFMAs.  Sources are uniform 64-bit bases plus one per-lane
 // offset; stages past K re-read the last k-block (branch-free, so the wait
 // counts are exact), and nothing reads what they bring in.
 //
@@ -398,25 +398,32 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_lds_kernel(GemmI8Args a)
 // lane's accumulators 4T .. 4T + 3 and fold without any exchange of lanes
 // (planes_epilogue's 12 cross-lane moves per accumulator were a third of the
 // 64 x 128 kernel's time at K = 2048).
-// The accumulators are pinned to the accumulation registers: left to itself the
-// register allocator moves them (and fragments) between the two register files
-// in the loop, up to 190 moves per 64 MFMAs.
-__device__ __forceinline__ void mfma_i8_acc(v4i& c, uint4 x, uint4 y) {
-  asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(c) : "v"(__builtin_bit_cast(v4i, x)), "v"(__builtin_bit_cast(v4i, y)));
+// ACC (8 row groups a wave, 512 registers): the accumulators are pinned to the
+// accumulation registers, as the register allocator left to itself moves them
+// (and fragments) between the two register files in the loop, up to 190 moves
+// per 64 MFMAs.  The fragments come from LDS reads alone, whose waits the
+// compiler sees.  Otherwise everything fits 256 registers and stays in place.
+template <bool ACC>
+__device__ __forceinline__ void mfma_i8(v4i& c, uint4 x, uint4 y) {
+  if constexpr (ACC)
+    asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(c) : "v"(__builtin_bit_cast(v4i, x)), "v"(__builtin_bit_cast(v4i, y)));
+  else
+    c = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, x), __builtin_bit_cast(v4i, y), c, 0, 0, 0);
 }
-// The wait states between the last MFMA's write and the first read of an
+// The wait states between the last asm MFMA's write and the first read of an
 // accumulator, which the compiler inserts only behind MFMAs that it issued
 // (at most 18 for the 4-pass i8 MFMA and a vector ALU read).
 __device__ __forceinline__ void mfma_i8_settle() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 
 enum { QUAD_F32, QUAD_PLANES, QUAD_I32 };   // outputs: scaled codes, folded planes, the sums
-template <int FM, int FN, int NST, int MODE>
-__global__ __launch_bounds__(256, FM * FN <= 24 ? 2 : 1) void gemm_i8_quad_kernel(GemmI8Args a) {
-  constexpr int MT = 2 * FM, NT = 2 * FN, TS = MT + NT;   // row groups, column groups, tiles per stage
-  constexpr int PA = MT / 4, PW = TS / 4;                 // copies per wave per stage (PA of them activations)
+template <int WM, int FM, int FN, int NST, int MODE>
+__global__ __launch_bounds__(128 * WM, FM == 8 ? 1 : 2) void gemm_i8_quad_kernel(GemmI8Args a) {
+  constexpr int NW = 2 * WM;                              // waves: WM x 2
+  constexpr int MT = WM * FM, NT = 2 * FN, TS = MT + NT;  // row groups, column groups, tiles per stage
+  constexpr int PA = MT / NW, PW = (TS + NW - 1) / NW;    // copies per wave per stage (PA of them activations)
   constexpr int NMEM = FM + FN + PW;                      // memory operations per wave per stage
   constexpr int MPO = FM * FN >= 2 * NMEM ? 2 : 1;        // MFMAs per memory operation
-  static_assert(MT % 4 == 0 && NT % 4 == 0, "copies must divide over the waves");
+  static_assert(MT % NW == 0, "activation copies must divide over the waves");
   static_assert(MODE != QUAD_PLANES || FM % 4 == 0, "a wave holds whole plane groups");
   static_assert(NST >= 3 && NST * TS <= 160 && PW * (NST - 1) < 64, "LDS size, vmcnt range");
   constexpr uint32_t SB = TS * 1024;                      // bytes per stage
@@ -430,23 +437,31 @@ __global__ __launch_bounds__(256, FM * FN <= 24 ? 2 : 1) void gemm_i8_quad_kerne
   const int ks = SLICES ? blockIdx.x / (a.ntm * a.ntn) : 0;
   const int bt = blockIdx.x - ks * a.ntm * a.ntn;
   int tm, tn;
-  tile_patch(bt, a.ntm, a.ntn, FM == 8 ? 4 : 8, tm, tn);
+  tile_patch(bt, a.ntm, a.ntn, MT == 16 ? 4 : 8, tm, tn);
   const int mg0 = tm * MT, ng0 = tn * NT;
   const int kb0 = SLICES ? (ks * a.KB) / a.S : 0;         // this work-group's k-blocks [kb0, kb0 + KB)
   const int KB = SLICES ? ((ks + 1) * a.KB) / a.S - kb0 : a.KB;
   const size_t astep = (size_t)a.MG * 1024, bstep = (size_t)a.NG * 1024;
 
-  // copy p of a stage: tile wv + 4 p of its A then B tiles; rows / columns
-  // past the matrix edge re-read a valid tile (never stored)
+  // copy p of a stage: tile wv + NW p of its A then B tiles (where NW does not
+  // divide them the last waves have one copy less); rows / columns past the
+  // matrix edge re-read a valid tile (never stored)
   const uint8_t* src[PW];
 #pragma unroll
   for (int p = 0; p < PW; p++)
-    src[p] = p < PA ? a.At + kb0 * astep + (size_t)min(mg0 + wv + 4 * p, a.MG - 1) * 1024
-                    : a.Bt + kb0 * bstep + (size_t)min(ng0 + wv + 4 * (p - PA), a.NG - 1) * 1024;
+    src[p] = p < PA ? a.At + kb0 * astep + (size_t)min(mg0 + wv + NW * p, a.MG - 1) * 1024
+                    : a.Bt + kb0 * bstep + (size_t)min(ng0 + wv + NW * (p - PA), a.NG - 1) * 1024;
+  constexpr bool EVEN = TS % NW == 0;
+  const bool last = EVEN || wv < TS % NW;                 // this wave has copy PW - 1
   const uint32_t lane16 = lane * 16;
   const uint32_t sbase = lds_addr(sS);
   auto copy = [&](size_t oa, size_t ob, uint32_t slot, int p) {
-    dma_tile_s(lane16, src[p] + (p < PA ? oa : ob), sbase + slot + (uint32_t)(wv + 4 * p) * 1024u);
+    if (EVEN || p < PW - 1 || last)
+      dma_tile_s(lane16, src[p] + (p < PA ? oa : ob), sbase + slot + (uint32_t)(wv + NW * p) * 1024u);
+  };
+  auto wait_stages = [&](auto n) {                        // all but the latest n stages' copies landed
+    if (EVEN || last) wait_vm<PW * n()>();
+    else wait_vm<(PW - 1) * n()>();
   };
 
   v4i acc[FM][FN];
@@ -466,7 +481,7 @@ __global__ __launch_bounds__(256, FM * FN <= 24 ? 2 : 1) void gemm_i8_quad_kerne
 #pragma unroll
     for (int p = 0; p < PW; p++) copy(sc * astep, sc * bstep, b * SB, p);
   }
-  wait_vm<PW * (NST - 1)>();
+  wait_stages([]() constexpr { return NST - 1; });
   stage_barrier();
 #pragma unroll
   for (int i = 0; i < FM; i++) fa[0][i] = ra[i * 64];
@@ -475,7 +490,7 @@ __global__ __launch_bounds__(256, FM * FN <= 24 ? 2 : 1) void gemm_i8_quad_kerne
 
   uint32_t slot = 0;                                      // slot of stage s (bytes)
   auto step = [&](int st, int c) {
-    wait_vm<PW * (NST - 2)>();                            // stage s + 1 landed (this wave's part)
+    wait_stages([]() constexpr { return NST - 2; });      // stage s + 1 landed (this wave's part)
     wait_lgkm0();                                         // this wave's reads of stage s are done
     stage_barrier();                                      // stage s + 1 visible; slot of stage s free
     const uint32_t nxt = slot + SB == NST * SB ? 0u : slot + SB;
@@ -491,7 +506,7 @@ __global__ __launch_bounds__(256, FM * FN <= 24 ? 2 : 1) void gemm_i8_quad_kerne
 #pragma unroll
     for (int m = 0; m < FM * FN; m++) {
       const int i = m / FN, j = m % FN;
-      mfma_i8_acc(acc[i][j], fb[c][j], fa[c][i]);
+      mfma_i8<FM == 8>(acc[i][j], fb[c][j], fa[c][i]);
       __builtin_amdgcn_sched_barrier(0);
       if (m % MPO == 0 && m / MPO < NMEM) mem_op(m / MPO);
       __builtin_amdgcn_sched_barrier(0);
@@ -509,7 +524,7 @@ __global__ __launch_bounds__(256, FM * FN <= 24 ? 2 : 1) void gemm_i8_quad_kerne
   }
   if (st < KB) step(st, 0);
   wait_vm<0>();   // no copy may still be landing in LDS when the work-group exits
-  mfma_i8_settle();
+  if constexpr (FM == 8) mfma_i8_settle();
   if constexpr (SLICES) {
     if (a.S > 1 && !merge_slices<FM, FN>(a, acc, wv, lane, bt, ks, reinterpret_cast<int*>(sS))) return;
   }
@@ -686,7 +701,7 @@ static void gemm_i8_plan(const GemmLaunch& L, int& cfg, int& split) {
     return n * (fixed + KB * pair) + (rem == 0 ? 0.0f : fixed + KB * (rem <= 256 ? alone : pair));
   };
   if (planes) {
-    offer(3, cdiv(tiles(3), 256) * (11.0f + 0.59f * KB), 1);
+    offer(3, cdiv(tiles(3), 256) * (6.5f + 0.605f * KB), 1);
     offer(4, cdiv(tiles(4), 256) * (8.0f + 0.50f * KB), 1);
     offer(6, paired(tiles(6), 3.9f, 0.265f, 0.435f), planes_slices(tiles(6), KB));
   } else {
@@ -718,19 +733,18 @@ void gemm_i8_needs(const GemmLaunch& L, size_t* part_bytes, size_t* counters) {
 
 // planes on 256 x 256, 256 x 192 and 128 x 128 tiles, codes on 128 x 192 and
 // 128 x 128 (i8_resolve)
-template <int FM, int FN, int NST>
+template <int WM, int FM, int FN, int NST>
 static void launch_quad(const GemmI8Args& a, int blocks, hipStream_t st) {
-  if constexpr (FM * FN != 24) {
+  const dim3 grid(blocks), block(128 * WM);
+  if constexpr (FM == 8 || FN != 6) {
     if (a.out == OUT_F32_X4) {
-      hipLaunchKernelGGL((gemm_i8_quad_kernel<FM, FN, NST, QUAD_PLANES>), dim3(blocks), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((gemm_i8_quad_kernel<WM, FM, FN, NST, QUAD_PLANES>), grid, block, 0, st, a);
       return;
     }
   }
-  if constexpr (FM * FN <= 24) {
-    if (a.out == OUT_I32)
-      hipLaunchKernelGGL((gemm_i8_quad_kernel<FM, FN, NST, QUAD_I32>), dim3(blocks), dim3(256), 0, st, a);
-    else
-      hipLaunchKernelGGL((gemm_i8_quad_kernel<FM, FN, NST, QUAD_F32>), dim3(blocks), dim3(256), 0, st, a);
+  if constexpr (WM == 2 && FM == 4) {
+    if (a.out == OUT_I32) hipLaunchKernelGGL((gemm_i8_quad_kernel<WM, FM, FN, NST, QUAD_I32>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((gemm_i8_quad_kernel<WM, FM, FN, NST, QUAD_F32>), grid, block, 0, st, a);
   }
 }
 
@@ -782,10 +796,10 @@ hipError_t launch_gemm_i8(const GemmLaunch& L, hipStream_t st) {
     case 0: hipLaunchKernelGGL((gemm_i8_lds_kernel<8, 12, 1, 4, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;
     case 1: hipLaunchKernelGGL((gemm_i8_lds_kernel<4, 8, 1, 8, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;
     case 2: hipLaunchKernelGGL((gemm_i8_lds_kernel<8, 8, 1, 8, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;
-    case 3: launch_quad<8, 8, 4>(a, blocks, st); break;
-    case 4: launch_quad<8, 6, 5>(a, blocks, st); break;
-    case 5: launch_quad<4, 6, 4>(a, blocks, st); break;
-    default: launch_quad<4, 4, 5>(a, blocks, st); break;
+    case 3: launch_quad<4, 4, 8, 5>(a, blocks, st); break;
+    case 4: launch_quad<2, 8, 6, 5>(a, blocks, st); break;
+    case 5: launch_quad<2, 4, 6, 4>(a, blocks, st); break;
+    default: launch_quad<2, 4, 4, 5>(a, blocks, st); break;
   }
   return hipGetLastError();
 }
