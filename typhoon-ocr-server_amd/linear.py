@@ -216,9 +216,14 @@ def _ptr(t) -> Optional[int]:
 
 
 def _stream(stream) -> Optional[int]:
+    """Handle of a stream, or of torch's current one.
+
+    The current stream's raw handle is asked for directly: building the Stream
+    object of torch.cuda.current_stream() takes 2.9 us a call, more than the
+    launch of a decode GEMV (7.0 -> 4.4 us per w8a32_linear_dev call)."""
     if stream is None:
         import torch
-        stream = torch.cuda.current_stream()
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     return stream.cuda_stream
 
 
