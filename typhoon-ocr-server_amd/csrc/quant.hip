@@ -76,6 +76,51 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const float* __restr
   }
 }
 
+// The same for rows of float4s (cols a multiple of 4, up to 1024 NV, src 16-byte
+// and dst 4-byte aligned): the row's loads are all in flight at once and stay in
+// registers, where the loops above wait for one load per round, twice over (200 x
+// 6144 6.6 -> 4.2 us).
+template <int NV>
+__global__ __launch_bounds__(256) void quantize_rows_vec_kernel(const float* __restrict__ src,
+                                                                int8_t* __restrict__ dst,
+                                                                float* __restrict__ scales, int cols,
+                                                                int clamp127) {
+  __shared__ uint32_t s_mx[4];
+  __shared__ float s_tail[4];
+  const int r = blockIdx.x;
+  const float4* r4 = reinterpret_cast<const float4*>(src + (size_t)r * cols);
+  uint32_t* o4 = reinterpret_cast<uint32_t*>(dst + (size_t)r * cols);
+  const int main_end = cols & ~15, n4 = cols >> 2;
+  float4 v[NV];
+#pragma unroll
+  for (int j = 0; j < NV; j++) v[j] = r4[min((int)threadIdx.x + 256 * j, n4 - 1)];   // repeats change no maximum
+  uint32_t mx = 0;
+  float tail = 0.0f;
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    if (4 * min((int)threadIdx.x + 256 * j, n4 - 1) < main_end) {
+      const uint32_t a = max(max(abs_bits(v[j].x), abs_bits(v[j].y)), max(abs_bits(v[j].z), abs_bits(v[j].w)));
+      mx = a > mx ? a : mx;
+    } else {
+      const float t[4] = {fabsf(v[j].x), fabsf(v[j].y), fabsf(v[j].z), fabsf(v[j].w)};
+#pragma unroll
+      for (int q = 0; q < 4; q++) tail = (t[q] > tail) ? t[q] : tail;
+    }
+  }
+  const float absmax = block_absmax_256(mx, tail, s_mx, s_tail);
+  const float scale = quant_scale(absmax);
+  const float inv = quant_inv(scale);
+  if (threadIdx.x == 0) scales[r] = scale;
+  const bool c127 = clamp127 != 0;
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    const int i = threadIdx.x + 256 * j, k = i << 2;
+    if (i < n4)
+      o4[i] = pack4(code_at(v[j].x, inv, k, cols, c127), code_at(v[j].y, inv, k + 1, cols, c127),
+                    code_at(v[j].z, inv, k + 2, cols, c127), code_at(v[j].w, inv, k + 3, cols, c127));
+  }
+}
+
 // One wave per row, 4 rows per work-group; codes are written straight into
 // the 16x64 tile layout (row r -> tile lanes (r & 15) + 16 lg), zero beyond K.
 // Lane l owns the 16-wide chunks c = l + 64 j of the row (64 contiguous bytes
@@ -289,16 +334,16 @@ hipError_t launch_split_i8x4(const float* X, int ldx, int M, int K, uint8_t* til
 // for the row groups of rows [0, rows) of w, written as row groups g0 .. of a
 // tile array with NGt row groups per k-block (g0 = 0, NGt = NG for a whole
 // matrix; a row chunk starting at row 16 g0 of a larger one otherwise)
+// (a work-group packs 4 row groups of one k-block, so that the split of its index
+// is one 32-bit division; per thread and in 64 bits it was most of the kernel:
+// 200 x 6144 3.7 -> 3.2 us)
 __global__ __launch_bounds__(256) void pack_tiles_kernel(const int8_t* __restrict__ w, int rows,
-                                                         int cols, int KB, long long total, int NGt,
+                                                         int cols, int nq, int NGt,
                                                          int g0, uint8_t* __restrict__ tiles) {
-  const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (t >= total) return;
-  const int lane = (int)(t & 63);
-  const long long tile = t >> 6;               // k-block-major: tile = kb * NG + g
-  const int NG = (rows + 15) / 16;
-  const int g = (int)(tile % NG);
-  const int kb = (int)(tile / NG);
+  const int lane = (int)(threadIdx.x & 63);
+  const int kb = (int)blockIdx.x / nq;         // nq: quads of row groups
+  const int g = 4 * ((int)blockIdx.x - kb * nq) + (int)(threadIdx.x >> 6);
+  if (g >= (rows + 15) / 16) return;
   const int r = g * 16 + (lane & 15);
   const int k0 = kb * 64 + (lane >> 4) * 16;
   uint4 q = make_uint4(0, 0, 0, 0);
@@ -397,8 +442,19 @@ hipError_t launch_copy_words(const void* src, void* dst, size_t bytes, hipStream
 hipError_t launch_quantize_rows(const float* src, int8_t* dst, float* scales, int rows, int cols,
                                 bool clamp127, hipStream_t st) {
   if (rows <= 0 || cols <= 0) return hipSuccess;
-  hipLaunchKernelGGL(quantize_rows_kernel, dim3(rows), dim3(256), 0, st, src, dst, scales, cols,
-                     clamp127 ? 1 : 0);
+  const int c = clamp127 ? 1 : 0;
+  const dim3 grid(rows), block(256);
+  const bool vec = (cols & 3) == 0 && (((uintptr_t)src) & 15) == 0 && (((uintptr_t)dst) & 3) == 0;
+  if (vec && cols <= 2048)
+    hipLaunchKernelGGL(quantize_rows_vec_kernel<2>, grid, block, 0, st, src, dst, scales, cols, c);
+  else if (vec && cols <= 4096)
+    hipLaunchKernelGGL(quantize_rows_vec_kernel<4>, grid, block, 0, st, src, dst, scales, cols, c);
+  else if (vec && cols <= 6144)
+    hipLaunchKernelGGL(quantize_rows_vec_kernel<6>, grid, block, 0, st, src, dst, scales, cols, c);
+  else if (vec && cols <= 8192)
+    hipLaunchKernelGGL(quantize_rows_vec_kernel<8>, grid, block, 0, st, src, dst, scales, cols, c);
+  else
+    hipLaunchKernelGGL(quantize_rows_kernel, grid, block, 0, st, src, dst, scales, cols, c);
   return hipGetLastError();
 }
 
@@ -429,10 +485,10 @@ hipError_t launch_pack_tiles_rows(const int8_t* w, int rows, int cols, int NGt, 
   if (rows <= 0 || cols <= 0) return hipSuccess;
   if (g0 < 0 || g0 + cdiv(rows, 16) > NGt) return hipErrorInvalidValue;
   const int KB = cdiv(cols, 64);
-  const long long total = (long long)cdiv(rows, 16) * KB * 64;
-  const long long blocks = (total + 255) / 256;
-  hipLaunchKernelGGL(pack_tiles_kernel, dim3((unsigned)blocks), dim3(256), 0, st, w, rows, cols, KB,
-                     total, NGt, g0, tiles);
+  const int nq = cdiv(rows, 64);
+  if ((long long)nq * KB > 0x7fffffffLL) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(pack_tiles_kernel, dim3((unsigned)nq * (unsigned)KB), dim3(256), 0, st, w, rows, cols, nq, NGt, g0,
+                     tiles);
   return hipGetLastError();
 }
 
