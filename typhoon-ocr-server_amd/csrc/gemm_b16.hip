@@ -21,7 +21,7 @@
 #include <algorithm>
 #include <atomic>
 
-#include "tl_common.h"
+#include "gemm_common.h"
 #include "tl_kernels.h"
 
 typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));

@@ -26,7 +26,7 @@
 #include <algorithm>
 #include <atomic>
 
-#include "tl_common.h"
+#include "gemm_common.h"
 #include "tl_kernels.h"
 
 namespace tl {

@@ -15,7 +15,7 @@
 // cache is [kv head][max_seq][128] per layer.
 #include <algorithm>
 
-#include "tl_common.h"
+#include "gemm_common.h"
 #include "tl_kernels.h"
 
 namespace tl {

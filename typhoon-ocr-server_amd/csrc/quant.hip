@@ -19,7 +19,7 @@
 // operand.
 //
 // pack_tiles_kernel re-lays a row-major int8 matrix into 16x64 tiles.
-#include "tl_common.h"
+#include "gemm_common.h"
 #include "tl_kernels.h"
 
 namespace tl {

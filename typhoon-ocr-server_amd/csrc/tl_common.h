@@ -318,15 +318,6 @@ __device__ __forceinline__ void planes4_i8(const float (&v)[4], int e, uint32_t 
     code[3] |= bp[2] << (8 * q);
   }
 }
-// Code row of plane p of token t: 4t + p, or grouped, where row group 4T + p
-// holds plane p of tokens 16T .. 16T + 15 (the layout of the quadrant GEMM);
-// and the code row groups of `rows` tokens.
-__host__ __device__ __forceinline__ int planes_row(int t, int p, bool grouped) {
-  return grouped ? 64 * (t >> 4) + 16 * p + (t & 15) : 4 * t + p;
-}
-__host__ __device__ __forceinline__ int planes_groups(int rows, bool grouped) {
-  return grouped ? 4 * cdiv(rows, 16) : cdiv(4 * rows, 16);
-}
 // the row exponent of the planes: frexp exponent of the absmax - 6 (0 for a
 // zero row), or kXeNonFinite when the row holds Inf or NaN
 __device__ __forceinline__ int planes_exponent(uint32_t absmax_bits) {
@@ -430,10 +421,6 @@ __device__ inline uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 // fp32 -> bf16 bits, round to nearest even
-// (rounds to nearest even, unlike v_cvt_pkrtz)
-__device__ inline uint32_t pack_f16x2(float a, float b) {
-  return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)a) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)b) << 16);
-}
 __device__ inline uint32_t f32_to_bf16_rne(float f) { return pack_bf16x2(f, 0.0f) & 0xffffu; }
 __device__ inline float bf16_to_f32(uint32_t h) { return __uint_as_float(h << 16); }
 
@@ -610,22 +597,6 @@ __device__ __forceinline__ void dma_tile_s(uint32_t voff, const void* sbase, uin
                : "memory");
 }
 __device__ __forceinline__ void stage_barrier() { asm volatile("s_barrier" ::: "memory"); }
-
-// Tile order of the quadrant GEMMs, for any tile counts (work-group b runs on
-// XCD b % 8): XCD x owns an eighth of the
-// tiles, consecutive in an order that walks bands of gm tile rows column by
-// column, so that the tiles an XCD runs at once are a patch of gm rows and its
-// L2 fills gm row panels and as many columns (against the int8 LDS-staged kernel's order over a sweep of
-// 130 shapes: 6 % faster where the columns divide over the XCDs and tiles
-// number more than 128, 10 % where they do not, equal below).
-__device__ __forceinline__ void tile_patch(int b, int ntm, int ntn, int gm, int& tm, int& tn) {
-  const int n = ntm * ntn, x = b % 8;
-  const int u = x * (n / 8) + min(x, n % 8) + b / 8;      // a bijection of [0, n)
-  const int grp = u / (gm * ntn), r = u - grp * gm * ntn;
-  const int rows = min(gm, ntm - gm * grp);
-  tm = gm * grp + r % rows;
-  tn = r / rows;
-}
 
 // Work-group b -> token row for kernels that write one token's int8 codes
 // per work-group into the 16x64 tile layout.  A 128-byte line of a tile holds
