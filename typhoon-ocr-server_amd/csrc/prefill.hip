@@ -295,10 +295,13 @@ constexpr int FT = 64;          // queries / keys per tile
 // lane & 15).  The fp32 MFMA (32 cycles) does not run beside vector
 // instructions (8 cycles each for one wave), so a key tile costs 256 MFMAs plus
 // its vector instructions, whatever the number of waves (two waves per SIMD over
-// halves of the keys measured the same).  Hence the softmax in powers of two (one
-// fma, one bound and one v_exp_f32 per score), masks only where a tile needs them
-// and rare rescaling: 1200 tokens 94.7 -> 79 us, 2048 tokens 211 -> 182 us (error
-// against float64 3.70e-7 -> 3.69e-7 and 4.56e-7 -> 4.54e-7).
+// halves of the keys measured the same).  Hence masks only where a tile needs
+// them, rescaling only where a maximum grew, and two chains of score MFMAs: 777 /
+// 1200 / 2048 tokens 49.7 / 94.2 / 202 -> 46.3 / 87.5 / 198 us, the same bits.
+// (A softmax in powers of two with rescaling past 2^8 alone took 42.2 / 79.2 /
+// 177 us, as close to float64, but the changed roundings grow over the layers
+// after it, to a relative 2.5e-3 over 28 layers and 1.6e-2 over two with int8
+// activations.)
 //   scores   D[key][query] += K[key][d] Q[query][d]: K is the first operand,
 //            Q (kept in registers) the second; MFMA t = 4u + e of a 16-key
 //            block reads, in lane group g, dimension d = 16u + 4g + e (any
@@ -372,7 +375,7 @@ struct FlashOrder {
   __host__ __device__ int at(int k) const { return (w[k >> 2] >> (8 * (k & 3))) & 0xff; }
 };
 
-__global__ __launch_bounds__(256, 2) void flash_prefill_mfma_kernel(const float* __restrict__ qkv,
+__global__ __launch_bounds__(256) void flash_prefill_mfma_kernel(const float* __restrict__ qkv,
                                                                  const float* __restrict__ kc,
                                                                  const float* __restrict__ vc, float* __restrict__ out,
                                                                  int S, int max_seq, int key0, int qoff, float scale,
@@ -410,11 +413,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_mfma_kernel(const float*
   v4f o[8];
 #pragma unroll
   for (int j = 0; j < 8; j++) o[j] = v4f{0.f, 0.f, 0.f, 0.f};
-  // softmax in powers of two: m is the running max of score x cs (never above
-  // the true one by more than a rounding, below it by at most kSlack)
-  constexpr float kSlack = 8.0f;
-  const float cs = scale * 1.44269504f;                   // log2(e)
-  float m = -1.0e30f, l = 0.0f;
+  float m = -3.0e38f, l = 0.0f;                           // running max and sum of query c
 
   const int nkt = (qoff + q0 + nq - 1) / FT + 1;
   const int kmid = (nkt + 1) / 2;
@@ -489,8 +488,12 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_mfma_kernel(const float*
     };
     vread(0, vf[0]);
     __builtin_amdgcn_sched_barrier(0);
-    // mask (tiles that reach past the work-group's first query), online softmax
-    // (query c: lanes c, c+16, c+32, c+48)
+    // scale, mask (tiles that reach past the work-group's first query), online
+    // softmax (query c: lanes c, c+16, c+32, c+48)
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) sc[b][r] = __fmul_rn(sc[b][r], scale);
     if (kt * FT + FT - 1 > min(qoff + q0, Sk - 1)) {
       const int klim = min(qpos, Sk - 1) - (kt * FT + g);   // keys of this lane: 16 b + 4 r up to it
 #pragma unroll
@@ -505,32 +508,31 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_mfma_kernel(const float*
       for (int r = 0; r < 4; r++) mx = fmaxf(mx, sc[b][r]);
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    mx = __fmul_rn(mx, cs);
-    // the sums are rescaled only where a max grew by more than kSlack: weights
-    // reach 2^kSlack, which costs fp32 sums nothing
-    if (__any(mx > m + kSlack)) {
+    // the sums are rescaled where a max of the wave grew; elsewhere every factor
+    // is exp(0) = 1, which changes no bit
+    float resc = 1.0f;
+    if (__any(mx > m)) {
       const float m_new = fmaxf(m, mx);
-      const float resc = __builtin_amdgcn_exp2f(__fsub_rn(m, m_new));
+      resc = expf(__fsub_rn(m, m_new));
       m = m_new;
-      l = __fmul_rn(l, resc);
 #pragma unroll
       for (int j = 0; j < 8; j++)
 #pragma unroll
         for (int r = 0; r < 4; r++) o[j][r] = __fmul_rn(o[j][r], resc);
     }
-    // weights 2^(score cs - m), one rounding before the exponential; the lower
-    // bound makes a NaN score's weight 0, and 2^-1000 is 0
+    // (a NaN score, like a masked one, weighs 0)
     float ps = 0.0f;
 #pragma unroll
     for (int b = 0; b < 4; b++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        sc[b][r] = __builtin_amdgcn_exp2f(fmaxf(__fmaf_rn(sc[b][r], cs, -m), -1000.0f));
-        ps = __fadd_rn(ps, sc[b][r]);
+        const float pv = sc[b][r] > -1.0e38f ? expf(__fsub_rn(sc[b][r], m)) : 0.0f;
+        sc[b][r] = pv;
+        ps = __fadd_rn(ps, pv);
       }
     ps = __fadd_rn(ps, __shfl_xor(ps, 16, 64));
     ps = __fadd_rn(ps, __shfl_xor(ps, 32, 64));
-    l = __fadd_rn(l, ps);
+    l = __fmaf_rn(l, resc, ps);
     // O^T[d][query] += V^T[d][key] P^T[key][query], keys 4 km + g, km = 4b + mm
 #pragma unroll
     for (int km = 0; km < 16; km++) {
@@ -576,7 +578,7 @@ __global__ __launch_bounds__(256, 2) void flash_prefill_mfma_kernel(const float*
     const float m0 = half == 0 ? m : mo, m1 = half == 0 ? mo : m;
     const float l0 = half == 0 ? l : lo, l1 = half == 0 ? lo : l;
     const float M = fmaxf(m0, m1);
-    const float a0 = __builtin_amdgcn_exp2f(__fsub_rn(m0, M)), a1 = __builtin_amdgcn_exp2f(__fsub_rn(m1, M));
+    const float a0 = expf(__fsub_rn(m0, M)), a1 = expf(__fsub_rn(m1, M));
     l = __fadd_rn(__fmul_rn(l0, a0), __fmul_rn(l1, a1));
 #pragma unroll
     for (int j = 0; j < 8; j++)
