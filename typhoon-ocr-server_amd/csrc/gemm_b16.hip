@@ -629,9 +629,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_b16_wave_kernel(GemmB16A
   // consecutive columns (stored straight from the accumulators a store covers 16
   // or 32 bytes of each of 32 rows).
   constexpr int COLS = 32 * CN;
-  constexpr int LDB = 4 * COLS + 16;                      // bytes per LDS row (fp32; 16-bit rows use half)
-  static_assert(NW * 32 * LDB <= NST * TS * 1024, "rows of a pass fit the ring");
-  uint8_t* const lw = reinterpret_cast<uint8_t*>(sS) + wv * (32 * LDB);
+  constexpr int LD4 = 4 * COLS + 16, LD2 = 2 * COLS + 16;  // bytes per LDS row of fp32 and of 16-bit outputs
+  static_assert(LD4 % 16 == 0 && LD2 % 16 == 0, "rows are read in aligned 16-byte pieces");
+  static_assert(NW * 32 * LD4 <= NST * TS * 1024, "rows of a pass fit the ring");
+  uint8_t* const lw = reinterpret_cast<uint8_t*>(sS) + wv * (32 * LD4);
   const int n0 = (ng0 + wn * 2 * CN) * 16;
   const int lrow = lane & 31, lcol = 4 * (lane >> 5);
   const bool wide = a.out == OUT_F32;
@@ -660,7 +661,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_b16_wave_kernel(GemmB16A
         for (int r = 0; r < 4; r++) y[r] = __fadd_rn(y[r], b[q][r]);
       }
       if (wide) {
-        *reinterpret_cast<v4f*>(lw + lrow * LDB + (8 * q + lcol) * 4) = y;
+        *reinterpret_cast<v4f*>(lw + lrow * LD4 + (8 * q + lcol) * 4) = y;
       } else {
         uint2 h;
         if (a.out == OUT_BF16) {
@@ -668,7 +669,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_b16_wave_kernel(GemmB16A
         } else {
           h = make_uint2(pack_f16x2(y[0], y[1]), pack_f16x2(y[2], y[3]));
         }
-        *reinterpret_cast<uint2*>(lw + lrow * (LDB / 2) + (8 * q + lcol) * 2) = h;
+        *reinterpret_cast<uint2*>(lw + lrow * LD2 + (8 * q + lcol) * 2) = h;
       }
     }
     auto rows_out = [&](auto width) {
@@ -676,7 +677,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_b16_wave_kernel(GemmB16A
 #pragma unroll 4
       for (int t = 0; t < 32 * CPR / 64; t++) {
         const int c = t * 64 + lane, r = c / CPR, col = (c - r * CPR) * PC;
-        const v4i v = *reinterpret_cast<const v4i*>(lw + r * (LDB * E / 4) + col * E);
+        const v4i v = *reinterpret_cast<const v4i*>(lw + r * (E == 4 ? LD4 : LD2) + col * E);
         uint8_t* yp = static_cast<uint8_t*>(a.Y) + ((size_t)(m0 + r) * a.ldy + n0 + col) * E;
         if (m0 + r >= a.M) continue;
         if (vec && col + PC <= room) {
