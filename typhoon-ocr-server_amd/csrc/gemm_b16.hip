@@ -672,6 +672,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_b16_wave_kernel(GemmB16A
         *reinterpret_cast<uint2*>(lw + lrow * LD2 + (8 * q + lcol) * 2) = h;
       }
     }
+    wave_lds_fence();                                     // lanes read what other lanes wrote
     auto rows_out = [&](auto width) {
       constexpr int E = width(), PC = 16 / E, CPR = COLS / PC;   // bytes per output, outputs per piece, pieces per row
 #pragma unroll 4
@@ -695,6 +696,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_b16_wave_kernel(GemmB16A
     };
     if (wide) rows_out([]() constexpr { return 4; });
     else rows_out([]() constexpr { return 2; });
+    wave_lds_fence();                                     // the next rows overwrite these
   }
 }
 

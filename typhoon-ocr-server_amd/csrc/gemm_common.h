@@ -20,6 +20,15 @@ __device__ inline uint32_t pack_f16x2(float a, float b) {
   return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)a) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)b) << 16);
 }
 
+// Orders a wave's LDS accesses across it: what its lanes wrote before is what
+// other lanes of the same wave read after, and no later write moves above an
+// earlier read.  (LDS works a wave's accesses off in order, so nothing waits.)
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Tile order of the tiled GEMMs, for any tile counts (work-group b runs on XCD
 // b % 8): XCD x owns an eighth of the tiles, consecutive in an order that walks
 // bands of gm tile rows column by column, so that the tiles an XCD runs at once
