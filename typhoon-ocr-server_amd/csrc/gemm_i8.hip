@@ -398,23 +398,11 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_lds_kernel(GemmI8Args a)
 // lane's accumulators 4T .. 4T + 3 and fold without any exchange of lanes
 // (planes_epilogue's 12 cross-lane moves per accumulator were a third of the
 // 64 x 128 kernel's time at K = 2048).
-// ACC (8 row groups a wave, 512 registers): the accumulators are pinned to the
-// accumulation registers, as the register allocator left to itself moves them
-// (and fragments) between the two register files in the loop, up to 190 moves
-// per 64 MFMAs.  The fragments come from LDS reads alone, whose waits the
-// compiler sees.  Otherwise everything fits 256 registers and stays in place.
-template <bool ACC>
-__device__ __forceinline__ void mfma_i8(v4i& c, uint4 x, uint4 y) {
-  if constexpr (ACC)
-    asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(c) : "v"(__builtin_bit_cast(v4i, x)), "v"(__builtin_bit_cast(v4i, y)));
-  else
-    c = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, x), __builtin_bit_cast(v4i, y), c, 0, 0, 0);
-}
-// The wait states between the last asm MFMA's write and the first read of an
-// accumulator, which the compiler inserts only behind MFMAs that it issued
-// (at most 18 for the 4-pass i8 MFMA and a vector ALU read).
-__device__ __forceinline__ void mfma_i8_settle() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
-
+// Accumulators and fragments are left to the register allocator.  Tiles of 8 row
+// groups a wave (512 registers) need MFMAs with accumulators in the vector
+// registers (a compiler option of this file, see the Makefile): it then keeps
+// the fragments, which LDS reads can write there, in the accumulation registers,
+// about ten moves per 96 MFMAs, where with accumulators in those it made 320.
 enum { QUAD_F32, QUAD_PLANES, QUAD_I32 };   // outputs: scaled codes, folded planes, the sums
 template <int WM, int FM, int FN, int NST, int MODE>
 __global__ __launch_bounds__(128 * WM, FM == 8 ? 1 : 2) void gemm_i8_quad_kernel(GemmI8Args a) {
@@ -506,7 +494,8 @@ __global__ __launch_bounds__(128 * WM, FM == 8 ? 1 : 2) void gemm_i8_quad_kernel
 #pragma unroll
     for (int m = 0; m < FM * FN; m++) {
       const int i = m / FN, j = m % FN;
-      mfma_i8<FM == 8>(acc[i][j], fb[c][j], fa[c][i]);
+      acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, fb[c][j]),
+                                                        __builtin_bit_cast(v4i, fa[c][i]), acc[i][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       if (m % MPO == 0 && m / MPO < NMEM) mem_op(m / MPO);
       __builtin_amdgcn_sched_barrier(0);
@@ -524,7 +513,6 @@ __global__ __launch_bounds__(128 * WM, FM == 8 ? 1 : 2) void gemm_i8_quad_kernel
   }
   if (st < KB) step(st, 0);
   wait_vm<0>();   // no copy may still be landing in LDS when the work-group exits
-  if constexpr (FM == 8) mfma_i8_settle();
   if constexpr (SLICES) {
     if (a.S > 1 && !merge_slices<FM, FN>(a, acc, wv, lane, bt, ks, reinterpret_cast<int*>(sS))) return;
   }
