@@ -400,14 +400,13 @@ static GemmKernel gemm_choice(const GemmLaunch& L) {
     if (fc == 3 && gemm_small_supported(L)) return GK_SMALL;
     if (((fc >= 0 && fc <= 2) || fc >= 4) && L.M > 16 && gemm_b16_supported(L)) return GK_B16;
   }
-  // 16-bit rows (the grid's y extent over the token groups), measured against
-  // the tiled kernel's best: 128 rows at N = 2048 / 4096, K = 2048 7.4 / 9.9 us
-  // against 12.2 / 13.9, 256 rows at N = 2048, K = 4096 14.6 against 16.7 (K = 6144
-  // 19.5 against 19.2; N = 4096, K = 4096 24.2 against 21.4), 64 rows at N = 8192,
-  // K = 3072 13.1 against 15.8, at N = 12288 15.6 against 13.8
+  // 16-bit rows past 16: the kernel of the smaller estimate (gemm_small.hip,
+  // gemm_b16.hip), both fitted with weights from HBM: 128 rows at N = 2048 / 4096,
+  // K = 2048 6.9 / 9.5 us against 12.2 / 13.6, 256 rows at N = 2048, K = 4096 /
+  // 6144 14.2 against 16.1 / 19.1 against 18.4, 64 rows at N = 8192, K = 3072 / N =
+  // 12288, K = 2048 13.1 against 15.7 / 15.6 against 14.4
   const int ng = cdiv(L.N, 16);
-  const bool b16_small = b16 && (L.M <= 32 || (L.M <= 64 && ng <= 512) || (L.M <= 128 && ng <= 256) ||
-                                 (L.M <= 256 && ng <= 128 && L.K <= 4096));
+  const bool b16_small = b16 && L.M <= 256 && gemm_small_b16_us(L.M, L.N, L.K) < gemm_b16_us(L.M, L.N, L.K);
   const bool wide_i8 = L.amode == A_I8 && L.M <= 32 && ng >= 2048;
   // int8 codes and fp32 rows: up to 64 rows at N <= 6144 and 32 rows at
   // N <= 12288 (W8A8 at K = 2048, N = 6144, 24..64 rows: 8.1-11.0 us against
@@ -431,6 +430,24 @@ bool gemm_planes_grouped(int M4, int N, int K) {
   L.N = N;
   L.K = K;
   return gemm_choice(L) == GK_I8;
+}
+
+// the kernel of a shape with contiguous, aligned rows (GemmKernel), and the tiled
+// kernels' configuration and K slices (0 and 1 for the others)
+int gemm_planned(int amode, int out, int M, int N, int K, int* cfg, int* split) {
+  static const uint8_t zeros[1] = {0};     // any address: nothing is read
+  GemmLaunch L;
+  L.amode = amode;
+  L.out = out;
+  L.M = M;
+  L.N = N;
+  L.K = L.lda = K;
+  L.zero_tile = zeros;
+  const GemmKernel k = gemm_choice(L);
+  *cfg = 0;
+  *split = 1;
+  if (k == GK_B16) gemm_b16_planned(L, cfg, split);
+  return k;
 }
 
 // split work-space of the kernel launch_gemm picks for L: partial-sum bytes
@@ -515,4 +532,7 @@ void tlk_gemm_needs(const GemmLaunch* L, size_t* part_bytes, size_t* counters) {
   tl::gemm_needs(*L, part_bytes, counters);
 }
 void tlk_gemm_b16_set_plan(int cfg, int split) { tl::gemm_b16_set_plan(cfg, split); }
+int tlk_gemm_planned(int amode, int out, int M, int N, int K, int* cfg, int* split) {
+  return tl::gemm_planned(amode, out, M, N, K, cfg, split);
+}
 }  // extern "C"

@@ -705,8 +705,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_b16_wave_kernel(GemmB16A
 // ---------------------------------------------------------------------------
 // cfg 0: LDS-staged kernel, 128 x 192 tiles
 // cfg 4..8: wave-grid kernel, 256 x 192 and 256 x 128 (8 waves), 128 x 128 (two
-//   work-groups per CU), 64 x 128 tiles with a 5-deep (two per CU) or 3-deep
-//   ring (three per CU)
+//   work-groups per CU), 64 x 128 tiles with a 4-deep (two per CU) or 3-deep
+//   ring (three per CU).  A 5-deep ring of those took as long as the 4-deep one
+//   with weights from HBM and up to 3 % longer with repeated ones
 static void b16_cfg(int cfg, int& mt, int& nt) {
   static const int dims[9][2] = {{8, 12}, {0, 0}, {0, 0}, {0, 0}, {16, 12}, {16, 8}, {8, 8}, {4, 8}, {4, 8}};
   mt = dims[cfg][0];
@@ -735,39 +736,55 @@ static int b16_tiles(int cfg, int MG, int NG) {
 }
 
 // Plan: the configuration and K slices of least estimated time, rounds of
-// work-groups times the time of one over KB k-blocks, the constants fitted to
-// measured launches (148 shapes: 40..2048 rows, N = 1024..12288, K = 1024..6144;
-// the choice is on average 0.8 % and at most 10 % slower than the best of its
-// shape).  K slices (the 4-wave configurations take them) cost a merge of three
-// dependent memory round trips, so they pay only where the tiles leave most CUs
-// idle: up to 96 tiles (333 x 2048 x 6144: 30.6 us unsplit, 23.3 with 4 slices of
-// 128 x 128; 1024 x 2048 x 6144, 128 tiles: 38.2 with 2, 34.1 unsplit).
+// work-groups times the time of one over KB k-blocks.  The constants are fitted
+// to launches whose weights come from HBM (more copies of them than the caches
+// hold, as in a model of many layers) and, at lower weight, to repeated ones, of
+// every configuration and 1..4 slices: 16 x 22 shapes of 17..2048 rows, N = 1024
+// .. 12288, K = 1000..6144.  The kernel chosen (the small-M kernel among them, up
+// to 256 rows) is on average 0.3 % and at most 8 % slower than the best of its
+// shape with weights from HBM, 0.6 % and 13 % with repeated ones.  (Constants from
+// repeated launches alone had picked the 3-deep ring for single rounds of 64 x 128
+// tiles: 17-18 us at 64 x 12288 and 256 x 4096, K = 2048, where 4 stages take
+// 13.5-14.5; repeated, both take 13.3.)  K slices (the 4-wave configurations take
+// them) cost a merge of three dependent memory round trips, so they pay only where
+// the tiles leave most CUs idle: offered up to 128 tiles (333 x 2048 x 6144: 30.6
+// us unsplit, 23.3 with 4 slices of 128 x 128).
+struct B16Plan {
+  int cfg, split;
+  float us;
+};
+static B16Plan b16_best(int MG, int NG, int KB) {
+  B16Plan best{0, 1, 3.0e38f};
+  auto offer = [&](int c, int s, float us) {
+    if (us < best.us) best = B16Plan{c, s, us};
+  };
+  // 8 waves, one work-group per CU
+  offer(4, 1, cdiv(b16_tiles(4, MG, NG), 256) * (10.3f + 1.1f * KB));
+  offer(5, 1, cdiv(b16_tiles(5, MG, NG), 256) * (6.71f + 0.638f * KB));
+  // 4 waves, work-groups share CUs: the time of a k-block grows with each half
+  // round of 256 (and part of the later ones' fixed time runs under others' loops)
+  static const float fixed[3] = {5.9f, 5.3f, 4.92f}, alone[3] = {0.416f, 0.256f, 0.362f},
+                     shared[3] = {0.483f, 0.282f, 0.306f}, later[3] = {-1.06f, 0.954f, -0.197f},
+                     merge[2] = {2.23f, 3.0f}, part[2] = {0.0267f, 0.0139f};
+  for (int c = 6; c <= 8; c++) {
+    const int i = c - 6, tiles = b16_tiles(c, MG, NG);
+    for (int s = 1; s <= (c < 8 && tiles <= 128 ? 4 : 1) && s <= KB; s++) {
+      const float half = 0.5f * (float)cdiv(tiles * s, 128), kb = (float)KB / s;
+      offer(c, s, fixed[i] + (tiles * s <= 256 ? kb * alone[i] : kb * shared[i] * half + later[i] * (half - 1.0f)) +
+                      (s > 1 ? merge[i] + part[i] * tiles * s : 0.0f));
+    }
+  }
+  return best;
+}
+// estimated us of the wave-grid kernel's plan
+float gemm_b16_us(int M, int N, int K) { return b16_best(cdiv(M, 16), cdiv(N, 16), cdiv(K, 64)).us; }
+
 static void b16_plan(int MG, int NG, int KB, bool off32, int& cfg_out, int& split_out) {
   int cfg = 0, split = 1;
   if (off32) {
-    float best = 3.0e38f;
-    auto offer = [&](int c, int s, float us) {
-      if (us < best) {
-        best = us;
-        cfg = c;
-        split = s;
-      }
-    };
-    // 8 waves, one work-group per CU
-    offer(4, 1, cdiv(b16_tiles(4, MG, NG), 256) * (11.0f + 1.0f * KB));
-    offer(5, 1, cdiv(b16_tiles(5, MG, NG), 256) * (6.6f + 0.64f * KB));
-    // 4 waves, work-groups share CUs: the time of a k-block grows with each half
-    // round of 256
-    static const float fixed[3] = {6.2f, 5.2f, 4.7f}, alone[3] = {0.40f, 0.253f, 0.265f},
-                       shared[3] = {0.438f, 0.25f, 0.234f}, merge[2] = {4.6f, 4.3f};
-    for (int c = 6; c <= 8; c++) {
-      const int tiles = b16_tiles(c, MG, NG);
-      for (int s = 1; s <= (c < 8 && tiles <= 96 ? 4 : 1) && s <= KB; s++) {
-        const float half = 0.5f * (float)cdiv(tiles * s, 128), kb = (float)KB / s;
-        offer(c, s, fixed[c - 6] + (tiles * s <= 256 ? kb * alone[c - 6] : kb * shared[c - 6] * half + 1.2f * (half - 1.0f)) +
-                        (s > 1 ? merge[c - 6] + 0.0018f * tiles * s : 0.0f));
-      }
-    }
+    const B16Plan best = b16_best(MG, NG, KB);
+    cfg = best.cfg;
+    split = best.split;
   }
   const int fc = g_b16_force_cfg.load(std::memory_order_relaxed);
   const int fs = g_b16_force_split.load(std::memory_order_relaxed);
@@ -779,6 +796,14 @@ static void b16_plan(int MG, int NG, int KB, bool off32, int& cfg_out, int& spli
   if (split > 1 && (cfg == 4 || cfg == 5)) cfg = 6;   // the 4-wave configurations take slices
   cfg_out = cfg;
   split_out = split;
+}
+
+// the configuration and K slices that launch_gemm_b16 takes for L: the wave-grid
+// kernel where every X byte offset fits 32 bits, else the LDS-staged one with its
+// 64-bit addresses
+void gemm_b16_planned(const GemmLaunch& L, int* cfg, int* split) {
+  const bool off32 = (size_t)L.M * (size_t)L.lda * 2 < ((size_t)1 << 32);
+  b16_plan(cdiv(L.M, 16), cdiv(L.N, 16), cdiv(L.K, 64), off32, *cfg, *split);
 }
 
 // partial-sum bytes and arrival counters the launch of this shape needs (the
@@ -813,7 +838,7 @@ static void launch_b16(const GemmB16Args& a, int cfg, int blocks, hipStream_t st
     case 4: launch_b16_wave<AMODE, 4, 2, 2, 3, 3>(a, blocks, st); break;
     case 5: launch_b16_wave<AMODE, 2, 4, 4, 1, 4>(a, blocks, st); break;
     case 6: launch_b16_wave<AMODE, 1, 4, 4, 1, 3>(a, blocks, st); break;
-    case 7: launch_b16_wave<AMODE, 1, 4, 2, 1, 5>(a, blocks, st); break;
+    case 7: launch_b16_wave<AMODE, 1, 4, 2, 1, 4>(a, blocks, st); break;
     default: launch_b16_wave<AMODE, 1, 4, 2, 1, 3>(a, blocks, st); break;
   }
 }
@@ -844,10 +869,7 @@ hipError_t launch_gemm_b16(const GemmLaunch& L, hipStream_t st) {
   a.out = L.out;
   a.zero_tile = L.zero_tile;
   int best, sp;
-  // the wave-grid kernel where every X byte offset fits 32 bits, else the
-  // LDS-staged one with its 64-bit addresses
-  const bool off32 = (size_t)L.M * (size_t)L.lda * 2 < ((size_t)1 << 32);
-  b16_plan(a.MG, a.NG, a.KB, off32, best, sp);
+  gemm_b16_planned(L, &best, &sp);
   int mt, nt;
   b16_cfg(best, mt, nt);
   a.ntm = cdiv(a.MG, mt);

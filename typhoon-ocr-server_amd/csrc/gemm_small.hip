@@ -516,6 +516,34 @@ static void launch_small_mode(const GemmSmallArgs& a, int u, int r, int tg, hipS
 static std::atomic<int> g_small_b16_shape{0};
 void gemm_small_set_b16_shape(int code) { g_small_b16_shape.store(code, std::memory_order_relaxed); }
 
+// 16-bit rows, 17..256 tokens: the widest work-group, most weight row
+// groups R and then most token groups TG (each 4, 2 or 1, TG at most the
+// token groups there are), that still leaves >= 192 work-groups; batches
+// of 4 tiles only below 4 (row group, token group) pairs.  Measured over
+// every shape (R, TG, U) at K = 2048 and M = 32..256, N = 2048 / 4096 /
+// 12288: the best shape or within 2 % of it at every point, e.g.
+// M = 256, N = 2048: 4 x 2 groups 9.3 us (1 x 4: 13.3, the tiled kernel
+// 11.5); M = 64, N = 4096: 4 x 1 groups 7.1 us (2 x 1: 8.7).
+static void small_b16_shape(int MG, int NG, int& r, int& tg) {
+  for (r = 4; r >= 1; r >>= 1)
+    for (tg = 4; tg >= 1; tg >>= 1)
+      if (tg <= MG && (long long)cdiv(NG, r) * cdiv(MG, tg) >= 192) return;
+  r = 1;
+  tg = 1;
+}
+
+// Estimated us of 16-bit rows here: per round of 256 work-groups a fixed part and
+// each k-block's time grow with the row x token groups of a work-group.  Fitted to
+// the same launches as the tiled kernel's estimate (b16_best, gemm_b16.hip).
+float gemm_small_b16_us(int M, int N, int K) {
+  int r, tg;
+  const int MG = cdiv(M, 16), NG = cdiv(N, 16);
+  small_b16_shape(MG, NG, r, tg);
+  const int rounds = cdiv(cdiv(NG, r) * cdiv(MG, tg), 256);
+  const float pairs = (float)(r * tg), rd = (float)rounds;
+  return 2.99f + rd * (0.325f * pairs - 0.682f) + (float)cdiv(K, 64) * rd * (0.0145f * pairs + 0.0551f);
+}
+
 hipError_t launch_gemm_small(const GemmLaunch& L, hipStream_t st) {
   if (!gemm_small_supported(L)) return hipErrorInvalidValue;
   GemmSmallArgs a;
@@ -574,25 +602,7 @@ hipError_t launch_gemm_small(const GemmLaunch& L, hipStream_t st) {
     }
   }
   if (b16 && a.MG >= 2) {
-    // 16-bit rows, 17..256 tokens: the widest work-group, most weight row
-    // groups R and then most token groups TG (each 4, 2 or 1, TG at most the
-    // token groups there are), that still leaves >= 192 work-groups; batches
-    // of 4 tiles only below 4 (row group, token group) pairs.  Measured over
-    // every shape (R, TG, U) at K = 2048 and M = 32..256, N = 2048 / 4096 /
-    // 12288: the best shape or within 2 % of it at every point, e.g.
-    // M = 256, N = 2048: 4 x 2 groups 9.3 us (1 x 4: 13.3, the tiled kernel
-    // 11.5); M = 64, N = 4096: 4 x 1 groups 7.1 us (2 x 1: 8.7).
-    r = 1;
-    tg = 1;
-    bool found = false;
-    for (int cr = 4; cr >= 1 && !found; cr >>= 1)
-      for (int ct = 4; ct >= 1; ct >>= 1)
-        if (ct <= a.MG && (long long)cdiv(a.NG, cr) * cdiv(a.MG, ct) >= 192) {
-          r = cr;
-          tg = ct;
-          found = true;
-          break;
-        }
+    small_b16_shape(a.MG, a.NG, r, tg);
     u_force = (r * tg >= 4 || n_t < 8) ? 2 : 4;
   }
   if (b16) {

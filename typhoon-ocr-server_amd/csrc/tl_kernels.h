@@ -256,6 +256,10 @@ void tlk_gemm_needs(const GemmLaunch* L, size_t* part_bytes, size_t* counters);
 // whether the GEMM of M4 = 4 x tokens plane rows takes them grouped
 // (GemmLaunch.planes_grouped; the split launches' `grouped`)
 bool tlk_gemm_planes_grouped(int M4, int N, int K);
+// the plan of a shape with contiguous, aligned rows: returns the kernel (0 small-M,
+// 1 int8 tiled, 2 16-bit tiled, 3 generic), and the tiled kernels' configuration
+// and K slices
+int tlk_gemm_planned(int amode, int out, int M, int N, int K, int* cfg, int* split);
 void tlk_gemm_i8_set_cfg(int cfg);   // tuning override of the int8 GEMM (-1 = planner)
 void tlk_gemm_i8_set_split(int s);   // tuning override of its K slices (0 = planner)
 // tuning override of the 16-bit GEMM: tile configuration 0..2 (-1 = planner)
@@ -355,6 +359,8 @@ bool gemm_planes_grouped(int M4, int N, int K);
 // LDS-staged 16-bit MFMA GEMM (gemm_b16.hip): A_BF16 / A_F16, used for M > 16
 // when X rows are 16-byte aligned pieces
 bool gemm_b16_supported(const GemmLaunch& L);
+void gemm_b16_planned(const GemmLaunch& L, int* cfg, int* split);
+float gemm_b16_us(int M, int N, int K);         // its estimated time of a shape
 hipError_t launch_gemm_b16(const GemmLaunch& L, hipStream_t st);
 void gemm_b16_needs(int M, int N, int K, size_t* part_bytes, size_t* counters);
 void gemm_b16_set_plan(int cfg, int split);
@@ -363,6 +369,7 @@ void gemm_small_set_b16_shape(int code);
 void gemm_needs(const GemmLaunch& L, size_t* part_bytes, size_t* counters);
 // M <= 16 rows (gemm_small.hip): GEMV-shaped MFMA kernel
 bool gemm_small_supported(const GemmLaunch& L);
+float gemm_small_b16_us(int M, int N, int K);   // its estimated time of 17..256 16-bit rows
 hipError_t launch_gemm_small(const GemmLaunch& L, hipStream_t st);
 
 bool rows_supported(const GemmLaunch& L);
