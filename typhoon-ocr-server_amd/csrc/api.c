@@ -596,7 +596,7 @@ done:
 static int run_gemm(Workspace* ws, GemmLaunch* L, hipStream_t st) {
   TRY(zero_tile(&L->zero_tile));
   size_t part_bytes = 0, counters = 0;
-  tlk_gemm_needs(L, &part_bytes, &counters);
+  tlk_gemm_resolve(L, &part_bytes, &counters);
   if (part_bytes > 0) {
     TRY(tlh_devbuf_ensure(&ws->part, part_bytes, st));
     L->part = ws->part.p;

@@ -361,17 +361,6 @@ GemmPlan gemm_plan(int amode, int M, int N, int K) {
   return p;
 }
 
-size_t gemm_workspace_bytes(int amode, int M, int N, int K) {
-  GemmPlan p = gemm_plan(amode, M, N, K);
-  if (p.split <= 1) return 0;
-  return (size_t)p.split * cdiv(M, 16) * 16 * (size_t)cdiv(N, 16) * 16 * 4;
-}
-
-size_t gemm_counter_count(int amode, int M, int N, int K) {
-  GemmPlan p = gemm_plan(amode, M, N, K);
-  return (size_t)p.ntm * p.ntn;
-}
-
 template <int AMODE>
 static hipError_t launch_mode(const GemmArgs& a, int cfg, int blocks, hipStream_t st) {
   if (cfg == 0)
@@ -383,7 +372,7 @@ static hipError_t launch_mode(const GemmArgs& a, int cfg, int blocks, hipStream_
   return hipGetLastError();
 }
 
-// which kernel launch_gemm runs for L
+// which kernel runs L
 enum GemmKernel { GK_SMALL, GK_I8, GK_B16, GK_GENERIC };
 static GemmKernel gemm_choice(const GemmLaunch& L) {
   if (L.planes_grouped) return GK_I8;      // only the quadrant kernel reads that layout
@@ -443,26 +432,26 @@ int gemm_planned(int amode, int out, int M, int N, int K, int* cfg, int* split) 
   L.N = N;
   L.K = L.lda = K;
   L.zero_tile = zeros;
-  const GemmKernel k = gemm_choice(L);
-  *cfg = 0;
-  *split = 1;
-  if (k == GK_B16) gemm_b16_planned(L, cfg, split);
-  return k;
+  size_t part_bytes, counters;
+  gemm_resolve(L, &part_bytes, &counters);
+  *cfg = L.cfg;
+  *split = L.split;
+  return L.kernel;
 }
 
-// split work-space of the kernel launch_gemm picks for L: partial-sum bytes
-// and zeroed arrival counters (0 and 0 when it needs none)
-void gemm_needs(const GemmLaunch& L, size_t* part_bytes, size_t* counters) {
+void gemm_resolve(GemmLaunch& L, size_t* part_bytes, size_t* counters) {
   *part_bytes = 0;
   *counters = 0;
-  switch (gemm_choice(L)) {
+  L.kernel = gemm_choice(L);
+  L.cfg = 0;
+  L.split = 1;
+  switch (L.kernel) {
     case GK_SMALL: return;
-    case GK_I8: gemm_i8_needs(L, part_bytes, counters); return;
-    case GK_B16: gemm_b16_needs(L.M, L.N, L.K, part_bytes, counters); return;
+    case GK_I8: gemm_i8_resolve(L, part_bytes, counters); return;
+    case GK_B16: gemm_b16_resolve(L, part_bytes, counters); return;
     default: break;
   }
-  GemmPlan p = gemm_plan(L.amode, L.M, L.N, L.K);
-  if (L.force_split > 0) p.split = L.force_split;
+  const GemmPlan p = gemm_plan(L.amode, L.M, L.N, L.K);
   if (p.split > 1) {
     *part_bytes = (size_t)p.split * cdiv(L.M, 16) * 16 * (size_t)cdiv(L.N, 16) * 16 * 4;
     *counters = (size_t)p.ntm * p.ntn;
@@ -487,24 +476,20 @@ hipError_t launch_gemm(const GemmLaunch& L, hipStream_t st) {
   a.NG = cdiv(L.N, 16);
   a.ep = L.ep;
   a.out = L.out;
-  GemmPlan p = gemm_plan(L.amode, L.M, L.N, L.K);
-  if (L.force_split > 0) {
-    p.split = L.force_split;
-    p.blocks = p.ntm * p.ntn * p.split;
-  }
+  const GemmPlan p = gemm_plan(L.amode, L.M, L.N, L.K);
   a.S = p.split;
   a.ntn = p.ntn;
   a.part = L.part;
   a.cnt = L.cnt;
   if (L.amode == A_I8 && L.out != OUT_I32 && L.out != OUT_F32_X4 && !L.xs) return hipErrorInvalidValue;
   if (L.out == OUT_F32_X4 && L.amode != A_I8) return hipErrorInvalidValue;
-  switch (gemm_choice(L)) {
+  switch (L.kernel) {
     case GK_SMALL: return launch_gemm_small(L, st);
     case GK_I8: return launch_gemm_i8(L, st);
     case GK_B16: return launch_gemm_b16(L, st);
-    default: break;
+    case GK_GENERIC: break;
+    default: return hipErrorInvalidValue;   // not resolved
   }
-  // the generic kernel's K split needs the work-space gemm_needs reports
   if (p.split > 1 && (!L.part || !L.cnt)) return hipErrorInvalidValue;
   switch (L.amode) {
     case A_I8: return launch_mode<A_I8>(a, p.cfg, p.blocks, st);
@@ -522,14 +507,9 @@ hipError_t launch_gemm(const GemmLaunch& L, hipStream_t st) {
 // ---------------------------------------------------------------------------
 extern "C" {
 bool tlk_gemm_planes_grouped(int M4, int N, int K) { return tl::gemm_planes_grouped(M4, N, K); }
-void tlk_gemm_plan(int amode, int M, int N, int K, GemmPlan* plan) { *plan = tl::gemm_plan(amode, M, N, K); }
-size_t tlk_gemm_workspace_bytes(int amode, int M, int N, int K) {
-  return tl::gemm_workspace_bytes(amode, M, N, K);
-}
-size_t tlk_gemm_counter_count(int amode, int M, int N, int K) { return tl::gemm_counter_count(amode, M, N, K); }
 hipError_t tlk_launch_gemm(const GemmLaunch* L, hipStream_t st) { return tl::launch_gemm(*L, st); }
-void tlk_gemm_needs(const GemmLaunch* L, size_t* part_bytes, size_t* counters) {
-  tl::gemm_needs(*L, part_bytes, counters);
+void tlk_gemm_resolve(GemmLaunch* L, size_t* part_bytes, size_t* counters) {
+  tl::gemm_resolve(*L, part_bytes, counters);
 }
 void tlk_gemm_b16_set_plan(int cfg, int split) { tl::gemm_b16_set_plan(cfg, split); }
 int tlk_gemm_planned(int amode, int out, int M, int N, int K, int* cfg, int* split) {

@@ -798,31 +798,17 @@ static void b16_plan(int MG, int NG, int KB, bool off32, int& cfg_out, int& spli
   split_out = split;
 }
 
-// the configuration and K slices that launch_gemm_b16 takes for L: the wave-grid
-// kernel where every X byte offset fits 32 bits, else the LDS-staged one with its
-// 64-bit addresses
-void gemm_b16_planned(const GemmLaunch& L, int* cfg, int* split) {
+// the wave-grid kernel where every X byte offset fits 32 bits, else the LDS-staged
+// one with its 64-bit addresses
+void gemm_b16_resolve(GemmLaunch& L, size_t* part_bytes, size_t* counters) {
+  const int MG = cdiv(L.M, 16), NG = cdiv(L.N, 16);
   const bool off32 = (size_t)L.M * (size_t)L.lda * 2 < ((size_t)1 << 32);
-  b16_plan(cdiv(L.M, 16), cdiv(L.N, 16), cdiv(L.K, 64), off32, *cfg, *split);
-}
-
-// partial-sum bytes and arrival counters the launch of this shape needs (the
-// larger of the two plans: which one the launch takes depends on the row stride,
-// which is not known here)
-void gemm_b16_needs(int M, int N, int K, size_t* part_bytes, size_t* counters) {
-  const int MG = cdiv(M, 16), NG = cdiv(N, 16);
-  *part_bytes = 0;
-  *counters = 0;
-  for (int off32 = 0; off32 < 2; off32++) {
-    int cfg, sp, mt, nt;
-    b16_plan(MG, NG, cdiv(K, 64), off32 != 0, cfg, sp);
-    b16_cfg(cfg, mt, nt);
-    const size_t tiles = (size_t)cdiv(MG, mt) * cdiv(NG, nt);
-    if (sp > 1) {
-      *part_bytes = std::max(*part_bytes, tiles * sp * (size_t)(256 * mt * nt) * sizeof(float));
-      *counters = std::max(*counters, tiles);
-    }
-  }
+  int mt, nt;
+  b16_plan(MG, NG, cdiv(L.K, 64), off32, L.cfg, L.split);
+  b16_cfg(L.cfg, mt, nt);
+  const size_t tiles = (size_t)cdiv(MG, mt) * cdiv(NG, nt);
+  *part_bytes = L.split > 1 ? tiles * L.split * (size_t)(256 * mt * nt) * sizeof(float) : 0;
+  *counters = L.split > 1 ? tiles : 0;
 }
 
 template <int AMODE, int WM, int WN, int RM, int CN, int NST>
@@ -868,10 +854,9 @@ hipError_t launch_gemm_b16(const GemmLaunch& L, hipStream_t st) {
   a.NG = cdiv(L.N, 16);
   a.out = L.out;
   a.zero_tile = L.zero_tile;
-  int best, sp;
-  gemm_b16_planned(L, &best, &sp);
+  const int sp = L.split;
   int mt, nt;
-  b16_cfg(best, mt, nt);
+  b16_cfg(L.cfg, mt, nt);
   a.ntm = cdiv(a.MG, mt);
   a.ntn = cdiv(a.NG, nt);
   a.S = sp;
@@ -881,8 +866,8 @@ hipError_t launch_gemm_b16(const GemmLaunch& L, hipStream_t st) {
   const long long blocks_ll = (long long)a.ntm * a.ntn * sp;
   if (blocks_ll > 0x7fffffffLL) return hipErrorInvalidValue;
   const int blocks = (int)blocks_ll;
-  if (L.amode == A_BF16) launch_b16<A_BF16>(a, best, blocks, st);
-  else launch_b16<A_F16>(a, best, blocks, st);
+  if (L.amode == A_BF16) launch_b16<A_BF16>(a, L.cfg, blocks, st);
+  else launch_b16<A_F16>(a, L.cfg, blocks, st);
   return hipGetLastError();
 }
 

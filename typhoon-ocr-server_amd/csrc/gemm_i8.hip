@@ -709,14 +709,14 @@ static void gemm_i8_plan(const GemmLaunch& L, int& cfg, int& split) {
   }
 }
 
-void gemm_i8_needs(const GemmLaunch& L, size_t* part_bytes, size_t* counters) {
-  int cfg, sp, mt, nt;
-  gemm_i8_plan(L, cfg, sp);
-  i8_cfg(cfg, mt, nt);
+void gemm_i8_resolve(GemmLaunch& L, size_t* part_bytes, size_t* counters) {
+  int mt, nt;
+  gemm_i8_plan(L, L.cfg, L.split);
+  i8_cfg(L.cfg, mt, nt);
   const int MG = L.out == OUT_F32_X4 ? planes_groups(L.M / 4, true) : cdiv(L.M, 16);
   const size_t tiles = (size_t)cdiv(MG, mt) * cdiv(cdiv(L.N, 16), nt);
-  *part_bytes = sp > 1 ? tiles * sp * (size_t)(256 * mt * nt) * sizeof(int32_t) : 0;
-  *counters = sp > 1 ? tiles : 0;
+  *part_bytes = L.split > 1 ? tiles * L.split * (size_t)(256 * mt * nt) * sizeof(int32_t) : 0;
+  *counters = L.split > 1 ? tiles : 0;
 }
 
 // planes on 256 x 256, 256 x 192 and 128 x 128 tiles, codes on 128 x 192 and
@@ -761,10 +761,9 @@ hipError_t launch_gemm_i8(const GemmLaunch& L, hipStream_t st) {
   if (!L.zero_tile) return hipErrorInvalidValue;
   // planes come grouped (gemm_planes_grouped)
   if (L.out == OUT_F32_X4 && !L.planes_grouped) return hipErrorInvalidValue;
-  int cfg, sp;
-  gemm_i8_plan(L, cfg, sp);
+  const int sp = L.split;
   int mt, nt;
-  i8_cfg(cfg, mt, nt);
+  i8_cfg(L.cfg, mt, nt);
   a.ntm = cdiv(a.MG, mt);
   a.ntn = cdiv(a.NG, nt);
   a.S = sp;
@@ -780,7 +779,7 @@ hipError_t launch_gemm_i8(const GemmLaunch& L, hipStream_t st) {
   const long long blocks_ll = (long long)a.ntm * a.ntn * sp;
   if (blocks_ll > 0x7fffffffLL) return hipErrorInvalidValue;
   const int blocks = (int)blocks_ll;
-  switch (cfg) {
+  switch (L.cfg) {
     case 0: hipLaunchKernelGGL((gemm_i8_lds_kernel<8, 12, 1, 4, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;
     case 1: hipLaunchKernelGGL((gemm_i8_lds_kernel<4, 8, 1, 8, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;
     case 2: hipLaunchKernelGGL((gemm_i8_lds_kernel<8, 8, 1, 8, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;

@@ -227,14 +227,15 @@ typedef struct GemmLaunch {
   int ldy TLK_DEF(0);
   int M TLK_DEF(0), N TLK_DEF(0), K TLK_DEF(0);
   int ep TLK_DEF(EP_SCALE), out TLK_DEF(OUT_F32);
-  void* part TLK_DEF(nullptr);           // split workspace (gemm_workspace_bytes)
-  uint32_t* cnt TLK_DEF(nullptr);        // gemm_counter_count zeroed counters
-  int force_split TLK_DEF(0);
+  void* part TLK_DEF(nullptr);           // partial sums and zeroed arrival counters, of the
+  uint32_t* cnt TLK_DEF(nullptr);        //   sizes tlk_gemm_resolve gives
   const uint8_t* zero_tile TLK_DEF(nullptr);   // 1 KiB of device zeros (LDS-staged int8 GEMM)
   const int* xe TLK_DEF(nullptr);        // OUT_F32_X4: per-token power-of-two exponents (split_i8x4)
   const float* xraw TLK_DEF(nullptr);    // OUT_F32_X4: the fp32 token rows [M / 4][ldxr] the planes came
   int ldxr TLK_DEF(0);                   //   from (outputs of a non-finite row from them); null: NaN
   bool planes_grouped TLK_DEF(false);    // OUT_F32_X4: row group 4T + p holds plane p of tokens 16T .. 16T + 15
+  // set by tlk_gemm_resolve: the kernel (-1 none yet), its configuration and K slices
+  int kernel TLK_DEF(-1), cfg TLK_DEF(0), split TLK_DEF(1);
 } GemmLaunch;
 static inline GemmLaunch tlk_gemm_launch_init(void) {
   GemmLaunch L;
@@ -242,17 +243,18 @@ static inline GemmLaunch tlk_gemm_launch_init(void) {
   L.amode = A_I8;
   L.ep = EP_SCALE;
   L.out = OUT_F32;
+  L.kernel = -1;
+  L.split = 1;
   return L;
 }
-void tlk_gemm_plan(int amode, int M, int N, int K, GemmPlan* plan);
-size_t tlk_gemm_workspace_bytes(int amode, int M, int N, int K);
-size_t tlk_gemm_counter_count(int amode, int M, int N, int K);
-// every GEMM shape: the small-M, int8 LDS-staged, 16-bit LDS-staged or
-// generic MFMA kernel
+// every GEMM shape: picks the small-M, tiled int8, tiled 16-bit or generic MFMA
+// kernel, its configuration and K slices into *L, and gives the work-space of that
+// choice: partial-sum bytes (L->part) and zeroed arrival counters (L->cnt); 0 when
+// none.  The launch takes the choice from *L: a tuning setter of another thread
+// between the two calls cannot make it use more work-space than was sized.
+void tlk_gemm_resolve(GemmLaunch* L, size_t* part_bytes, size_t* counters);
+// (hipErrorInvalidValue for an L that was not resolved)
 hipError_t tlk_launch_gemm(const GemmLaunch* L, hipStream_t st);
-// split work-space of the kernel tlk_launch_gemm picks for *L: partial-sum
-// bytes (L->part) and zeroed arrival counters (L->cnt); 0 when none
-void tlk_gemm_needs(const GemmLaunch* L, size_t* part_bytes, size_t* counters);
 // whether the GEMM of M4 = 4 x tokens plane rows takes them grouped
 // (GemmLaunch.planes_grouped; the split launches' `grouped`)
 bool tlk_gemm_planes_grouped(int M4, int N, int K);
@@ -345,28 +347,25 @@ hipError_t launch_gemv_i8(const GemvLaunch& L, hipStream_t st);
 void gemv_set_plan(int rows, int u);
 
 GemmPlan gemm_plan(int amode, int M, int N, int K);
-size_t gemm_workspace_bytes(int amode, int M, int N, int K);
-size_t gemm_counter_count(int amode, int M, int N, int K);
 hipError_t launch_gemm(const GemmLaunch& L, hipStream_t st);
 
 // W8A8 LDS-staged int8 MFMA GEMM (gemm_i8.hip), used for M > 16
 hipError_t launch_gemm_i8(const GemmLaunch& L, hipStream_t st);
 void gemm_i8_set_cfg(int cfg);
 void gemm_i8_set_split(int s);
-void gemm_i8_needs(const GemmLaunch& L, size_t* part_bytes, size_t* counters);
+void gemm_i8_resolve(GemmLaunch& L, size_t* part_bytes, size_t* counters);
 bool gemm_planes_grouped(int M4, int N, int K);
 
 // LDS-staged 16-bit MFMA GEMM (gemm_b16.hip): A_BF16 / A_F16, used for M > 16
 // when X rows are 16-byte aligned pieces
 bool gemm_b16_supported(const GemmLaunch& L);
-void gemm_b16_planned(const GemmLaunch& L, int* cfg, int* split);
 float gemm_b16_us(int M, int N, int K);         // its estimated time of a shape
 hipError_t launch_gemm_b16(const GemmLaunch& L, hipStream_t st);
-void gemm_b16_needs(int M, int N, int K, size_t* part_bytes, size_t* counters);
+void gemm_b16_resolve(GemmLaunch& L, size_t* part_bytes, size_t* counters);
 void gemm_b16_set_plan(int cfg, int split);
 int gemm_b16_forced_cfg();
 void gemm_small_set_b16_shape(int code);
-void gemm_needs(const GemmLaunch& L, size_t* part_bytes, size_t* counters);
+void gemm_resolve(GemmLaunch& L, size_t* part_bytes, size_t* counters);
 // M <= 16 rows (gemm_small.hip): GEMV-shaped MFMA kernel
 bool gemm_small_supported(const GemmLaunch& L);
 float gemm_small_b16_us(int M, int N, int K);   // its estimated time of 17..256 16-bit rows
