@@ -93,3 +93,50 @@ def test_override_between_sizing_and_launch(lin, dev, amode, M, N, K):
         override(lib, amode, 0)
     assert (pbuf[part // 4:] == 123).all() and (cbuf == 0).all()
     assert torch.equal(y.cpu(), want)
+
+
+class RowsPlan(ctypes.Structure):            # csrc/tl_kernels.h
+    _fields_ = [(n, i32) for n in ("tg", "nkb", "cpt", "kbs", "split", "r", "blocks")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(2, 2048, 6144), (7, 270, 4096)])
+def test_rows_override_between_sizing_and_launch(lin, dev, M, N, K):
+    """The same for the digit rows of up to 8 fp32 tokens: planned in 2 slices (or
+    the fewest that fit), launched after the override went to 16."""
+    import torch
+    say(f"rows plan M={M} N={N} K={K}")
+    lib = lin.load_library()
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randint(-3, 4, (M, K), generator=g).float()
+    w = torch.randint(-3, 4, (N, K), generator=g).float()
+    w[:, 0] = 127.0
+    want = (x.double() @ w.double().T).float()
+    wt = torch.zeros((N + 15) // 16 * 16 * K, dtype=torch.uint8, device=dev)
+    ws = torch.zeros((N + 15) // 16 * 16, device=dev)
+    lin.w8a8_quantize_tiles_dev(w.to(dev), wt, ws)
+    xd = x.to(dev)
+    y = torch.full((M, N), -1.0, device=dev)
+    L = GemmLaunch(amode=3, A=xd.data_ptr(), lda=K, Bt=wt.data_ptr(), ws=ws.data_ptr(), Y=y.data_ptr(), ldy=N, M=M, N=N,
+                   K=K, ep=0, out=OUT_F32, kernel=-1, split=1)
+    plan = RowsPlan()
+    lib.tlk_rows_workspace_bytes.restype = lib.tlk_rows_counter_count.restype = ctypes.c_size_t
+    try:
+        assert lib.tl_rows_set_split(2) == 0
+        lib.tlk_rows_plan(M, N, K, ctypes.byref(plan))
+        part = lib.tlk_rows_workspace_bytes(ctypes.byref(plan), M, N)
+        assert 2 <= plan.split <= 4 and part == plan.split * M * N * 4
+        assert lib.tl_rows_set_split(16) == 0
+        pbuf = torch.full((part // 4 + 4096,), 123, dtype=torch.int32, device=dev)
+        cbuf = torch.zeros(lib.tlk_rows_counter_count(N) + 64, dtype=torch.int32, device=dev)
+        L.part, L.cnt = pbuf.data_ptr(), cbuf.data_ptr()
+        for _ in range(2):
+            assert lib.tlk_launch_rows(ctypes.byref(L), ctypes.byref(plan),
+                                       vp(torch.cuda.current_stream().cuda_stream)) == 0
+        torch.cuda.synchronize()
+    finally:
+        assert lib.tl_rows_set_split(0) == 0
+    assert (pbuf[part // 4:] == 123).all() and (cbuf == 0).all()
+    # the planes hold a value to 2^-32 of its row's absmax; the fold, the scale and
+    # the slices' sum round at most 16 times, each within 2^-24 of the sum of terms
+    assert ((y.cpu() - want).abs() <= 16 * 2.0 ** -24 * (x.abs() @ w.abs().T)).all()

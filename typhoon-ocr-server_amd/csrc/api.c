@@ -633,11 +633,11 @@ static int run_rows(Workspace* ws, GemmLaunch* L, hipStream_t st, bool* done) {
   RowsPlan p;
   tlk_rows_plan(L->M, L->N, L->K, &p);
   if (p.split > 1) {
-    TRY(tlh_devbuf_ensure(&ws->part, tlk_rows_workspace_bytes(L->M, L->N, L->K), st));
+    TRY(tlh_devbuf_ensure(&ws->part, tlk_rows_workspace_bytes(&p, L->M, L->N), st));
     L->part = ws->part.p;
     TRY(ensure_counters(ws, tlk_rows_counter_count(L->N), st, &L->cnt));
   }
-  HIP_TRY(tlk_launch_rows(L, st));
+  HIP_TRY(tlk_launch_rows(L, &p, st));
   *done = true;
   return 0;
 }

@@ -461,10 +461,6 @@ RowsPlan rows_plan(int M, int N, int K) {
   return p;
 }
 
-size_t rows_workspace_bytes(int M, int N, int K) {
-  const RowsPlan p = rows_plan(M, N, K);
-  return p.split > 1 ? (size_t)p.split * M * N * sizeof(float) : 0;
-}
 size_t rows_counter_count(int N) { return (size_t)cdiv(N, 16); }
 
 template <int AMODE, int TG, int NKB, int R>
@@ -495,9 +491,8 @@ static void launch_rows_mode(const RowsArgs& a, const RowsPlan& p, hipStream_t s
   }
 }
 
-hipError_t launch_rows(const GemmLaunch& L, hipStream_t st) {
+hipError_t launch_rows(const GemmLaunch& L, const RowsPlan& p, hipStream_t st) {
   if (!rows_supported(L)) return hipErrorInvalidValue;
-  const RowsPlan p = rows_plan(L.M, L.N, L.K);
   const int lmp = L.M <= 1 ? 0 : (L.M <= 2 ? 1 : (L.M <= 4 ? 2 : 3));
   if ((p.tg == 2 && p.nkb > 32) || p.split < 1 || (p.kbs << lmp) * 4 > 256 * p.cpt) return hipErrorInvalidValue;
   if (p.r < 1 || p.r > 3 || (p.r > 1 && p.nkb > 32) || p.blocks != cdiv(cdiv(L.N, 16), p.r) * p.split)
@@ -535,10 +530,12 @@ hipError_t launch_rows(const GemmLaunch& L, hipStream_t st) {
 extern "C" {
 bool tlk_rows_supported(const GemmLaunch* L) { return tl::rows_supported(*L); }
 void tlk_rows_plan(int M, int N, int K, RowsPlan* plan) { *plan = tl::rows_plan(M, N, K); }
-size_t tlk_rows_workspace_bytes(int M, int N, int K) { return tl::rows_workspace_bytes(M, N, K); }
+size_t tlk_rows_workspace_bytes(const RowsPlan* p, int M, int N) {
+  return p->split > 1 ? (size_t)p->split * M * N * sizeof(float) : 0;
+}
 size_t tlk_rows_counter_count(int N) { return tl::rows_counter_count(N); }
 void tlk_rows_set_split(int s) { tl::rows_set_split(s); }
 int tlk_rows_forced_split(void) { return tl::g_rows_force_split.load(std::memory_order_relaxed); }
 void tlk_rows_set_groups(int r) { tl::rows_set_groups(r); }
-hipError_t tlk_launch_rows(const GemmLaunch* L, hipStream_t st) { return tl::launch_rows(*L, st); }
+hipError_t tlk_launch_rows(const GemmLaunch* L, const RowsPlan* p, hipStream_t st) { return tl::launch_rows(*L, *p, st); }
 }  // extern "C"

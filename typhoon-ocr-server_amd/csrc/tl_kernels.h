@@ -276,13 +276,15 @@ typedef struct RowsPlan {
       blocks TLK_DEF(0);
 } RowsPlan;
 bool tlk_rows_supported(const GemmLaunch* L);
+// made once a call: sizes and launch take the same plan, whatever a tuning setter
+// of another thread does in between
 void tlk_rows_plan(int M, int N, int K, RowsPlan* plan);
-size_t tlk_rows_workspace_bytes(int M, int N, int K);   // partials when split > 1
+size_t tlk_rows_workspace_bytes(const RowsPlan* plan, int M, int N);   // partials when split > 1
 size_t tlk_rows_counter_count(int N);                   // zeroed arrival counters
 void tlk_rows_set_split(int s);                         // tuning override (0 = planner)
 int tlk_rows_forced_split(void);                        // that override (0 = none)
 void tlk_rows_set_groups(int r);                        // tuning override (0 = planner)
-hipError_t tlk_launch_rows(const GemmLaunch* L, hipStream_t st);
+hipError_t tlk_launch_rows(const GemmLaunch* L, const RowsPlan* plan, hipStream_t st);
 
 #ifdef __cplusplus
 }  // extern "C"
@@ -373,11 +375,10 @@ hipError_t launch_gemm_small(const GemmLaunch& L, hipStream_t st);
 
 bool rows_supported(const GemmLaunch& L);
 RowsPlan rows_plan(int M, int N, int K);
-size_t rows_workspace_bytes(int M, int N, int K);
 size_t rows_counter_count(int N);
 void rows_set_split(int s);
 void rows_set_groups(int r);
-hipError_t launch_rows(const GemmLaunch& L, hipStream_t st);
+hipError_t launch_rows(const GemmLaunch& L, const RowsPlan& p, hipStream_t st);
 
 }  // namespace tl
 #endif
