@@ -55,3 +55,11 @@ def lib(pkg):
 
 def test_w8a16_planner(lib):
     _check(_costs(lib, "w8a16", A_BF16, OUT_BF16), {"hbm": (1.007, 1.11), "repeated": (1.013, 1.17)})
+
+
+def test_w8a8_planner(lib):
+    _check(_costs(lib, "w8a8", A_I8, OUT_F32), {"hbm": (1.01, 1.2), "repeated": (1.018, 1.32)})
+
+
+def test_w8a32_planner(lib):
+    _check(_costs(lib, "w8a32", A_I8, OUT_F32_X4, planes=4), {"hbm": (1.01, 1.32), "repeated": (1.008, 1.26)})

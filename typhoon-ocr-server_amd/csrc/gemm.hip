@@ -376,9 +376,8 @@ static hipError_t launch_mode(const GemmArgs& a, int cfg, int blocks, hipStream_
 enum GemmKernel { GK_SMALL, GK_I8, GK_B16, GK_GENERIC };
 static GemmKernel gemm_choice(const GemmLaunch& L) {
   if (L.planes_grouped) return GK_I8;      // only the quadrant kernel reads that layout
-  // up to 16 token rows always stream the weights once; more rows too while N
-  // is small (N <= 4096: the tiled kernels would leave CUs idle), up to 64
-  // int8 rows; for wide N the activation
+  // up to 16 token rows always stream the weights once; more rows too while N and K
+  // are small (the tiled kernels would leave CUs idle); for wide N the activation
   // fragments every work-group re-reads cost more than the tiled kernels' reuse,
   // except up to 32 int8 rows at lm_head width (>= 2048 row groups, four per
   // work-group share each fragment): the int8 planes of 5-8 fp32 tokens,
@@ -396,13 +395,15 @@ static GemmKernel gemm_choice(const GemmLaunch& L) {
   // 12288, K = 2048 13.1 against 15.7 / 15.6 against 14.4
   const int ng = cdiv(L.N, 16);
   const bool b16_small = b16 && L.M <= 256 && gemm_small_b16_us(L.M, L.N, L.K) < gemm_b16_us(L.M, L.N, L.K);
-  const bool wide_i8 = L.amode == A_I8 && L.M <= 32 && ng >= 2048;
-  // int8 codes and fp32 rows: up to 64 rows at N <= 6144 and 32 rows at
-  // N <= 12288 (W8A8 at K = 2048, N = 6144, 24..64 rows: 8.1-11.0 us against
-  // 12.7-13.7 us on the tiled kernel; N = 12288 at 24 / 32 rows 12.1 / 12.4
-  // against 13.4, at 48 / 64 rows 15.4 / 16.3 against 14.2 / 14.4)
-  const bool mid_i8 = !b16 && ((L.M <= 64 && ng <= 384) || (L.M <= 32 && ng <= 768));
-  if (gemm_small_supported(L) && (L.M <= 16 || mid_i8 || b16_small || wide_i8))
+  // int8 code and plane rows past 16: at lm_head width up to 32 rows; else the
+  // smaller estimate again (codes at K = 2048, N = 6144 / 12288, 64 rows 9.0 against
+  // 11.2 / 14.1 against 11.8 us; N = K = 6144 21.6 against 16.8)
+  const bool i8_small = L.amode == A_I8 && L.M <= 64 &&
+                        (ng >= 2048 ? L.M <= 32
+                                    : gemm_small_i8_us(L.out, L.M, L.N, L.K) < gemm_i8_us(L.out, L.M, L.N, L.K));
+  // fp32 rows: up to 64 rows at N <= 6144 and 32 rows at N <= 12288
+  const bool f32_small = L.amode == A_F32X3 && ((L.M <= 64 && ng <= 384) || (L.M <= 32 && ng <= 768));
+  if (gemm_small_supported(L) && (L.M <= 16 || b16_small || i8_small || f32_small))
     return GK_SMALL;
   if (L.amode == A_I8 && L.M > 16) return GK_I8;
   if (L.amode != A_I8 && L.M > 16 && gemm_b16_supported(L)) return GK_B16;

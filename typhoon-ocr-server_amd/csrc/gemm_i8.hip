@@ -635,24 +635,6 @@ static std::atomic<int> g_i8_force_split{0};
 void gemm_i8_set_cfg(int cfg) { g_i8_force_cfg.store(cfg, std::memory_order_relaxed); }
 void gemm_i8_set_split(int s) { g_i8_force_split.store(s > 0 ? s : 0, std::memory_order_relaxed); }
 
-// K slices of `tiles` tiles whose work-groups would leave most CUs idle.  A merge
-// costs three dependent memory round trips (partials stored, arrival counted,
-// partials read back), about 3 us, and at K = 2048 every slice count measured
-// slower than none.
-// Codes, 64 x 128 tiles: below 128 tiles at K >= 4096 up to 4 slices of at
-// least 16 k-blocks (200 x 2048 x 6144: 18.2 -> 14.9 us).
-static int codes_slices(int tiles, int KB) {
-  if (tiles >= 128 || KB < 64) return 1;
-  return std::min(std::min(4, 256 / tiles), KB / 16);
-}
-// Planes, 128 x 128 tiles: 4 slices up to 32 tiles, 3 up to 64, 2 up to 95 (the
-// last from K = 6144), measured with 1..8 (20 / 100 / 160 tokens, 2048 x 6144:
-// 24.9 -> 18.1, 27.6 -> 23.3, 28.2 -> 26.4 us).
-static int planes_slices(int tiles, int KB) {
-  if (KB < 64) return 1;
-  return tiles <= 32 ? 4 : (tiles <= 64 ? 3 : (tiles < 96 && KB >= 96 ? 2 : 1));
-}
-
 // the configuration that runs where `cfg` is forced: planes have no 128 x 192
 // tiles and only quadrant ones, codes no 256-row ones (7 is 128 x 128 too)
 static int i8_resolve(int cfg, bool planes) {
@@ -660,43 +642,72 @@ static int i8_resolve(int cfg, bool planes) {
   return cfg == 3 || cfg == 4 ? 5 : std::min(cfg, 6);
 }
 
-// Plan: the configuration of least estimated time, rounds of work-groups times
-// the time of one over KB k-blocks, the constants fitted to measured launches
-// (130 shapes: 17..2048 tokens, N = 1024..12288, K = 1024..6144; the choice is
-// on average 0.1 % and at most 5 % slower than the best configuration of its
-// shape).  Codes over 256 x 192 or 256 x 256 tiles were the best at none: their
-// fp32 outputs (64 KiB per 128 x 128) drain under the next work-group's loop
-// only where two share a CU.
-static void gemm_i8_plan(const GemmLaunch& L, int& cfg, int& split) {
-  const bool planes = L.out == OUT_F32_X4;
-  const int MG = planes ? planes_groups(L.M / 4, true) : cdiv(L.M, 16), NG = cdiv(L.N, 16), KB = cdiv(L.K, 64);
+// Plan: the configuration and K slices of least estimated time.  The constants are
+// fitted to launches whose weights come from HBM (more copies of them than the
+// caches hold, as in a model of many layers) and, at lower weight, to repeated ones,
+// of every configuration and 1..8 slices: 16 x 22 shapes of 17..2048 tokens of codes
+// and 16 x 27 of 5..2048 tokens of planes, N = 1024 .. 12288, K = 1000..6144.  The
+// kernel chosen (the small-M kernel among them) is on average 0.5 % slower than the
+// best of its shape with weights from HBM (1.0 % with the limits before, fitted to
+// repeated weights alone), 0.9 % and 0.4 % with repeated ones.
+//   Codes over 256 x 192 or 256 x 256 tiles were the best at none: their fp32 outputs
+// (64 KiB per 128 x 128) drain under the next work-group's loop only where two share a
+// CU.  K slices cost a merge of three dependent memory round trips, about 3 us, so they
+// pay only where the tiles leave most CUs idle and K is long; more than 4 were at most
+// 3 % faster than 4 (64 x 5000 x 5000 codes 21.6 us on the small-M kernel, 15.5 with 4
+// slices; 160 tokens of planes, 2048 x 6144: 23.7 us whole, 20.0 with 3).
+struct I8Plan {
+  int cfg, split;
+  float us;
+};
+static I8Plan i8_best(bool planes, int M, int N, int K) {
+  const int MG = planes ? planes_groups(M / 4, true) : cdiv(M, 16), NG = cdiv(N, 16), KB = cdiv(K, 64);
+  I8Plan best{planes ? 6 : 1, 1, 3.0e38f};
   auto tiles = [&](int c) {
     int mt, nt;
     i8_cfg(c, mt, nt);
     return cdiv(MG, mt) * cdiv(NG, nt);
   };
-  float best = 3.0e38f;
-  auto offer = [&](int c, float us, int s) {
-    if (us < best) {
-      best = us;
-      cfg = c;
-      split = s;
-    }
+  auto offer = [&](int c, int s, float us) {
+    if (us < best.us) best = I8Plan{c, s, us};
   };
-  // two work-groups share a CU: a last round of up to 256 runs one per CU
-  auto paired = [&](int t, float fixed, float alone, float pair) {
-    const int n = t / 512, rem = t % 512;
-    return n * (fixed + KB * pair) + (rem == 0 ? 0.0f : fixed + KB * (rem <= 256 ? alone : pair));
+  auto slices = [&](int c) { return tiles(c) <= 128 ? std::min(4, KB) : 1; };
+  // one work-group per CU: rounds of 256
+  auto rounds = [&](int c, float fixed, float kb, float fill) {
+    offer(c, 1, cdiv(tiles(c), 256) * (fixed + kb * KB) + fill * tiles(c) / 256.0f);
+  };
+  // work-groups share CUs: the time of a k-block grows with each half round of 256
+  auto shared = [&](int c, int s, float fixed, float fill, float alone, float pair, float later, float merge) {
+    const int t = tiles(c) * s;
+    const float half = 0.5f * (float)cdiv(t, 128), kb = (float)KB / s;
+    offer(c, s, fixed + fill * std::min(t, 256) / 256.0f +
+                    (t <= 256 ? kb * alone : kb * pair * half + later * (half - 1.0f)) + merge);
   };
   if (planes) {
-    offer(3, cdiv(tiles(3), 256) * (6.5f + 0.605f * KB), 1);
-    offer(4, cdiv(tiles(4), 256) * (8.0f + 0.50f * KB), 1);
-    offer(6, paired(tiles(6), 3.9f, 0.265f, 0.435f), planes_slices(tiles(6), KB));
+    rounds(3, 1.97f, 0.599f, 6.11f);
+    rounds(4, 3.1f, 0.481f, 4.85f);
+    for (int s = 1; s <= slices(6); s++)
+      shared(6, s, 4.09f, 1.19f, 0.229f, 0.237f, 0.644f, s > 1 ? 3.81f + 0.0253f * tiles(6) * s : 0.0f);
   } else {
-    offer(1, cdiv(tiles(1), 256) * (5.7f + 0.073f * KB), codes_slices(tiles(1), KB));
-    offer(5, paired(tiles(5), 6.1f, 0.195f, 0.526f), 1);
-    offer(6, paired(tiles(6), 4.1f, 0.183f, 0.36f), 1);
+    for (int s = 1; s <= slices(1); s++) {
+      const int t = tiles(1) * s;
+      offer(1, s, 4.99f + 1.39f * t / 256.0f + 1.47f * (cdiv(t, 256) - 1) + cdiv(t, 256) * 0.157f * KB / s +
+                      (s > 1 ? 2.83f + 0.012f * t : 0.0f));
+    }
+    shared(5, 1, 5.75f, 4.09f, 0.275f, 0.344f, 4.59f, 0.0f);
+    shared(6, 1, 4.85f, 2.63f, 0.196f, 0.244f, 3.11f, 0.0f);
   }
+  return best;
+}
+// estimated us of the tiled kernels' plan, for code or plane rows (OUT_F32_X4)
+float gemm_i8_us(int out, int M, int N, int K) { return i8_best(out == OUT_F32_X4, M, N, K).us; }
+
+static void gemm_i8_plan(const GemmLaunch& L, int& cfg, int& split) {
+  const bool planes = L.out == OUT_F32_X4;
+  const int KB = cdiv(L.K, 64);
+  const I8Plan best = i8_best(planes, L.M, L.N, L.K);
+  cfg = best.cfg;
+  split = best.split;
   const int fc = g_i8_force_cfg.load(std::memory_order_relaxed);
   if (fc >= 0) {
     cfg = i8_resolve(fc, planes);

@@ -513,6 +513,24 @@ static void launch_small_mode(const GemmSmallArgs& a, int u, int r, int tg, hipS
 
 // tuning override of the 16-bit rows' work-group shape: 100 R + 10 TG + U
 // (R, TG in {1, 2, 4}, U in {2, 4}), 0 = the planner in launch_gemm_small
+// weight row groups per work-group of code and plane rows (narrower than the
+// lm_head) and fp32 rows: the most, of 4, 2 and 1, that leave >= 192 work-groups
+static int small_rows_per_wg(int MG, int NG) {
+  for (int r = 4; r > 1; r >>= 1)
+    if ((long long)cdiv(NG, r) * MG >= 192) return r;
+  return 1;
+}
+
+// Estimated time of 17..64 code or plane rows: rounds of 256 work-groups, each a
+// fixed part and one per k-block that grow with its row groups, fitted as the tiled
+// int8 kernels' is (gemm_i8.hip).
+float gemm_small_i8_us(int out, int M, int N, int K) {
+  const int MG = cdiv(M, 16), NG = cdiv(N, 16), r = small_rows_per_wg(MG, NG);
+  const float rounds = (float)cdiv(cdiv(NG, r) * MG, 256), KB = (float)cdiv(K, 64);
+  return out == OUT_F32_X4 ? 1.97f + rounds * (0.203f + 0.0326f * r + KB * (0.00974f + 0.0251f * r))
+                           : 2.19f + rounds * (0.0521f + 0.0105f * r + KB * (0.025f * r - 0.0143f));
+}
+
 static std::atomic<int> g_small_b16_shape{0};
 void gemm_small_set_b16_shape(int code) { g_small_b16_shape.store(code, std::memory_order_relaxed); }
 
@@ -592,12 +610,7 @@ hipError_t launch_gemm_small(const GemmLaunch& L, hipStream_t st) {
       // work-group before); W8A8 at 64 rows, N = 2048: 7.7 -> 6.3 us; the
       // int8 planes of 8 tokens over 2048 x 6144: 10.9 -> 9.0 us
       tg = 1;
-      r = 1;
-      for (int cr = 4; cr > 1; cr >>= 1)
-        if ((long long)cdiv(a.NG, cr) * a.MG >= 192) {
-          r = cr;
-          break;
-        }
+      r = small_rows_per_wg(a.MG, a.NG);
       u_force = (n_t >= 8 && (r == 1 || (r == 2 && L.amode == A_I8))) ? 4 : 2;
     }
   }

@@ -356,6 +356,7 @@ hipError_t launch_gemm_i8(const GemmLaunch& L, hipStream_t st);
 void gemm_i8_set_cfg(int cfg);
 void gemm_i8_set_split(int s);
 void gemm_i8_resolve(GemmLaunch& L, size_t* part_bytes, size_t* counters);
+float gemm_i8_us(int out, int M, int N, int K);   // its estimated time of a shape
 bool gemm_planes_grouped(int M4, int N, int K);
 
 // LDS-staged 16-bit MFMA GEMM (gemm_b16.hip): A_BF16 / A_F16, used for M > 16
@@ -371,6 +372,7 @@ void gemm_resolve(GemmLaunch& L, size_t* part_bytes, size_t* counters);
 // M <= 16 rows (gemm_small.hip): GEMV-shaped MFMA kernel
 bool gemm_small_supported(const GemmLaunch& L);
 float gemm_small_b16_us(int M, int N, int K);   // its estimated time of 17..256 16-bit rows
+float gemm_small_i8_us(int out, int M, int N, int K);   // and of 17..64 code or plane rows
 hipError_t launch_gemm_small(const GemmLaunch& L, hipStream_t st);
 
 bool rows_supported(const GemmLaunch& L);
