@@ -64,13 +64,15 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restri
 // the arithmetic of quantize_rows_tiled_vec_kernel (quant.hip) on the same
 // values, so the codes equal those of quantizing the stored row afterwards.
 //
-// PLANES: instead, the four int8 planes of the row as code rows
+// ROW_PLANES, ROW_GROUPED: instead, the four int8 planes of the row as code rows
 // planes_row(row, p, grouped) and its exponent in `xe` (split_i8x4_kernel's
-// arithmetic, quant.hip), the activations of the fp32-semantics GEMM.
-template <int NV, bool PLANES>
+// arithmetic, quant.hip), the activations of the fp32-semantics GEMM.  The layout is
+// a template argument, so that the four stores of a float4 share one address.
+enum { ROW_CODES, ROW_PLANES, ROW_GROUPED };
+template <int NV, int MODE>
 __device__ __forceinline__ void quantize_row_to_tiles(const float4 (&v)[NV], int n4, int row, int MG,
                                                       uint8_t* __restrict__ tiles, float* __restrict__ scales,
-                                                      int* __restrict__ xe, uint32_t* s_mx, bool grouped) {
+                                                      int* __restrict__ xe, uint32_t* s_mx) {
   const int tid = threadIdx.x;
   uint32_t mx = 0;
 #pragma unroll
@@ -81,7 +83,7 @@ __device__ __forceinline__ void quantize_row_to_tiles(const float4 (&v)[NV], int
   if ((tid & 63) == 0) s_mx[tid >> 6] = mx;
   __syncthreads();
   mx = max(max(s_mx[0], s_mx[1]), max(s_mx[2], s_mx[3]));
-  if constexpr (PLANES) {
+  if constexpr (MODE != ROW_CODES) {
     const int ee = planes_exponent(mx);
     const bool finite = ee != kXeNonFinite;
     const int e = finite ? ee : 0;
@@ -96,7 +98,7 @@ __device__ __forceinline__ void quantize_row_to_tiles(const float4 (&v)[NV], int
       planes4_i8(w4, e, code);
 #pragma unroll
       for (int p = 0; p < 4; p++) {
-        const int rr = planes_row(row, p, grouped);
+        const int rr = planes_row(row, p, MODE == ROW_GROUPED);
         t32[(((size_t)(f >> 4) * MG + (rr >> 4)) * 64 + (rr & 15) + 16 * ((f >> 2) & 3)) * 4 + (f & 3)] = code[p];
       }
     }
@@ -122,11 +124,11 @@ __device__ __forceinline__ void quantize_row_to_tiles(const float4 (&v)[NV], int
 // output, one work-group per token: the normalised values of
 // rmsnorm_rows_kernel, quantized in registers and written as int8 tiles and
 // scales (the fp32 row is never stored; K % 64 == 0, K <= 2048).
-template <bool PLANES>
+template <int MODE>
 __global__ __launch_bounds__(256) void rmsnorm_rows_q_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                              int rows, int K, float eps, int MG,
                                                              uint8_t* __restrict__ tiles, float* __restrict__ scales,
-                                                             int* __restrict__ xe, bool grouped) {
+                                                             int* __restrict__ xe) {
   __shared__ float s_part[4];
   __shared__ uint32_t s_mx[4];
   const int rr = xcd_grouped_row(blockIdx.x);
@@ -158,20 +160,19 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_q_kernel(const float* __rest
   for (int i = 0; i < 2; i++)
     y[i] = make_float4(__fmul_rn(__fmul_rn(v[i].x, r), wv[i].x), __fmul_rn(__fmul_rn(v[i].y, r), wv[i].y),
                        __fmul_rn(__fmul_rn(v[i].z, r), wv[i].z), __fmul_rn(__fmul_rn(v[i].w, r), wv[i].w));
-  quantize_row_to_tiles<2, PLANES>(y, n4, (int)row, MG, tiles, scales, xe, s_mx, grouped);
+  quantize_row_to_tiles<2, MODE>(y, n4, (int)row, MG, tiles, scales, xe, s_mx);
 }
 
 // fp32 token rows -> their four int8 planes and exponents (split_i8x4_kernel's
 // result, quant.hip), one work-group per row: the row is loaded once into
 // registers (float4 tid + 256 j) and quantize_row_to_tiles writes the planes,
 // where split_i8x4_kernel makes one wave walk the row twice.  K = 1024 NV.
-// PLANES false: the W8A8 per-token codes and scales instead
+// ROW_CODES: the W8A8 per-token codes and scales instead
 // (quantize_rows_tiled's result).
-template <int NV, bool PLANES>
+template <int NV, int MODE>
 __global__ __launch_bounds__(256) void split_rows_planes_kernel(const float* __restrict__ x, int ldx, int rows,
                                                                 int MG, uint8_t* __restrict__ tiles,
-                                                                float* __restrict__ scales, int* __restrict__ xe,
-                                                                bool grouped) {
+                                                                float* __restrict__ scales, int* __restrict__ xe) {
   __shared__ uint32_t s_mx[4];
   const int rr = xcd_grouped_row(blockIdx.x);
   if (rr >= rows) return;                   // the whole work-group
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(256) void split_rows_planes_kernel(const float* __r
   float4 v[NV];
 #pragma unroll
   for (int j = 0; j < NV; j++) v[j] = xr[threadIdx.x + 256 * j];
-  quantize_row_to_tiles<NV, PLANES>(v, 256 * NV, rr, MG, tiles, scales, xe, s_mx, grouped);
+  quantize_row_to_tiles<NV, MODE>(v, 256 * NV, rr, MG, tiles, scales, xe, s_mx);
 }
 
 // SwiGLU of one token's interleaved gate/up row (the values of
@@ -189,10 +190,10 @@ __global__ __launch_bounds__(256) void split_rows_planes_kernel(const float* __r
 // is computed in two halves: holding a whole 6144-wide row's loads and values
 // in registers took 127 VGPRs, 4 work-groups per CU, and a 1200-token batch
 // then ran in two rounds; at 24 KB of LDS per work-group all 1200 are resident.
-template <int NV, bool PLANES>
+template <int NV, int MODE>
 __global__ __launch_bounds__(256) void swiglu_rows_q_kernel(const float* __restrict__ gu, int S, int ffn, int MG,
                                                             uint8_t* __restrict__ tiles, float* __restrict__ scales,
-                                                            int* __restrict__ xe, bool grouped) {
+                                                            int* __restrict__ xe) {
   __shared__ uint32_t s_mx[4];
   __shared__ float4 s_y[NV][256];
   const int tt = xcd_grouped_row(blockIdx.x);
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(256) void swiglu_rows_q_kernel(const float* __restr
   float4 y[NV];
 #pragma unroll
   for (int j = 0; j < NV; j++) y[j] = s_y[j][threadIdx.x];
-  quantize_row_to_tiles<NV, PLANES>(y, ffn >> 2, (int)t, MG, tiles, scales, xe, s_mx, grouped);
+  quantize_row_to_tiles<NV, MODE>(y, ffn >> 2, (int)t, MG, tiles, scales, xe, s_mx);
 }
 
 // One wave per 128-wide head vector of a token: the token's nq = 2 nkv q
@@ -631,43 +632,56 @@ hipError_t launch_rmsnorm_rows(const float* x, const float* w, float* out, int r
   return hipGetLastError();
 }
 
+// f(MODE) with the row quantizers' output as a constant
+template <class F>
+static void row_mode(bool planes, bool grouped, F f) {
+  if (!planes) f([]() constexpr { return (int)ROW_CODES; });
+  else if (grouped) f([]() constexpr { return (int)ROW_GROUPED; });
+  else f([]() constexpr { return (int)ROW_PLANES; });
+}
+
 hipError_t launch_rmsnorm_rows_q(const float* x, const float* w, uint8_t* tiles, float* scales, int* xe, int rows,
                                  int K, float eps, bool grouped, hipStream_t st) {
   if (K % 64 != 0 || K > 2048 || rows < 1 || (!scales == !xe)) return hipErrorInvalidValue;
   const dim3 grid(cdiv(rows, 64) * 64);     // xcd_grouped_row: whole groups of 64 rows
-  if (xe)
-    hipLaunchKernelGGL(rmsnorm_rows_q_kernel<true>, grid, dim3(256), 0, st, x, w, rows, K, eps,
-                       planes_groups(rows, grouped), tiles, scales, xe, grouped);
-  else
-    hipLaunchKernelGGL(rmsnorm_rows_q_kernel<false>, grid, dim3(256), 0, st, x, w, rows, K, eps, cdiv(rows, 16),
-                       tiles, scales, xe, false);
+  const int MG = xe ? planes_groups(rows, grouped) : cdiv(rows, 16);
+  row_mode(xe != nullptr, grouped, [&](auto mode) {
+    hipLaunchKernelGGL(rmsnorm_rows_q_kernel<mode()>, grid, dim3(256), 0, st, x, w, rows, K, eps, MG, tiles, scales, xe);
+  });
   return hipGetLastError();
 }
 
-template <bool PLANES>
+template <int NV, int MODE>
+static void launch_rows_nv(const float* x, int ldx, int rows, int MG, uint8_t* tiles, float* scales, int* xe,
+                           hipStream_t st) {
+  const dim3 grid(cdiv(rows, 64) * 64);     // xcd_grouped_row: whole groups of 64 rows
+  hipLaunchKernelGGL((split_rows_planes_kernel<NV, MODE>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe);
+}
 static hipError_t launch_rows_q(const float* x, int ldx, int rows, int K, uint8_t* tiles, float* scales, int* xe,
                                 bool grouped, hipStream_t st) {
   if (rows < 1 || ldx < K || ldx % 4 != 0 || (((uintptr_t)x) & 15) != 0) return hipErrorInvalidValue;
-  const dim3 grid(cdiv(rows, 64) * 64);     // xcd_grouped_row: whole groups of 64 rows
-  const int MG = PLANES ? planes_groups(rows, grouped) : cdiv(rows, 16);
-  switch (K) {
-    case 1024: hipLaunchKernelGGL((split_rows_planes_kernel<1, PLANES>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe, grouped); break;
-    case 2048: hipLaunchKernelGGL((split_rows_planes_kernel<2, PLANES>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe, grouped); break;
-    case 4096: hipLaunchKernelGGL((split_rows_planes_kernel<4, PLANES>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe, grouped); break;
-    case 6144: hipLaunchKernelGGL((split_rows_planes_kernel<6, PLANES>), grid, dim3(256), 0, st, x, ldx, rows, MG, tiles, scales, xe, grouped); break;
-    default: return hipErrorInvalidValue;
-  }
+  if (K != 1024 && K != 2048 && K != 4096 && K != 6144) return hipErrorInvalidValue;
+  const int MG = xe ? planes_groups(rows, grouped) : cdiv(rows, 16);
+  row_mode(xe != nullptr, grouped, [&](auto mode) {
+    switch (K) {
+      case 1024: launch_rows_nv<1, mode()>(x, ldx, rows, MG, tiles, scales, xe, st); break;
+      case 2048: launch_rows_nv<2, mode()>(x, ldx, rows, MG, tiles, scales, xe, st); break;
+      case 4096: launch_rows_nv<4, mode()>(x, ldx, rows, MG, tiles, scales, xe, st); break;
+      default: launch_rows_nv<6, mode()>(x, ldx, rows, MG, tiles, scales, xe, st); break;
+    }
+  });
   return hipGetLastError();
 }
 
 hipError_t launch_split_rows_planes(const float* x, int ldx, int rows, int K, uint8_t* tiles, int* xe,
                                     bool grouped, hipStream_t st) {
-  return launch_rows_q<true>(x, ldx, rows, K, tiles, nullptr, xe, grouped, st);
+  if (!xe) return hipErrorInvalidValue;
+  return launch_rows_q(x, ldx, rows, K, tiles, nullptr, xe, grouped, st);
 }
 
 hipError_t launch_quantize_rows_by_row(const float* x, int rows, int K, uint8_t* tiles, float* scales,
                                        hipStream_t st) {
-  return launch_rows_q<false>(x, K, rows, K, tiles, scales, nullptr, false, st);
+  return launch_rows_q(x, K, rows, K, tiles, scales, nullptr, false, st);
 }
 
 hipError_t launch_swiglu_rows_q(const float* gu, uint8_t* tiles, float* scales, int* xe, int S, int ffn,
@@ -675,16 +689,13 @@ hipError_t launch_swiglu_rows_q(const float* gu, uint8_t* tiles, float* scales, 
   if (S < 1 || (!scales == !xe)) return hipErrorInvalidValue;
   const int MG = xe ? planes_groups(S, grouped) : cdiv(S, 16);
   const dim3 grid(cdiv(S, 64) * 64);        // xcd_grouped_row: whole groups of 64 rows
-  if (ffn == 6144 && xe)
-    hipLaunchKernelGGL((swiglu_rows_q_kernel<6, true>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe, grouped);
-  else if (ffn == 6144)
-    hipLaunchKernelGGL((swiglu_rows_q_kernel<6, false>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe, grouped);
-  else if (ffn == 2048 && xe)
-    hipLaunchKernelGGL((swiglu_rows_q_kernel<2, true>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe, grouped);
-  else if (ffn == 2048)
-    hipLaunchKernelGGL((swiglu_rows_q_kernel<2, false>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe, grouped);
-  else
-    return hipErrorInvalidValue;
+  if (ffn != 6144 && ffn != 2048) return hipErrorInvalidValue;
+  row_mode(xe != nullptr, grouped, [&](auto mode) {
+    if (ffn == 6144)
+      hipLaunchKernelGGL((swiglu_rows_q_kernel<6, mode()>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe);
+    else
+      hipLaunchKernelGGL((swiglu_rows_q_kernel<2, mode()>), grid, dim3(256), 0, st, gu, S, ffn, MG, tiles, scales, xe);
+  });
   return hipGetLastError();
 }
 
