@@ -38,7 +38,7 @@ def test_w8a32_planes_configs(lin, orc, T, N, K):
     xd, bd = torch.from_numpy(x).cuda(), torch.from_numpy(b).cuda()
     first = None
     try:
-        for cfg, split in [(-1, 0), (3, 0), (4, 0), (6, 0), (6, 2), (6, 3), (6, 4), (-1, 8)]:
+        for cfg, split in [(-1, 0), (3, 0), (4, 0), (6, 0), (6, 2), (6, 3), (6, 4), (7, 0), (7, 3), (-1, 8)]:
             say(f"  cfg={cfg} split={split}")
             assert lib.tl_gemm_i8_set_cfg(cfg) == 0 and lib.tl_gemm_i8_set_split(split) == 0
             y = torch.full((T, N), 7.0, device="cuda")

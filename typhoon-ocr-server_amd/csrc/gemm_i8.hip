@@ -94,10 +94,10 @@ __device__ __forceinline__ void tile_of(int b, int ntm, int ntn, int& tm, int& t
 // sums, so any order gives the same bits; slice order here) and returns true.
 // flag: a word of the stage ring, which no copy or read uses any more (an LDS
 // word of its own would push the 80 KiB rings past two work-groups per CU).
-template <int FM, int FN>
+template <int NW, int FM, int FN>
 __device__ __forceinline__ bool merge_slices(const GemmI8Args& a, v4i (&acc)[FM][FN], int wv, int lane, int bt, int ks,
                                              int* flag) {
-  constexpr int TF = 4 * FM * FN * 256;
+  constexpr int TF = NW * FM * FN * 256;        // sums per partial tile
   int32_t* mine = a.part + ((size_t)bt * a.S + ks) * TF;
 #pragma unroll
   for (int i = 0; i < FM; i++)
@@ -325,7 +325,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_lds_kernel(GemmI8Args a)
 
   wait_vm<0>();   // no copy may still be landing in LDS when the work-group exits
 
-  if (a.S > 1 && !merge_slices<FM, FN>(a, acc, wv, lane, bt, ks, reinterpret_cast<int*>(s0))) return;
+  if (a.S > 1 && !merge_slices<NW, FM, FN>(a, acc, wv, lane, bt, ks, reinterpret_cast<int*>(s0))) return;
 
   // epilogue: y = fl(fl(fl(acc) * ws[n]) * xs[m]) (+ bias[n]); 16-byte
   // streaming stores when the 4 columns are inside N and the row is 16-byte
@@ -378,7 +378,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_lds_kernel(GemmI8Args a)
 // fed through each other's reads, copies and barriers (one wave issues an
 // instruction every 8-9 cycles, two every 5): 8 waves on 256 x 256 tiles (4 waves
 // of twice the block, in 512 registers: 116 -> 109 us at 1200 tokens of planes
-// over N = 12288, K = 2048), two work-groups per CU on 128-row ones.  256 x 192
+// over N = 12288, K = 2048), two work-groups per CU on 128-row ones.  Few tokens of
+// planes leave CUs without a 128-row tile: 64 x 128 ones, of 2 waves, are two and more
+// work-groups where those are one (32 tokens, weights from HBM: N = 12288, K = 2048
+// 12.8 -> 10.7 us, N = 2048, K = 6144 in 4 slices 15.6 -> 13.4).  256 x 192
 // tiles keep 4 waves (8 waves: 54 -> 57 us at N = 2048, K = 6144).  Against the
 // kernels before it (64 x 128 tiles with weights straight to registers): 2048
 // tokens of planes over N = 12288, K = 2048 (split included) 313 -> 173 us (2.4
@@ -405,7 +408,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_lds_kernel(GemmI8Args a)
 // about ten moves per 96 MFMAs, where with accumulators in those it made 320.
 enum { QUAD_F32, QUAD_PLANES, QUAD_I32 };   // outputs: scaled codes, folded planes, the sums
 template <int WM, int FM, int FN, int NST, int MODE>
-__global__ __launch_bounds__(128 * WM, FM == 8 ? 1 : 2) void gemm_i8_quad_kernel(GemmI8Args a) {
+__global__ __launch_bounds__(128 * WM, FM == 8 || WM == 1 ? 1 : 2) void gemm_i8_quad_kernel(GemmI8Args a) {
   constexpr int NW = 2 * WM;                              // waves: WM x 2
   constexpr int MT = WM * FM, NT = 2 * FN, TS = MT + NT;  // row groups, column groups, tiles per stage
   constexpr int PA = MT / NW, PW = (TS + NW - 1) / NW;    // copies per wave per stage (PA of them activations)
@@ -514,7 +517,7 @@ __global__ __launch_bounds__(128 * WM, FM == 8 ? 1 : 2) void gemm_i8_quad_kernel
   if (st < KB) step(st, 0);
   wait_vm<0>();   // no copy may still be landing in LDS when the work-group exits
   if constexpr (SLICES) {
-    if (a.S > 1 && !merge_slices<FM, FN>(a, acc, wv, lane, bt, ks, reinterpret_cast<int*>(sS))) return;
+    if (a.S > 1 && !merge_slices<NW, FM, FN>(a, acc, wv, lane, bt, ks, reinterpret_cast<int*>(sS))) return;
   }
 
   // Epilogue.  Every operand is loaded before the first store: memory
@@ -622,9 +625,9 @@ __global__ __launch_bounds__(128 * WM, FM == 8 ? 1 : 2) void gemm_i8_quad_kernel
 // cfg 0..2: LDS-staged kernel, 128 x 192, 64 x 128, 128 x 128 tiles (4, 8, 8
 //   stage buffers); cfg 1 is the planner's for small tile counts, 0 and 2 run
 //   only when forced
-// cfg 3..6: quadrant kernel, 256 x 256, 256 x 192, 128 x 192, 128 x 128 tiles
+// cfg 3..7: quadrant kernel, 256 x 256, 256 x 192, 128 x 192, 128 x 128, 64 x 128 tiles
 static void i8_cfg(int cfg, int& mt, int& nt) {
-  static const int dims[7][2] = {{8, 12}, {4, 8}, {8, 8}, {16, 16}, {16, 12}, {8, 12}, {8, 8}};
+  static const int dims[8][2] = {{8, 12}, {4, 8}, {8, 8}, {16, 16}, {16, 12}, {8, 12}, {8, 8}, {4, 8}};
   mt = dims[cfg][0];
   nt = dims[cfg][1];
 }
@@ -636,9 +639,9 @@ void gemm_i8_set_cfg(int cfg) { g_i8_force_cfg.store(cfg, std::memory_order_rela
 void gemm_i8_set_split(int s) { g_i8_force_split.store(s > 0 ? s : 0, std::memory_order_relaxed); }
 
 // the configuration that runs where `cfg` is forced: planes have no 128 x 192
-// tiles and only quadrant ones, codes no 256-row ones (7 is 128 x 128 too)
+// tiles and only quadrant ones, codes no 256-row ones and their 64 x 128 LDS-staged
 static int i8_resolve(int cfg, bool planes) {
-  if (planes) return cfg == 3 || cfg == 4 ? cfg : 6;
+  if (planes) return cfg == 3 || cfg == 4 || cfg == 7 ? cfg : 6;
   return cfg == 3 || cfg == 4 ? 5 : std::min(cfg, 6);
 }
 
@@ -647,15 +650,15 @@ static int i8_resolve(int cfg, bool planes) {
 // caches hold, as in a model of many layers) and, at lower weight, to repeated ones,
 // of every configuration and 1..8 slices: 16 x 22 shapes of 17..2048 tokens of codes
 // and 16 x 27 of 5..2048 tokens of planes, N = 1024 .. 12288, K = 1000..6144.  The
-// kernel chosen (the small-M kernel among them) is on average 0.5 % slower than the
-// best of its shape with weights from HBM (1.0 % with the limits before, fitted to
-// repeated weights alone), 0.9 % and 0.4 % with repeated ones.
+// kernel chosen (the small-M kernel among them) is on average 0.5 % (codes) and 0.3 %
+// (planes) slower than the best of its shape with weights from HBM (1.0 % with limits
+// fitted to repeated weights alone), 0.9 % and 0.5 % with repeated ones.
 //   Codes over 256 x 192 or 256 x 256 tiles were the best at none: their fp32 outputs
 // (64 KiB per 128 x 128) drain under the next work-group's loop only where two share a
 // CU.  K slices cost a merge of three dependent memory round trips, about 3 us, so they
 // pay only where the tiles leave most CUs idle and K is long; more than 4 were at most
 // 3 % faster than 4 (64 x 5000 x 5000 codes 21.6 us on the small-M kernel, 15.5 with 4
-// slices; 160 tokens of planes, 2048 x 6144: 23.7 us whole, 20.0 with 3).
+// slices; 32 tokens of planes, 2048 x 6144: 22.2 us whole, 13.4 with 4).
 struct I8Plan {
   int cfg, split;
   float us;
@@ -684,10 +687,12 @@ static I8Plan i8_best(bool planes, int M, int N, int K) {
                     (t <= 256 ? kb * alone : kb * pair * half + later * (half - 1.0f)) + merge);
   };
   if (planes) {
-    rounds(3, 1.97f, 0.599f, 6.11f);
-    rounds(4, 3.1f, 0.481f, 4.85f);
+    rounds(3, 1.26f, 0.601f, 8.5f);
+    rounds(4, 2.95f, 0.478f, 5.01f);
     for (int s = 1; s <= slices(6); s++)
-      shared(6, s, 4.09f, 1.19f, 0.229f, 0.237f, 0.644f, s > 1 ? 3.81f + 0.0253f * tiles(6) * s : 0.0f);
+      shared(6, s, 3.8f, 1.28f, 0.207f, 0.239f, 0.65f, s > 1 ? 4.23f + 0.0178f * tiles(6) * s : 0.0f);
+    for (int s = 1; s <= slices(7); s++)
+      shared(7, s, 4.05f, 0.372f, 0.175f, 0.149f, 0.592f, s > 1 ? 2.62f + 0.0123f * tiles(7) * s : 0.0f);
   } else {
     for (int s = 1; s <= slices(1); s++) {
       const int t = tiles(1) * s;
@@ -716,7 +721,7 @@ static void gemm_i8_plan(const GemmLaunch& L, int& cfg, int& split) {
   const int fs = g_i8_force_split.load(std::memory_order_relaxed);
   if (fs > 0) {
     split = std::min(fs, KB);
-    if (split > 1 && cfg >= 3) cfg = planes ? 6 : 1;   // the kernels that take slices
+    if (split > 1 && cfg >= 3 && !(planes && cfg == 7)) cfg = planes ? 6 : 1;   // the kernels that take slices
   }
 }
 
@@ -730,8 +735,8 @@ void gemm_i8_resolve(GemmLaunch& L, size_t* part_bytes, size_t* counters) {
   *counters = L.split > 1 ? tiles : 0;
 }
 
-// planes on 256 x 256, 256 x 192 and 128 x 128 tiles, codes on 128 x 192 and
-// 128 x 128 (i8_resolve)
+// planes on 256 x 256, 256 x 192, 128 x 128 and 64 x 128 tiles, codes on 128 x 192
+// and 128 x 128 (i8_resolve)
 template <int WM, int FM, int FN, int NST>
 static void launch_quad(const GemmI8Args& a, int blocks, hipStream_t st) {
   const dim3 grid(blocks), block(128 * WM);
@@ -797,6 +802,7 @@ hipError_t launch_gemm_i8(const GemmLaunch& L, hipStream_t st) {
     case 3: launch_quad<4, 4, 8, 5>(a, blocks, st); break;
     case 4: launch_quad<2, 8, 6, 5>(a, blocks, st); break;
     case 5: launch_quad<2, 4, 6, 4>(a, blocks, st); break;
+    case 7: launch_quad<1, 4, 4, 5>(a, blocks, st); break;
     default: launch_quad<2, 4, 4, 5>(a, blocks, st); break;
   }
   return hipGetLastError();

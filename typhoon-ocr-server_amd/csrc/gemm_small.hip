@@ -511,8 +511,6 @@ static void launch_small_mode(const GemmSmallArgs& a, int u, int r, int tg, hipS
   else launch_small_r<AMODE, 1>(a, u, tg, st);
 }
 
-// tuning override of the 16-bit rows' work-group shape: 100 R + 10 TG + U
-// (R, TG in {1, 2, 4}, U in {2, 4}), 0 = the planner in launch_gemm_small
 // weight row groups per work-group of code and plane rows (narrower than the
 // lm_head) and fp32 rows: the most, of 4, 2 and 1, that leave >= 192 work-groups
 static int small_rows_per_wg(int MG, int NG) {
@@ -521,16 +519,21 @@ static int small_rows_per_wg(int MG, int NG) {
   return 1;
 }
 
-// Estimated time of 17..64 code or plane rows: rounds of 256 work-groups, each a
+// Estimated us of 17..64 code or plane rows: rounds of 256 work-groups, each a
 // fixed part and one per k-block that grow with its row groups, fitted as the tiled
-// int8 kernels' is (gemm_i8.hip).
+// int8 kernels' is (i8_best, gemm_i8.hip).
 float gemm_small_i8_us(int out, int M, int N, int K) {
-  const int MG = cdiv(M, 16), NG = cdiv(N, 16), r = small_rows_per_wg(MG, NG);
-  const float rounds = (float)cdiv(cdiv(NG, r) * MG, 256), KB = (float)cdiv(K, 64);
-  return out == OUT_F32_X4 ? 1.97f + rounds * (0.203f + 0.0326f * r + KB * (0.00974f + 0.0251f * r))
-                           : 2.19f + rounds * (0.0521f + 0.0105f * r + KB * (0.025f * r - 0.0143f));
+  const int MG = cdiv(M, 16), NG = cdiv(N, 16), r = small_rows_per_wg(MG, NG), wgs = cdiv(NG, r) * MG;
+  const float rounds = (float)cdiv(wgs, 256), KB = (float)cdiv(K, 64);
+  if (out == OUT_F32_X4) {
+    const float rd = 0.932f * rounds + 0.068f * std::max(1.0f, wgs / 256.0f);
+    return 1.85f + rd * (0.215f + 0.0492f * r + KB * (0.0308f + 0.0203f * r));
+  }
+  return 2.19f + rounds * (0.0521f + 0.0105f * r + KB * (0.025f * r - 0.0143f));
 }
 
+// tuning override of the 16-bit rows' work-group shape: 100 R + 10 TG + U
+// (R, TG in {1, 2, 4}, U in {2, 4}), 0 = the planner in launch_gemm_small
 static std::atomic<int> g_small_b16_shape{0};
 void gemm_small_set_b16_shape(int code) { g_small_b16_shape.store(code, std::memory_order_relaxed); }
 
