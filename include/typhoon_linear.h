@@ -105,16 +105,16 @@ int tl_gemv_set_plan(int rows, int u);
 
 /* Tuning override of the int8 MFMA GEMM (W8A8 at M > 16 and the int8 planes of
  * W8A32 batches) for every later call in the process: -1 restores the
- * planner; 0..2 the LDS-staged kernel (tiles 128x192, 64x128, 128x128), 3..7
- * the quadrant kernel (tiles 256x256, 256x192, 128x192, 128x128, 64x128).
- * Planes run on 3, 4, 6 and 7 (6 for the others), codes on 0..2, 5 and 6 (5
- * for 3 and 4, 6 for 7). */
+ * planner; 1 the LDS-staged kernel (tiles 64x128, codes only); 3..7 the quadrant
+ * kernel (tiles 256x256, 256x192, 128x192, 128x128, 64x128).  Codes run on 1, 5 and
+ * 6, planes on 3, 4, 6 and 7; the others of 0..7 run the nearest of those tiles. */
 int tl_gemm_i8_set_cfg(int cfg);
 
 /* Tuning override of the same GEMM's K slices for every later call in the
- * process: 0 restores the planner (slices where a shape has fewer than 128
+ * process: 0 restores the planner (up to 4 slices where a shape has at most 128
  * tiles), 1..64 force that many work-groups per tile (codes on the LDS-staged
- * kernel, planes on the quadrant kernel's 128x128 or, with cfg 7, 64x128 tiles), whose exact int32 partial sums the last to arrive adds. */
+ * kernel, planes on the quadrant kernel's 128x128 or, with cfg 7, 64x128 tiles),
+ * whose exact int32 partial sums the last to arrive adds. */
 int tl_gemm_i8_set_split(int split);
 
 /* Tuning override of the 16-bit MFMA GEMM (W8A16, M > 16 on the tiled

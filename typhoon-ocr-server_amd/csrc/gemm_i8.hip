@@ -622,12 +622,10 @@ __global__ __launch_bounds__(128 * WM, FM == 8 || WM == 1 ? 1 : 2) void gemm_i8_
 // ---------------------------------------------------------------------------
 // planning and launch
 // ---------------------------------------------------------------------------
-// cfg 0..2: LDS-staged kernel, 128 x 192, 64 x 128, 128 x 128 tiles (4, 8, 8
-//   stage buffers); cfg 1 is the planner's for small tile counts, 0 and 2 run
-//   only when forced
+// cfg 1: LDS-staged kernel, 64 x 128 tiles (8 stage buffers), of codes only
 // cfg 3..7: quadrant kernel, 256 x 256, 256 x 192, 128 x 192, 128 x 128, 64 x 128 tiles
 static void i8_cfg(int cfg, int& mt, int& nt) {
-  static const int dims[8][2] = {{8, 12}, {4, 8}, {8, 8}, {16, 16}, {16, 12}, {8, 12}, {8, 8}, {4, 8}};
+  static const int dims[8][2] = {{0, 0}, {4, 8}, {0, 0}, {16, 16}, {16, 12}, {8, 12}, {8, 8}, {4, 8}};
   mt = dims[cfg][0];
   nt = dims[cfg][1];
 }
@@ -638,11 +636,11 @@ static std::atomic<int> g_i8_force_split{0};
 void gemm_i8_set_cfg(int cfg) { g_i8_force_cfg.store(cfg, std::memory_order_relaxed); }
 void gemm_i8_set_split(int s) { g_i8_force_split.store(s > 0 ? s : 0, std::memory_order_relaxed); }
 
-// the configuration that runs where `cfg` is forced: planes have no 128 x 192
-// tiles and only quadrant ones, codes no 256-row ones and their 64 x 128 LDS-staged
+// the configuration that runs where `cfg` (0..7) is forced: planes have quadrant tiles
+// other than 128 x 192, codes the LDS-staged 64 x 128 ones and quadrant tiles of 128 rows
 static int i8_resolve(int cfg, bool planes) {
-  if (planes) return cfg == 3 || cfg == 4 || cfg == 7 ? cfg : 6;
-  return cfg == 3 || cfg == 4 ? 5 : std::min(cfg, 6);
+  static const int of_planes[8] = {6, 6, 6, 3, 4, 6, 6, 7}, of_codes[8] = {5, 1, 6, 5, 5, 5, 6, 6};
+  return planes ? of_planes[cfg] : of_codes[cfg];
 }
 
 // Plan: the configuration and K slices of least estimated time.  The constants are
@@ -796,9 +794,7 @@ hipError_t launch_gemm_i8(const GemmLaunch& L, hipStream_t st) {
   if (blocks_ll > 0x7fffffffLL) return hipErrorInvalidValue;
   const int blocks = (int)blocks_ll;
   switch (L.cfg) {
-    case 0: hipLaunchKernelGGL((gemm_i8_lds_kernel<8, 12, 1, 4, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;
     case 1: hipLaunchKernelGGL((gemm_i8_lds_kernel<4, 8, 1, 8, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;
-    case 2: hipLaunchKernelGGL((gemm_i8_lds_kernel<8, 8, 1, 8, 2, 2>), dim3(blocks), dim3(256), 0, st, a); break;
     case 3: launch_quad<4, 4, 8, 5>(a, blocks, st); break;
     case 4: launch_quad<2, 8, 6, 5>(a, blocks, st); break;
     case 5: launch_quad<2, 4, 6, 4>(a, blocks, st); break;
