@@ -72,3 +72,15 @@ def test_bad_arguments_report_errors_without_gpu(lin):
                      None, lin._p(y, ctypes.c_float), None, 0, 16, 16)
     msg = lib.tl_last_error()
     assert msg is not None and b"batch" in msg
+
+
+def test_current_stream_without_the_raw_accessor(lin, monkeypatch):
+    """The raw handle of the current stream comes from an accessor of torch that is
+    not public; a torch without it still gives the handle of the Stream object."""
+    import torch
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: type("S", (), {"cuda_stream": 77})())
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda d: 40 + d, raising=False)
+    assert lin._stream(None) == 43
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    assert lin._stream(None) == 77

@@ -220,10 +220,14 @@ def _stream(stream) -> Optional[int]:
 
     The current stream's raw handle is asked for directly: building the Stream
     object of torch.cuda.current_stream() takes 2.9 us a call, more than the
-    launch of a decode GEMV (7.0 -> 4.4 us per w8a32_linear_dev call)."""
+    launch of a decode GEMV (7.0 -> 4.4 us per w8a32_linear_dev call).  That
+    accessor is not one of torch's public names: without it, the Stream object."""
     if stream is None:
         import torch
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is not None:
+            return raw(torch.cuda.current_device())
+        stream = torch.cuda.current_stream()
     return stream.cuda_stream
 
 
