@@ -591,10 +591,11 @@ def test_w8a8_gemm(lin, orc, dev, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(80, 130, 300), (100, 2048, 6144), (300, 1000, 1000), (1024, 6144, 2048),
                                    (128, 2048, 2048)])
 def test_w8a8_gemm_configs_bit_exact(lin, orc, dev, M, N, K):
-    """Every int8 MFMA GEMM configuration (both LDS-staged layouts and the
-    register-loaded weight variants with each prefetch depth) gives the exact
-    int32 accumulators and the exact fp32 epilogue, on ragged shapes (M, N, K
-    off the tile sizes, K shorter than the prefetch distance) and full size;
+    """Every int8 MFMA GEMM configuration of codes (the LDS-staged 64 x 128
+    tiles and the quadrant kernel's; the other numbers run the nearest of
+    those) gives the exact int32 accumulators and the exact fp32 epilogue, on
+    ragged shapes (M, N, K off the tile sizes, K shorter than the stage ring)
+    and full size;
     so do K ranges split over 2..8 work-groups per tile (the planner's own
     split included), called twice each."""
     import torch
@@ -754,7 +755,7 @@ def test_w8a16_bf16_fp16(lin, orc, dev, M, N):
     w8a16_kernel.c:187-216): bf16 X with bf16 out and fp16 X with fp16 out
     within relative L2 2e-3 in every row, bf16 X with fp32 out within 1e-5 in
     every row.  At M = 1024 x N = 12288 that is every M tile of the
-    column-split GEMM in its XCD-grouped launch order."""
+    tiled GEMM in its XCD-grouped launch order."""
     import torch
     K = 2048
     say(f"w8a16 bf16/fp16/fp32-out M={M} N={N} K={K}, all rows")
@@ -855,9 +856,9 @@ def test_batch1_padded_paths_capture_into_a_graph(lin, orc, dev, path, K):
 def test_w8a16_k_slices(lin, orc, dev, M, N, K):
     """The 16-bit GEMM with its K range split over 1..4 work-groups per tile
     (every tile configuration, forced through tl_gemm_b16_set_plan: the
-    LDS-staged kernel's 0..2 and the column-split kernel's 4..8, which K not a
-    multiple of 64 runs on configuration 0's kernel; uneven slices where the
-    K blocks do not divide): fp32 out within 1e-5 and bf16
+    LDS-staged kernel's, which 0..2 all name, and the wave-grid kernel's 4..8,
+    with K a multiple of 64 and not; uneven slices where the K blocks do not
+    divide): fp32 out within 1e-5 and bf16
     out within 2e-3 of a float64 product in every row, and a repeated call
     bit-identical (the last work-group to arrive adds the slices in slice
     order, whichever it is)."""

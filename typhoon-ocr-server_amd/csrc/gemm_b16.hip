@@ -432,8 +432,9 @@ __device__ __forceinline__ void set_dword(uint4& u, int c, uint32_t v) {
 // cycles, two waves on a SIMD one every 4.  A widened dword (two weights) costs
 // 3 vector instructions, so a 16 x 16 tile of weights costs 24 and feeds four
 // 32 x 32 x 16 MFMAs (32 cycles each) per 64 rows of X.  Hence 32 x 32 MFMAs
-// (half the instructions of 16 x 16 ones), and two waves per SIMD everywhere:
-// 8 waves on the large tiles, two work-groups per CU on the small ones.  A small
+// (half the instructions of 16 x 16 ones), and two waves per SIMD: 8 waves on the
+// large tiles, two work-groups per CU on the small ones (one, and so one wave per
+// SIMD, where a launch has no more than 256 of those).  A small
 // tile's waves split its columns only (WM = 1), so that each weight is widened
 // once.  The outputs leave through LDS for the same reason: unrolled over the
 // accumulators, scaling and storing took 17 us per 256 x 192 work-group, now 5.

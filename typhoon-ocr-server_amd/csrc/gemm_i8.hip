@@ -392,15 +392,15 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_lds_kernel(GemmI8Args a)
 // Stage s lives in ring slot s % NST.  Step s waits until stage s + 1 has
 // landed, one barrier makes it visible and frees slot s % NST; the MFMAs of
 // stage s run with the fragment reads of stage s + 1 and the copies of stage
-// s + NST spread between them, one every MPO MFMAs.  Sources are uniform 64-bit bases plus one per-lane
-// offset; stages past K re-read the last k-block (branch-free, so the wait
-// counts are exact), and nothing reads what they bring in.
+// s + NST spread between them, one every MPO MFMAs.  Sources are uniform 64-bit
+// bases plus one per-lane offset; stages past K re-read the last k-block
+// (branch-free, so the wait counts are exact), and nothing reads what they bring in.
 //
 // QUAD_PLANES: grouped planes (GemmLaunch::planes_grouped): row group 4T + p holds
 // plane p of tokens 16T .. 16T + 15, so the four sums of one output are the same
 // lane's accumulators 4T .. 4T + 3 and fold without any exchange of lanes
-// (planes_epilogue's 12 cross-lane moves per accumulator were a third of the
-// 64 x 128 kernel's time at K = 2048).
+// (with rows 4t + p the sums of an output lie in four lanes: 12 cross-lane moves per
+// accumulator, a third of a 64 x 128 kernel's time at K = 2048).
 // Accumulators and fragments are left to the register allocator.  Tiles of 8 row
 // groups a wave (512 registers) need MFMAs with accumulators in the vector
 // registers (a compiler option of this file, see the Makefile): it then keeps
@@ -597,7 +597,7 @@ __global__ __launch_bounds__(128 * WM, FM == 8 || WM == 1 ? 1 : 2) void gemm_i8_
   }
   if constexpr (MODE == QUAD_PLANES) {
     // tokens flagged kXeNonFinite: the same lane stores their outputs again
-    // with the reference's fp32 value (as planes_fixup)
+    // with the reference's fp32 value
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < FM / RI; i++) bad |= e_xe[i] == kXeNonFinite;

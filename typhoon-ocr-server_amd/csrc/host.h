@@ -109,6 +109,9 @@ int tlh_linear_w8a8(const float* X, const tl_weights* W, const float* bias, floa
 int tlh_linear_w8a8_tiles(const uint8_t* tiles, const float* xs, const tl_weights* W, float* Y, int batch,
                           hipStream_t st);
 /* the fp32-semantics GEMM (w8a32_linear at batch > 32) on activations already
- * split into four int8 planes per token (code rows 4t + p) with their exponents */
+ * split into four int8 planes per token with their exponents: code rows 4t + p, or
+ * (grouped) row t % 16 of row group 4 (t / 16) + p.  `grouped` has to be what the
+ * tiles were written with, which has to be tlk_gemm_planes_grouped of the shape: a
+ * wrong one gives wrong sums and no error */
 int tlh_linear_w8a32_planes(const uint8_t* tiles, const int* xe, const tl_weights* W, float* Y, int batch,
                             bool grouped, hipStream_t st);

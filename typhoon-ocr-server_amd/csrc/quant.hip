@@ -265,8 +265,8 @@ __global__ __launch_bounds__(256) void quantize_rows_tiled_vec_kernel(const floa
 //   r_p = 254 r_{p-1} - q_p for p = 1..3 (|254 r| <= 127: every q fits int8).
 // So x = 2^e (q0 + q1/254 + q2/254^2 + q3/254^3 + d) with |d| below
 // 2^-26 of 64 (the rounding of 254 r and the last residual): about 2^-32 of
-// the row's absmax.  Plane p of token t is code row 4t + p of the 16x64 tile
-// array (each lane writes one dword per plane for its 4 consecutive k; k past
+// the row's absmax.  Plane p of token t is code row planes_row(t, p, grouped) of
+// the 16x64 tile array (each lane writes one dword per plane for its 4 consecutive k; k past
 // K inside the last k-block gets zero codes).  A row holding Inf or NaN gets
 // xe = kXeNonFinite and zero codes.
 __global__ __launch_bounds__(256) void split_i8x4_kernel(const float* __restrict__ X, int ldx, int M, int K,

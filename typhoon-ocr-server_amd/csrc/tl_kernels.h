@@ -45,7 +45,7 @@ enum { NORM_NONE = 0, NORM_NUMPY = 1, NORM_DECODER = 2 };
 // GEMM A-operand modes and output types (gemm.hip)
 enum { A_I8 = 0, A_BF16 = 1, A_F16 = 2, A_F32X3 = 3 };
 enum { OUT_F32 = 0, OUT_BF16 = 1, OUT_F16 = 2, OUT_I32 = 3,
-       OUT_F32_X4 = 4 };   // A_I8 rows 4t..4t+3 are the int8 planes of fp32 token t (split_i8x4):
+       OUT_F32_X4 = 4 };   // A_I8 rows are the int8 planes of fp32 tokens (split_i8x4):
                            // y[t][n] = ldexp((a0 + a1/254 + a2/254^2 + a3/254^3) * ws[n], xe[t]) (+ bias[n])
 // GEMM float epilogues: fl(acc*ws) then + bias, or fma(acc, ws, bias|0)
 enum { EP_SCALE = 0, EP_SCALE_FMA = 1 };
@@ -63,13 +63,15 @@ hipError_t tlk_launch_pack_tiles_rows(const int8_t* w, int rows, int cols, int N
                                       hipStream_t st);
 // whole-matrix tiles -> row-major int8 codes
 hipError_t tlk_launch_unpack_tiles(const uint8_t* tiles, int rows, int cols, int8_t* w, hipStream_t st);
-// fp32 rows X [M][ldx] -> int8 code tiles of 4 M rows (tile row groups
-// MG = ceil(4M / 16), k-blocks ceil(K / 64); row 4t + p is plane p of token
-// t) and per-token exponents xe[M]: x = 2^e (q0 + q1/254 + q2/254^2 +
-// q3/254^3) up to 2^-32 of the row's absmax; a row holding Inf or NaN gets
-// (grouped: MG = 4 ceil(M / 16), row t % 16 of row group 4 (t / 16) + p instead);
-// a row holding Inf or NaN gets xe = kXeNonFinite (tl_common.h; the GEMM epilogues given the fp32 rows in
-// GemmLaunch.xraw take that row's outputs from them, nonfinite_dot, else NaN)
+// fp32 rows X [M][ldx] -> int8 code tiles of their four planes (k-blocks
+// ceil(K / 64)) and per-token exponents xe[M]: x = 2^e (q0 + q1/254 + q2/254^2 +
+// q3/254^3) up to 2^-32 of the row's absmax.  Plane p of token t is code row 4t + p
+// of ceil(4M / 16) row groups or, grouped, row t % 16 of row group 4 (t / 16) + p of
+// 4 ceil(M / 16); the GEMM that reads them has to be given the same layout
+// (GemmLaunch.planes_grouped; tlk_gemm_planes_grouped says which one it takes).  A
+// row holding Inf or NaN gets xe = kXeNonFinite (tl_common.h; the GEMM epilogues
+// given the fp32 rows in GemmLaunch.xraw take that row's outputs from them,
+// nonfinite_dot, else NaN)
 hipError_t tlk_launch_split_i8x4(const float* X, int ldx, int M, int K, uint8_t* tiles, int* xe, bool grouped,
                                  hipStream_t st);
 // 4-byte-word copy by a kernel (bytes % 4 == 0), e.g. from mapped pinned host memory
@@ -152,8 +154,8 @@ hipError_t tlk_launch_swiglu_rows(const float* gu, float* mlp, int S, int ffn, h
 //   scales: the W8A8 per-token quantization, int8 code tiles (ceil(rows / 16)
 //           row groups) and per-token scales, the codes of
 //           launch_quantize_rows_tiled on the stored rows, bit for bit;
-//   xe:     the four int8 planes per row (code rows 4t + p, ceil(4 rows / 16)
-//           row groups) and exponents of launch_split_i8x4, bit for bit
+//   xe:     the four int8 planes per row and exponents of launch_split_i8x4, in
+//           the layout that `grouped` says, bit for bit
 hipError_t tlk_launch_rmsnorm_rows_q(const float* x, const float* w, uint8_t* tiles, float* scales, int* xe,
                                      int rows, int K, float eps, bool grouped, hipStream_t st);
 // the result of tlk_launch_split_i8x4 with one work-group per row, for
@@ -264,8 +266,9 @@ bool tlk_gemm_planes_grouped(int M4, int N, int K);
 int tlk_gemm_planned(int amode, int out, int M, int N, int K, int* cfg, int* split);
 void tlk_gemm_i8_set_cfg(int cfg);   // tuning override of the int8 GEMM (-1 = planner)
 void tlk_gemm_i8_set_split(int s);   // tuning override of its K slices (0 = planner)
-// tuning override of the 16-bit GEMM: tile configuration 0..2 (-1 = planner)
-// and K slices (0 = planner)
+// tuning override of the 16-bit GEMM: tile configuration (0..2 the LDS-staged
+// kernel, 3 the small-M one, 4..8 the wave-grid one's tiles; -1 = planner) and K
+// slices (0 = planner)
 void tlk_gemm_b16_set_plan(int cfg, int split);
 
 // ---- 2..8 rows of fp32 activations as int8 digit planes (rows.hip): amode
