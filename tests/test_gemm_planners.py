@@ -58,7 +58,7 @@ def test_w8a16_planner(lib):
 
 
 def test_w8a8_planner(lib):
-    _check(_costs(lib, "w8a8", A_I8, OUT_F32), {"hbm": (1.01, 1.2), "repeated": (1.018, 1.32)})
+    _check(_costs(lib, "w8a8", A_I8, OUT_F32), {"hbm": (1.009, 1.2), "repeated": (1.0165, 1.32)})
 
 
 def test_w8a32_planner(lib):

@@ -648,9 +648,9 @@ static int i8_resolve(int cfg, bool planes) {
 // caches hold, as in a model of many layers) and, at lower weight, to repeated ones,
 // of every configuration and 1..8 slices: 16 x 22 shapes of 17..2048 tokens of codes
 // and 16 x 27 of 5..2048 tokens of planes, N = 1024 .. 12288, K = 1000..6144.  The
-// kernel chosen (the small-M kernel among them) is on average 0.5 % (codes) and 0.3 %
+// kernel chosen (the small-M kernel among them) is on average 0.4 % (codes) and 0.3 %
 // (planes) slower than the best of its shape with weights from HBM (1.0 % with limits
-// fitted to repeated weights alone), 0.9 % and 0.5 % with repeated ones.
+// fitted to repeated weights alone), 0.8 % and 0.5 % with repeated ones.
 //   Codes over 256 x 192 or 256 x 256 tiles were the best at none: their fp32 outputs
 // (64 KiB per 128 x 128) drain under the next work-group's loop only where two share a
 // CU.  K slices cost a merge of three dependent memory round trips, about 3 us, so they
@@ -684,6 +684,13 @@ static I8Plan i8_best(bool planes, int M, int N, int K) {
     offer(c, s, fixed + fill * std::min(t, 256) / 256.0f +
                     (t <= 256 ? kb * alone : kb * pair * half + later * (half - 1.0f)) + merge);
   };
+  // two work-groups share a CU: rounds of 512, a last one of up to 256 one per CU
+  auto paired = [&](int c, float fixed, float fill, float full, float full_kb, float alone, float alone_kb) {
+    const int t = tiles(c), n = t / 512, rem = t % 512;
+    const float round = full + full_kb * KB;
+    offer(c, 1, fixed + fill * std::min(t, 256) / 256.0f + n * round +
+                    (rem == 0 ? 0.0f : (rem <= 256 ? alone + alone_kb * KB : round)));
+  };
   if (planes) {
     rounds(3, 1.26f, 0.601f, 8.5f);
     rounds(4, 2.95f, 0.478f, 5.01f);
@@ -694,11 +701,10 @@ static I8Plan i8_best(bool planes, int M, int N, int K) {
   } else {
     for (int s = 1; s <= slices(1); s++) {
       const int t = tiles(1) * s;
-      offer(1, s, 4.99f + 1.39f * t / 256.0f + 1.47f * (cdiv(t, 256) - 1) + cdiv(t, 256) * 0.157f * KB / s +
-                      (s > 1 ? 2.83f + 0.012f * t : 0.0f));
+      offer(1, s, 3.53f + 1.03f * t / 256.0f + cdiv(t, 256) * 0.168f * KB / s + (s > 1 ? 3.67f + 0.0117f * t : 0.0f));
     }
-    shared(5, 1, 5.75f, 4.09f, 0.275f, 0.344f, 4.59f, 0.0f);
-    shared(6, 1, 4.85f, 2.63f, 0.196f, 0.244f, 3.11f, 0.0f);
+    paired(5, -2.73f, 2.46f, 4.75f, 0.579f, 5.7f, 0.233f);
+    paired(6, 0.275f, 0.429f, 2.27f, 0.406f, 3.67f, 0.208f);
   }
   return best;
 }
