@@ -428,8 +428,10 @@ __device__ __forceinline__ void set_dword(uint4& u, int c, uint32_t v) {
 // row-major tiles, xtile_*) and the int8 weight tiles of a 64-wide K stage pass
 // through one LDS ring; a wave widens the weights it reads.
 //
-// What bounds it is instruction issue: one wave issues an instruction every 8
-// cycles, two waves on a SIMD one every 4.  A widened dword (two weights) costs
+// What bounds it is instruction issue beside the matrix pipe: a wave issues an
+// instruction of the widening every 5.8 cycles at most, two waves on a SIMD one every
+// 4.7; an MFMA with 6 of them takes 41.7 cycles of a SIMD with one wave, 33.4 with two.
+// A widened dword (two weights) costs
 // 3 vector instructions, so a 16 x 16 tile of weights costs 24 and feeds four
 // 32 x 32 x 16 MFMAs (32 cycles each) per 64 rows of X.  Hence 32 x 32 MFMAs
 // (half the instructions of 16 x 16 ones), and two waves per SIMD: 8 waves on the

@@ -375,9 +375,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_lds_kernel(GemmI8Args a)
 // movement of operands: per 64-wide K stage a wave reads FM + FN fragments (1 KiB
 // each) for FM FN MFMAs of 16 cycles, and a 256 x 256 tile pulls 32 B/clk per CU
 // from L2 where 64 x 128 tiles need 96.  Two waves per SIMD keep the matrix pipe
-// fed through each other's reads, copies and barriers (one wave issues an
-// instruction every 8-9 cycles, two every 5): 8 waves on 256 x 256 tiles (4 waves
-// of twice the block, in 512 registers: 116 -> 109 us at 1200 tokens of planes
+// fed through each other's reads, copies and barriers: 8 waves on 256 x 256 tiles
+// (4 waves of twice the block, in 512 registers: 116 -> 109 us at 1200 tokens of planes
 // over N = 12288, K = 2048), two work-groups per CU on 128-row ones.  Few tokens of
 // planes leave CUs without a 128-row tile: 64 x 128 ones, of 2 waves, are two and more
 // work-groups where those are one (32 tokens, weights from HBM: N = 12288, K = 2048

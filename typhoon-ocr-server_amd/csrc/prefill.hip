@@ -293,8 +293,8 @@ __global__ __launch_bounds__(256) void prefill_qk_kernel(float* __restrict__ qkv
 constexpr int FT = 64;          // queries / keys per tile
 
 // Wave w holds the 16 queries q0 + 16 w + c in lanes (g, c) = (lane >> 4,
-// lane & 15).  The fp32 MFMA (32 cycles) does not run beside vector
-// instructions (8 cycles each for one wave), so a key tile costs 256 MFMAs plus
+// lane & 15).  The fp32 MFMA (32.6 cycles) does not run beside vector
+// instructions (54 with two adds, 62 with four), so a key tile costs 256 MFMAs plus
 // its vector instructions, whatever the number of waves (two waves per SIMD over
 // halves of the keys measured the same).  Hence masks only where a tile needs
 // them, rescaling only where a maximum grew, and two chains of score MFMAs: 777 /
