@@ -15,7 +15,7 @@ vp, i32 = ctypes.c_void_p, ctypes.c_int
 class GemmLaunch(ctypes.Structure):          # csrc/tl_kernels.h
     _fields_ = [("amode", i32), ("A", vp), ("lda", i32), ("Bt", vp), ("ws", vp), ("xs", vp), ("bias", vp), ("Y", vp),
                 ("ldy", i32), ("M", i32), ("N", i32), ("K", i32), ("ep", i32), ("out", i32), ("part", vp), ("cnt", vp),
-                ("zero_tile", vp), ("xe", vp), ("xraw", vp), ("ldxr", i32), ("planes_grouped", ctypes.c_bool),
+                ("zero_tile", vp), ("xe", vp), ("xraw", vp), ("ldxr", i32), ("planes_grouped", ctypes.c_bool), ("whole", ctypes.c_bool),
                 ("kernel", i32), ("cfg", i32), ("split", i32)]
 
 
@@ -140,3 +140,35 @@ def test_rows_override_between_sizing_and_launch(lin, dev, M, N, K):
     # the planes hold a value to 2^-32 of its row's absmax; the fold, the scale and
     # the slices' sum round at most 16 times, each within 2^-24 of the sum of terms
     assert ((y.cpu() - want).abs() <= 16 * 2.0 ** -24 * (x.abs() @ w.abs().T)).all()
+
+
+@pytest.mark.gpu
+def test_capture_without_split_workspace(lin, dev):
+    """A shape that the planner gives K slices, captured on a stream that has no
+    work-space for them (it cannot be allocated under capture): whole tiles, the same
+    bits as the eager call, in every replay."""
+    import torch
+    M, N, K = 64, 6144, 6144
+    say(f"int8 GEMM captured without a work-space M={M} N={N} K={K}")
+    g = torch.Generator().manual_seed(7)
+    W = lin.DeviceWeights.quantize(torch.randn(N, K, generator=g).to(dev))
+    t = torch.empty(M * K, dtype=torch.uint8, device=dev)
+    s = torch.empty(M, device=dev)
+    y, captured = torch.empty(M, N, device=dev), torch.empty(M, N, device=dev)
+    x = torch.randn(M, K, generator=g)
+    lin.w8a8_quantize_tiles_dev(x.to(dev), t, s)
+    lin.w8a8_linear_tiles_dev(t, s, W, y)
+    torch.cuda.synchronize()
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        lin.w8a8_linear_tiles_dev(t, s, W, captured)
+    for i in range(3):
+        lin.w8a8_quantize_tiles_dev((x * (i + 1)).to(dev).roll(i, 0), t, s)
+        lin.w8a8_linear_tiles_dev(t, s, W, y)
+        captured.fill_(-1.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, y)
+    del graph
+    W.close()

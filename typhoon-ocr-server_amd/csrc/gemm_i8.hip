@@ -647,9 +647,10 @@ static int i8_resolve(int cfg, bool planes) {
 // caches hold, as in a model of many layers) and, at lower weight, to repeated ones,
 // of every configuration and 1..8 slices: 16 x 22 shapes of 17..2048 tokens of codes
 // and 16 x 27 of 5..2048 tokens of planes, N = 1024 .. 12288, K = 1000..6144.  The
-// kernel chosen (the small-M kernel among them) is on average 0.4 % (codes) and 0.3 %
+// kernel chosen (the small-M kernel among them) is on average 0.5 % (codes) and 0.4 %
 // (planes) slower than the best of its shape with weights from HBM (1.0 % with limits
-// fitted to repeated weights alone), 0.8 % and 0.5 % with repeated ones.
+// fitted to repeated weights alone), 0.8 % and 0.4 % with repeated ones; over 99 shapes
+// outside that range (N = 256 .. 151936, K = 512 .. 6144) 1.4 % and 1.1 %.
 //   Codes over 256 x 192 or 256 x 256 tiles were the best at none: their fp32 outputs
 // (64 KiB per 128 x 128) drain under the next work-group's loop only where two share a
 // CU.  K slices cost a merge of three dependent memory round trips, about 3 us, so they
@@ -660,7 +661,7 @@ struct I8Plan {
   int cfg, split;
   float us;
 };
-static I8Plan i8_best(bool planes, int M, int N, int K) {
+static I8Plan i8_best(bool planes, int M, int N, int K, bool whole = false) {
   const int MG = planes ? planes_groups(M / 4, true) : cdiv(M, 16), NG = cdiv(N, 16), KB = cdiv(K, 64);
   I8Plan best{planes ? 6 : 1, 1, 3.0e38f};
   auto tiles = [&](int c) {
@@ -671,39 +672,35 @@ static I8Plan i8_best(bool planes, int M, int N, int K) {
   auto offer = [&](int c, int s, float us) {
     if (us < best.us) best = I8Plan{c, s, us};
   };
-  auto slices = [&](int c) { return tiles(c) <= 128 ? std::min(4, KB) : 1; };
+  auto slices = [&](int c) { return tiles(c) <= 128 && !whole ? std::min(4, KB) : 1; };
   // one work-group per CU: rounds of 256
   auto rounds = [&](int c, float fixed, float kb, float fill) {
     offer(c, 1, cdiv(tiles(c), 256) * (fixed + kb * KB) + fill * tiles(c) / 256.0f);
   };
-  // work-groups share CUs: the time of a k-block grows with each half round of 256
-  auto shared = [&](int c, int s, float fixed, float fill, float alone, float pair, float later, float merge) {
-    const int t = tiles(c) * s;
-    const float half = 0.5f * (float)cdiv(t, 128), kb = (float)KB / s;
-    offer(c, s, fixed + fill * std::min(t, 256) / 256.0f +
-                    (t <= 256 ? kb * alone : kb * pair * half + later * (half - 1.0f)) + merge);
-  };
-  // two work-groups share a CU: rounds of 512, a last one of up to 256 one per CU
-  auto paired = [&](int c, float fixed, float fill, float full, float full_kb, float alone, float alone_kb) {
-    const int t = tiles(c), n = t / 512, rem = t % 512;
-    const float round = full + full_kb * KB;
-    offer(c, 1, fixed + fill * std::min(t, 256) / 256.0f + n * round +
-                    (rem == 0 ? 0.0f : (rem <= 256 ? alone + alone_kb * KB : round)));
+  // two work-groups share a CU: rounds of 512, a last one of up to 256 one per CU;
+  // K slices and their merge
+  auto paired = [&](int c, int s, float fixed, float fill, float full, float full_kb, float alone, float alone_kb,
+                    float merge = 0.0f, float part = 0.0f) {
+    const int t = tiles(c) * s, n = t / 512, rem = t % 512;
+    const float kb = (float)KB / s, round = full + full_kb * kb;
+    offer(c, s, fixed + fill * std::min(t, 256) / 256.0f + n * round +
+                    (rem == 0 ? 0.0f : (rem <= 256 ? alone + alone_kb * kb : round)) + (s > 1 ? merge + part * t : 0.0f));
   };
   if (planes) {
-    rounds(3, 1.26f, 0.601f, 8.5f);
-    rounds(4, 2.95f, 0.478f, 5.01f);
+    rounds(3, 1.6f, 0.612f, 8.04f);
+    rounds(4, 5.56f, 0.463f, 2.66f);
     for (int s = 1; s <= slices(6); s++)
-      shared(6, s, 3.8f, 1.28f, 0.207f, 0.239f, 0.65f, s > 1 ? 4.23f + 0.0178f * tiles(6) * s : 0.0f);
+      paired(6, s, 0.159f, 1.23f, 4.11f, 0.425f, 3.41f, 0.205f, 3.76f, 0.0192f);
     for (int s = 1; s <= slices(7); s++)
-      shared(7, s, 4.05f, 0.372f, 0.175f, 0.149f, 0.592f, s > 1 ? 2.62f + 0.0123f * tiles(7) * s : 0.0f);
+      paired(7, s, 0.323f, 0.481f, 3.68f, 0.26f, 3.31f, 0.176f, 3.15f, 0.00935f);
   } else {
+    // 64 x 128 tiles: as one round
     for (int s = 1; s <= slices(1); s++) {
       const int t = tiles(1) * s;
-      offer(1, s, 3.53f + 1.03f * t / 256.0f + cdiv(t, 256) * 0.168f * KB / s + (s > 1 ? 3.67f + 0.0117f * t : 0.0f));
+      if (t <= 256) offer(1, s, 5.71f + 0.634f * t / 256.0f + 0.138f * KB / s + (s > 1 ? 3.11f + 0.0109f * t : 0.0f));
     }
-    paired(5, -2.73f, 2.46f, 4.75f, 0.579f, 5.7f, 0.233f);
-    paired(6, 0.275f, 0.429f, 2.27f, 0.406f, 3.67f, 0.208f);
+    paired(5, 1, 0.0553f, 2.57f, 21.4f, 0.335f, 5.91f, 0.273f);
+    paired(6, 1, 0.222f, 0.103f, 11.8f, 0.361f, 4.99f, 0.207f);
   }
   return best;
 }
@@ -713,7 +710,7 @@ float gemm_i8_us(int out, int M, int N, int K) { return i8_best(out == OUT_F32_X
 static void gemm_i8_plan(const GemmLaunch& L, int& cfg, int& split) {
   const bool planes = L.out == OUT_F32_X4;
   const int KB = cdiv(L.K, 64);
-  const I8Plan best = i8_best(planes, L.M, L.N, L.K);
+  const I8Plan best = i8_best(planes, L.M, L.N, L.K, L.whole);
   cfg = best.cfg;
   split = best.split;
   const int fc = g_i8_force_cfg.load(std::memory_order_relaxed);

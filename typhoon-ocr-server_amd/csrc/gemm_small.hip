@@ -524,12 +524,10 @@ static int small_rows_per_wg(int MG, int NG) {
 // int8 kernels' is (i8_best, gemm_i8.hip).
 float gemm_small_i8_us(int out, int M, int N, int K) {
   const int MG = cdiv(M, 16), NG = cdiv(N, 16), r = small_rows_per_wg(MG, NG), wgs = cdiv(NG, r) * MG;
-  const float rounds = (float)cdiv(wgs, 256), KB = (float)cdiv(K, 64);
-  if (out == OUT_F32_X4) {
-    const float rd = 0.932f * rounds + 0.068f * std::max(1.0f, wgs / 256.0f);
-    return 1.85f + rd * (0.215f + 0.0492f * r + KB * (0.0308f + 0.0203f * r));
-  }
-  return 2.19f + rounds * (0.0521f + 0.0105f * r + KB * (0.025f * r - 0.0143f));
+  const float rounds = (float)cdiv(wgs, 256), fill = std::max(1.0f, wgs / 256.0f), KB = (float)cdiv(K, 64);
+  return out == OUT_F32_X4
+             ? 2.21f + rounds * (0.118f + 0.113f * r + KB * (0.0f + 0.0189f * r)) + 0.00801f * KB * r * fill
+             : 2.17f + rounds * (0.0577f + 0.21f * r + KB * (0.00962f + 0.0172f * r)) + 0.00249f * KB * r * fill;
 }
 
 // tuning override of the 16-bit rows' work-group shape: 100 R + 10 TG + U
