@@ -172,3 +172,33 @@ def test_capture_without_split_workspace(lin, dev):
         assert torch.equal(captured, y)
     del graph
     W.close()
+
+
+@pytest.mark.gpu
+def test_16bit_capture_without_split_workspace(lin, dev):
+    """The same for 16-bit rows, whose sums are taken in another order then: each
+    output within K 2^-24 of the sum of its terms' magnitudes, twice (the bound of
+    fp32 summation in any order, on both sides)."""
+    import torch
+    M, N, K = 333, 2048, 6144
+    say(f"16-bit GEMM captured without a work-space M={M} N={N} K={K}")
+    g = torch.Generator().manual_seed(8)
+    w = torch.randn(N, K, generator=g)
+    W = lin.DeviceWeights.quantize(w.to(dev))
+    x = torch.randn(M, K, generator=g).bfloat16()
+    xd = x.to(dev)
+    y, captured = torch.empty(M, N, device=dev), torch.empty(M, N, device=dev)
+    lin.w8a16_linear_dev(xd, W, y)
+    torch.cuda.synchronize()
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        lin.w8a16_linear_dev(xd, W, captured)
+    bar = 2 * K * 2.0 ** -24 * (x.float().abs().to(dev) @ (w.abs().to(dev) * 1.01).t().contiguous())
+    for _ in range(3):
+        captured.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert ((captured - y).abs() <= bar).all()
+    del graph
+    W.close()

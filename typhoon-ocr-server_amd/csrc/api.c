@@ -597,9 +597,10 @@ static int run_gemm(Workspace* ws, GemmLaunch* L, hipStream_t st) {
   TRY(zero_tile(&L->zero_tile));
   size_t part_bytes = 0, counters = 0;
   tlk_gemm_resolve(L, &part_bytes, &counters);
-  if (L->amode == A_I8 && (part_bytes > ws->part.n || counters > ws->cnt_n)) {
-    /* the work-space cannot grow while the stream is being captured: whole tiles
-     * then, which give the same bits (int8 sums are exact) */
+  if (part_bytes > ws->part.n || counters > ws->cnt_n) {
+    /* the work-space cannot grow while the stream is being captured: the tiled
+     * kernels take whole tiles then (int8 sums are exact, so the same bits; 16-bit
+     * ones are summed in one order instead of slice by slice) */
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();
     else if (cs == hipStreamCaptureStatusActive) {

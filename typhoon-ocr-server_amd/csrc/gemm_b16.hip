@@ -756,7 +756,7 @@ struct B16Plan {
   int cfg, split;
   float us;
 };
-static B16Plan b16_best(int MG, int NG, int KB) {
+static B16Plan b16_best(int MG, int NG, int KB, bool whole = false) {
   B16Plan best{0, 1, 3.0e38f};
   auto offer = [&](int c, int s, float us) {
     if (us < best.us) best = B16Plan{c, s, us};
@@ -771,7 +771,7 @@ static B16Plan b16_best(int MG, int NG, int KB) {
                      merge[2] = {2.23f, 3.0f}, part[2] = {0.0267f, 0.0139f};
   for (int c = 6; c <= 8; c++) {
     const int i = c - 6, tiles = b16_tiles(c, MG, NG);
-    for (int s = 1; s <= (c < 8 && tiles <= 128 ? 4 : 1) && s <= KB; s++) {
+    for (int s = 1; s <= (c < 8 && tiles <= 128 && !whole ? 4 : 1) && s <= KB; s++) {
       const float half = 0.5f * (float)cdiv(tiles * s, 128), kb = (float)KB / s;
       offer(c, s, fixed[i] + (tiles * s <= 256 ? kb * alone[i] : kb * shared[i] * half + later[i] * (half - 1.0f)) +
                       (s > 1 ? merge[i] + part[i] * tiles * s : 0.0f));
@@ -782,10 +782,10 @@ static B16Plan b16_best(int MG, int NG, int KB) {
 // estimated us of the wave-grid kernel's plan
 float gemm_b16_us(int M, int N, int K) { return b16_best(cdiv(M, 16), cdiv(N, 16), cdiv(K, 64)).us; }
 
-static void b16_plan(int MG, int NG, int KB, bool off32, int& cfg_out, int& split_out) {
+static void b16_plan(int MG, int NG, int KB, bool off32, bool whole, int& cfg_out, int& split_out) {
   int cfg = 0, split = 1;
   if (off32) {
-    const B16Plan best = b16_best(MG, NG, KB);
+    const B16Plan best = b16_best(MG, NG, KB, whole);
     cfg = best.cfg;
     split = best.split;
   }
@@ -807,7 +807,7 @@ void gemm_b16_resolve(GemmLaunch& L, size_t* part_bytes, size_t* counters) {
   const int MG = cdiv(L.M, 16), NG = cdiv(L.N, 16);
   const bool off32 = (size_t)L.M * (size_t)L.lda * 2 < ((size_t)1 << 32);
   int mt, nt;
-  b16_plan(MG, NG, cdiv(L.K, 64), off32, L.cfg, L.split);
+  b16_plan(MG, NG, cdiv(L.K, 64), off32, L.whole, L.cfg, L.split);
   b16_cfg(L.cfg, mt, nt);
   const size_t tiles = (size_t)cdiv(MG, mt) * cdiv(NG, nt);
   *part_bytes = L.split > 1 ? tiles * L.split * (size_t)(256 * mt * nt) * sizeof(float) : 0;

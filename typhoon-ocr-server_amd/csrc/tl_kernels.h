@@ -236,7 +236,7 @@ typedef struct GemmLaunch {
   const float* xraw TLK_DEF(nullptr);    // OUT_F32_X4: the fp32 token rows [M / 4][ldxr] the planes came
   int ldxr TLK_DEF(0);                   //   from (outputs of a non-finite row from them); null: NaN
   bool planes_grouped TLK_DEF(false);    // OUT_F32_X4: row group 4T + p holds plane p of tokens 16T .. 16T + 15
-  bool whole TLK_DEF(false);             // A_I8: no K slices (the same bits), so no work-space
+  bool whole TLK_DEF(false);             // tiled kernels: no K slices, so no work-space
   // set by tlk_gemm_resolve: the kernel (-1 none yet), its configuration and K slices
   int kernel TLK_DEF(-1), cfg TLK_DEF(0), split TLK_DEF(1);
 } GemmLaunch;
